@@ -1,8 +1,8 @@
 """Builds ``hemelb_amd/libhemelb_amd.so`` in-tree.
 
-* ``csrc/lbm_kernels.hip`` and ``csrc/unet_kernels.hip`` -> hipcc for gfx950
-  (device code; no FMA contraction so binary64 results match the
-  reference's evaluation order).
+* ``csrc/lbm_kernels.hip`` (once per layout), ``csrc/lbm_fields.hip`` and
+  ``csrc/unet_kernels.hip`` -> hipcc for gfx950 (device code; no FMA
+  contraction so binary64 results match the reference's evaluation order).
 * ``csrc/solver.cpp``, ``csrc/geometry.cpp``, ``csrc/extraction.cpp`` and
   ``csrc/unet.cpp`` -> g++ (host code; the same compiler runtime and libm as the reference's own
   g++ build).
@@ -17,6 +17,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -54,16 +55,17 @@ def _run(cmd):
 
 def build() -> str:
     os.makedirs(BUILD, exist_ok=True)
-    objs = []
-    for hip in ("lbm_kernels.hip", "unet_kernels.hip"):
-        k_obj = os.path.join(BUILD, hip.replace(".hip", ".o"))
-        _run([os.path.join(ROCM, "bin", "hipcc")] + HIPCC_FLAGS +
-             ["-c", os.path.join(CSRC, hip), "-o", k_obj])
-        objs.append(k_obj)
-    for src in ("solver.cpp", "geometry.cpp", "extraction.cpp", "unet.cpp"):
-        obj = os.path.join(BUILD, src.replace(".cpp", ".o"))
-        _run(["g++"] + GXX_FLAGS + ["-c", os.path.join(CSRC, src), "-o", obj])
-        objs.append(obj)
+    hipcc = [os.path.join(ROCM, "bin", "hipcc")] + HIPCC_FLAGS
+    jobs = [(hipcc + [f"-DHLB_LAYOUT={k}"], "lbm_kernels.hip", f"lbm_kernels_{k}.o")
+            for k in (1, 2, 0)]
+    jobs += [(hipcc, src, src.replace(".hip", ".o")) for src in ("lbm_fields.hip",
+                                                                 "unet_kernels.hip")]
+    jobs += [(["g++"] + GXX_FLAGS, src, src.replace(".cpp", ".o"))
+             for src in ("solver.cpp", "geometry.cpp", "extraction.cpp", "unet.cpp")]
+    objs = [os.path.join(BUILD, obj) for _, _, obj in jobs]
+    with ThreadPoolExecutor(max_workers=4) as pool:
+        list(pool.map(lambda j: _run(j[0] + ["-c", os.path.join(CSRC, j[1]), "-o",
+                                             os.path.join(BUILD, j[2])]), jobs))
     tmp = LIB + ".tmp"
     _run(["g++", "-shared", "-o", tmp] + objs +
          ["-L", os.path.join(ROCM, "lib"), "-lamdhip64", "-lz",

@@ -1,5 +1,5 @@
 // Internal interface between the host solver (solver.cpp, built with g++)
-// and the HIP kernels (lbm_kernels.hip, built with hipcc).  Plain structs of
+// and the HIP kernels (lbm_kernels.hip, lbm_fields.hip, built with hipcc).  Plain structs of
 // device pointers; no HIP types so that the host side needs no device
 // compiler.
 #pragma once

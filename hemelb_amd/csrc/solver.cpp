@@ -197,7 +197,7 @@ uint64_t spread3(uint64_t v) {
 }
 
 // Slot of a site inside its 8^3 block: x plane major, then the in-plane
-// lane, the order the block-layout kernels address (lbm_kernels.hip
+// lane, the order the block-layout kernels address (lbm_device.h
 // kMortonLanes): with `morton` (binary64 storage) the bits of (y, z)
 // interleaved, z in bits 0, 2, 4 and y in bits 1, 3, 5; otherwise rows of z
 // (y * 8 + z).
@@ -886,7 +886,7 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
     for (int64_t w = 0; w < nwaves; ++w)
       if (h_wf[w]) (h_wb[w] ? h_bndw : h_bulkw).push_back((uint32_t)w);
     // Check, on the host, every neighbour the block-layout kernel will
-    // compute (BlockLayout::src in lbm_kernels.hip): each bulk pull of each
+    // compute (BlockLayout::src in lbm_device.h): each bulk pull of each
     // fluid site must land on the slot of its source site.
     for (int64_t o2 = 0; o2 < n; ++o2) {
       const int64_t i = s->perm[o2];

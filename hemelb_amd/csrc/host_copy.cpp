@@ -1,0 +1,161 @@
+// Device-to-host copies through a ring of pinned chunks, emptied by several
+// host threads.
+//
+// A plain copy into pageable memory runs at about 10 GB/s here whatever its
+// size: one thread of the runtime touches (the kernel zeroes) the caller's
+// pages and moves the data.  The link delivers more than 50 GB/s into pinned
+// memory, so the copy goes into pinned chunks and worker threads move them
+// on, each taking the page faults of its own chunks.
+#include "host_copy.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <mutex>
+#include <system_error>
+#include <thread>
+
+namespace hlb {
+namespace {
+
+constexpr size_t kChunk = size_t(1) << 20;
+constexpr int kSlots = 16;          // 16 MiB of pinned memory per process
+constexpr int kMaxWorkers = 8;
+// Smaller copies are left to the runtime: starting the workers costs more
+// than they save.
+constexpr size_t kDirect = size_t(4) << 20;
+
+struct Staging {
+  std::mutex mu;       // held by the copy that uses the buffer
+  char* pinned = nullptr;
+  std::mutex users_mu;
+  int users = 0;
+};
+Staging& staging() {
+  static Staging* s = new Staging;   // never destroyed: solvers may outlive statics
+  return *s;
+}
+
+hipError_t copy_direct(const std::vector<HostSegment>& segments, hipStream_t stream) {
+  for (const HostSegment& g : segments) {
+    const hipError_t e = hipMemcpyAsync(g.dst, g.src, g.bytes, hipMemcpyDeviceToHost, stream);
+    if (e != hipSuccess) return e;
+  }
+  return hipStreamSynchronize(stream);
+}
+
+// The chunks of one copy and the hand-over between the issuing thread and the
+// workers: chunk i travels through slot i % kSlots, which is issued again
+// only after done[i].
+struct Job {
+  std::vector<HostSegment> chunks;
+  std::vector<std::atomic<bool>> done;
+  std::atomic<size_t> next{0}, issued{0};
+  std::atomic<int> error{(int)hipSuccess};
+  hipEvent_t arrived[kSlots] = {};
+  char* pinned;
+  int device;
+
+  Job(std::vector<HostSegment> c, char* p, int dev)
+      : chunks(std::move(c)), done(chunks.size()), pinned(p), device(dev) {
+    for (auto& d : done) d.store(false, std::memory_order_relaxed);
+  }
+  ~Job() {
+    for (auto& e : arrived)
+      if (e) (void)hipEventDestroy(e);
+  }
+  void fail(hipError_t e) {
+    int none = (int)hipSuccess;
+    error.compare_exchange_strong(none, (int)e);
+  }
+  bool failed() const { return error.load() != (int)hipSuccess; }
+
+  void work() {
+    (void)hipSetDevice(device);
+    for (;;) {
+      const size_t i = next.fetch_add(1);
+      if (i >= chunks.size()) return;
+      while (issued.load(std::memory_order_acquire) <= i) {
+        if (failed()) return;
+        std::this_thread::yield();
+      }
+      const hipError_t e = hipEventSynchronize(arrived[i % kSlots]);
+      if (e != hipSuccess) return fail(e);
+      std::memcpy(chunks[i].dst, pinned + (i % kSlots) * kChunk, chunks[i].bytes);
+      done[i].store(true, std::memory_order_release);
+    }
+  }
+  void issue(hipStream_t stream) {
+    for (size_t i = 0; i < chunks.size(); ++i) {
+      const int slot = (int)(i % kSlots);
+      if (i >= (size_t)kSlots)
+        while (!done[i - kSlots].load(std::memory_order_acquire)) {
+          if (failed()) return;
+          std::this_thread::yield();
+        }
+      hipError_t e = hipMemcpyAsync(pinned + slot * kChunk, chunks[i].src, chunks[i].bytes,
+                                    hipMemcpyDeviceToHost, stream);
+      if (e == hipSuccess) e = hipEventRecord(arrived[slot], stream);
+      if (e != hipSuccess) return fail(e);
+      issued.store(i + 1, std::memory_order_release);
+    }
+  }
+};
+
+}  // namespace
+
+hipError_t copy_to_host(const std::vector<HostSegment>& segments, hipStream_t stream) {
+  size_t total = 0;
+  for (const HostSegment& g : segments) total += g.bytes;
+  Staging& st = staging();
+  std::unique_lock<std::mutex> lock(st.mu, std::try_to_lock);
+  // another thread's copy has the staging buffer: take the runtime's path
+  if (total < kDirect || !lock.owns_lock()) return copy_direct(segments, stream);
+  if (!st.pinned && hipHostMalloc((void**)&st.pinned, kSlots * kChunk) != hipSuccess) {
+    st.pinned = nullptr;
+    (void)hipGetLastError();
+    return copy_direct(segments, stream);
+  }
+  std::vector<HostSegment> chunks;
+  for (const HostSegment& g : segments)
+    for (size_t a = 0; a < g.bytes; a += kChunk)
+      chunks.push_back({(char*)g.dst + a, (const char*)g.src + a, std::min(kChunk, g.bytes - a)});
+  int device = 0;
+  hipError_t e = hipGetDevice(&device);
+  if (e != hipSuccess) return e;
+  Job job(std::move(chunks), st.pinned, device);
+  for (auto& ev : job.arrived) {
+    e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (e != hipSuccess) return e;
+  }
+  const size_t wanted = std::min<size_t>(kMaxWorkers, total / (2 * kChunk));
+  std::vector<std::thread> workers;
+  workers.reserve(wanted);
+  try {
+    for (size_t k = 0; k < wanted; ++k) workers.emplace_back([&job] { job.work(); });
+  } catch (const std::system_error&) {
+  }
+  if (workers.empty()) return copy_direct(segments, stream);
+  job.issue(stream);
+  for (auto& w : workers) w.join();
+  // no copy may still write the staging buffer or read the source
+  e = hipStreamSynchronize(stream);
+  return job.failed() ? (hipError_t)job.error.load() : e;
+}
+
+void staging_acquire() {
+  Staging& st = staging();
+  std::lock_guard<std::mutex> lock(st.users_mu);
+  ++st.users;
+}
+
+void staging_release() {
+  Staging& st = staging();
+  std::lock_guard<std::mutex> lock(st.users_mu);
+  if (--st.users > 0) return;
+  std::lock_guard<std::mutex> copy(st.mu);
+  if (st.pinned) (void)hipHostFree(st.pinned);
+  st.pinned = nullptr;
+}
+
+}  // namespace hlb

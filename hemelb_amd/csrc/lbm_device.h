@@ -1341,6 +1341,19 @@ inline bool narrow_offsets(const DevDomain& d, const StepArgs& a, size_t esize) 
   return !a.wide && (uint64_t)a.Q * (uint64_t)d.np * esize <= 0xFFFFFFFFull;
 }
 
+// As dispatch, with BlockLayout32 in the place of BlockLayout where its
+// offsets reach the whole state.
+template <typename Fn>
+int dispatch_narrow(const DevDomain& d, const StepArgs& a, Fn&& fn) {
+  return dispatch(d, a, [&](auto q, auto k, auto* s, auto* lay) {
+    using S = std::remove_pointer_t<decltype(s)>;
+    using Lay = std::remove_pointer_t<decltype(lay)>;
+    if constexpr (std::is_same<Lay, BlockLayout>::value)
+      if (narrow_offsets(d, a, sizeof(S))) return fn(q, k, s, (BlockLayout32*)nullptr);
+    return fn(q, k, s, lay);
+  });
+}
+
 }  // namespace
 
 // The timestep's launches for one layout (lbm_kernels.hip, compiled once per

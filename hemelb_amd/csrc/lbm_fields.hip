@@ -12,33 +12,6 @@ static __device__ __align__(256) double scratch[hlb::kStaticScratchDoubles];
 namespace hlb {
 namespace {
 
-// Post-stream distributions in binary64, compact SoA [Q][npc].
-template <int Q, typename S, class Lay>
-__global__ __launch_bounds__(256) void k_stream_only(DevDomain D, StepArgs A,
-                                                     const S* __restrict__ fin,
-                                                     double* __restrict__ out,
-                                                     int from_post_stream) {
-  using T = typename Store<S>::T;
-  SiteRef r;
-  if (!Lay::locate(D, r)) return;
-  T f[Q];
-  if (from_post_stream) {
-    sfor<0, Q>([&](auto di) {
-      constexpr int d = decltype(di)::value;
-      f[d] = Store<S>::ld(fin + Lay::template at<Q>(D, d, r.x));
-    });
-  } else {
-    gather<Q, S, T, Lay>(D, A, fin, r, f);
-  }
-  const int64_t c = Lay::compact(D, r);
-  sfor<0, Q>([&](auto di) {
-    constexpr int d = decltype(di)::value;
-    double v = (double)f[d];
-    if constexpr (kShifted<S>) v += Lat<Q>::w[d] * A.rho0;
-    out[(int64_t)d * D.npc + c] = v;
-  });
-}
-
 // Device-copy ceiling of the step's traffic: the Q state arrays (stride
 // `stride` words of type W) copied from `in` to `out`, `words` per array,
 // one word per thread and array, all loads issued before the streamed
@@ -133,111 +106,86 @@ __global__ void k_fill(int64_t nslots, int64_t np, int blockwise, const double* 
   });
 }
 
-__global__ void k_soa_to_aos(int Q, int64_t n, int64_t np, const double* soa,
-                             const int64_t* perm, double* aos) {
-  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= n) return;
-  const int64_t c = perm[x];
-  for (int d = 0; d < Q; ++d) aos[c * Q + d] = soa[(int64_t)d * np + x];
-}
-
-template <int Q>
-__global__ void k_moments(int64_t n, int64_t np, const double* soa, double* rho,
-                          double* u) {
-  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= n) return;
-  double f[Q];
+// Post-stream distributions of a site (the reference's fOld) in binary64:
+// the state itself when it already is post-stream, else the pull.
+template <int Q, typename S, class Lay>
+__device__ __forceinline__ void post_stream_site(const DevDomain& D, const StepArgs& A,
+                                                 const S* __restrict__ fin,
+                                                 int from_post_stream, const SiteRef& r,
+                                                 double (&g)[Q]) {
+  using T = typename Store<S>::T;
+  T f[Q];
+  if (from_post_stream) {
+    sfor<0, Q>([&](auto di) {
+      constexpr int d = decltype(di)::value;
+      f[d] = Store<S>::ld(own_ptr<Q, Lay>(D, r, fin, d));
+    });
+  } else {
+    gather<Q, S, T, Lay>(D, A, fin, r, f);
+  }
   sfor<0, Q>([&](auto di) {
     constexpr int d = decltype(di)::value;
-    f[d] = soa[(int64_t)d * np + x];
+    double v = (double)f[d];
+    if constexpr (kShifted<S>) v += Lat<Q>::w[d] * A.rho0;
+    g[d] = v;
   });
-  double r, mx, my, mz;
-  moments<Q, double>(f, r, mx, my, mz);
-  rho[x] = r;
-  u[x] = mx / r;
-  u[np + x] = my / r;
-  u[2 * np + x] = mz / r;
 }
 
-// Per-block binary64 reductions in a fixed tree order: [mass, min rho,
-// max rho, max |u|, unstable] per block.
-template <int Q>
-__global__ __launch_bounds__(256) void k_reduce(int64_t n, int64_t np,
-                                                const double* soa,
-                                                const double* rho,
-                                                const double* u,
-                                                double* partials) {
-  __shared__ double s_sum[256], s_min[256], s_max[256], s_u[256], s_bad[256];
+// Calls visit(site) for every site of workgroup blockIdx.x: without `range`
+// the x planes g*W + k*W*grid (W waves per workgroup) of the block layouts, or
+// the compact sites g*256 + t + k*256*grid of the pull table, so that a
+// reduction's partials depend on the grid size only; with it, the planes (or
+// sites) range[2g] .. range[2g+1].
+template <class Lay, typename V>
+__device__ __forceinline__ void visit_sites(const DevDomain& D, const int64_t* range, V&& visit) {
   const int t = threadIdx.x;
-  double sum = 0.0, mn = 1.7976931348623157e308, mx = -1.7976931348623157e308,
-         um = 0.0, bad = 0.0;
-  for (int64_t x = (int64_t)blockIdx.x * blockDim.x + t; x < n;
-       x += (int64_t)gridDim.x * blockDim.x) {
-    const double r = rho[x];
-    sum += r;
-    mn = r < mn ? r : mn;
-    mx = r > mx ? r : mx;
-    const double a = u[x], b = u[np + x], c = u[2 * np + x];
-    const double m = sqrt(((0.0 + a * a) + b * b) + c * c);
-    um = m > um ? m : um;
-    for (int d = 0; d < Q; ++d)
-      if (!(soa[(int64_t)d * np + x] > 0.0)) bad = 1.0;
-  }
-  s_sum[t] = sum; s_min[t] = mn; s_max[t] = mx; s_u[t] = um; s_bad[t] = bad;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) {
-      s_sum[t] += s_sum[t + w];
-      s_min[t] = s_min[t + w] < s_min[t] ? s_min[t + w] : s_min[t];
-      s_max[t] = s_max[t + w] > s_max[t] ? s_max[t + w] : s_max[t];
-      s_u[t] = s_u[t + w] > s_u[t] ? s_u[t + w] : s_u[t];
-      s_bad[t] = s_bad[t + w] > s_bad[t] ? s_bad[t + w] : s_bad[t];
+  if constexpr (kWaveLayout<Lay>) {
+    const uint32_t wpg = blockDim.x >> 6;
+    const uint32_t step = range ? wpg : gridDim.x * wpg;
+    const uint32_t end = range ? (uint32_t)range[2 * blockIdx.x + 1] : D.nwaves;
+    for (uint32_t base = range ? (uint32_t)range[2 * blockIdx.x] : blockIdx.x * wpg; base < end;
+         base += step) {
+      const uint32_t w = __builtin_amdgcn_readfirstlane(base + ((uint32_t)t >> 6));
+      SiteRef r;
+      if (w < end && Lay::locate_wave(D, w, r)) visit(r);
     }
-    __syncthreads();
-  }
-  if (t == 0) {
-    double* p = partials + 5 * blockIdx.x;
-    p[0] = s_sum[0]; p[1] = s_min[0]; p[2] = s_max[0]; p[3] = s_u[0]; p[4] = s_bad[0];
+  } else {
+    const int64_t step = range ? blockDim.x : (int64_t)gridDim.x * blockDim.x;
+    const int64_t end = range ? range[2 * blockIdx.x + 1] : D.n;
+    for (int64_t x = (range ? range[2 * blockIdx.x] : (int64_t)blockIdx.x * blockDim.x) + t;
+         x < end; x += step) {
+      SiteRef r;
+      Lay::at(D, x, r);
+      visit(r);
+    }
   }
 }
 
 // The monitor's statistics straight from the state, without an exported
-// copy: every site's fOld (the state itself when it is post-stream, else the
-// pull of k_stream_only), its density and velocity as k_moments computes
-// them, and per workgroup [mass, min rho, max rho, max |u|, unstable] as
-// k_reduce combines them.  Workgroup g visits the x planes g*W + k*W*grid
-// (W waves per workgroup) of the block layouts, or the compact sites
-// g*256 + t + k*256*grid of the pull table, so the partials depend on the
-// grid size only.  The density and velocity of every iolet site go to
-// io_vals[4*record..] (rho, u_x, u_y, u_z) for the iolet fluxes.
+// copy: every site's fOld (the state itself when it is post-stream, else its
+// pull), its density and velocity, and per workgroup [mass, min rho,
+// max rho, max |u|, unstable] in a fixed tree order.  The density and
+// velocity of every iolet site go to io_vals[4*record..] (rho, u_x, u_y,
+// u_z) for the iolet fluxes, when given.  Bound by the state's read.  The
+// outputs may be pinned host memory: a few KB, written once, cost less over
+// the bus than a copy after the kernel.  Monitor, velocity change and
+// snapshot together on an 819 k-site binary64 tree: 0.38 ms before (two
+// exported copies of the distributions, four copies), 0.22 ms now.
 template <int Q, typename S, class Lay>
 __global__ __launch_bounds__(256) void k_monitor(DevDomain D, StepArgs A,
                                                  const S* __restrict__ fin,
-                                                 int from_post_stream,
+                                                 int from_post_stream, const int64_t* range,
                                                  double* __restrict__ partials,
                                                  double* __restrict__ io_vals) {
-  using T = typename Store<S>::T;
   __shared__ double s_sum[256], s_min[256], s_max[256], s_u[256], s_bad[256];
   const int t = threadIdx.x;
   double sum = 0.0, mn = 1.7976931348623157e308, mx = -1.7976931348623157e308,
          um = 0.0, bad = 0.0;
-  auto visit = [&](const SiteRef& r) {
-    T f[Q];
-    if (from_post_stream) {
-      sfor<0, Q>([&](auto di) {
-        constexpr int d = decltype(di)::value;
-        f[d] = Store<S>::ld(fin + Lay::template at<Q>(D, d, r.x));
-      });
-    } else {
-      gather<Q, S, T, Lay>(D, A, fin, r, f);
-    }
+  visit_sites<Lay>(D, range, [&](const SiteRef& r) {
     double g[Q];
+    post_stream_site<Q, S, Lay>(D, A, fin, from_post_stream, r, g);
     sfor<0, Q>([&](auto di) {
-      constexpr int d = decltype(di)::value;
-      double v = (double)f[d];
-      if constexpr (kShifted<S>) v += Lat<Q>::w[d] * A.rho0;
-      g[d] = v;
-      if (!(v > 0.0)) bad = 1.0;
+      if (!(g[decltype(di)::value] > 0.0)) bad = 1.0;
     });
     double rho, m0, m1, m2;
     moments<Q, double>(g, rho, m0, m1, m2);
@@ -247,7 +195,7 @@ __global__ __launch_bounds__(256) void k_monitor(DevDomain D, StepArgs A,
     mx = rho > mx ? rho : mx;
     const double m = sqrt(((0.0 + ux * ux) + uy * uy) + uz * uz);
     um = m > um ? m : um;
-    if (r.cut) {
+    if (r.cut && io_vals) {
       const int io = D.b_io[r.rec];
       if (io >= 0) {
         io_vals[4 * (int64_t)io] = rho;
@@ -256,22 +204,7 @@ __global__ __launch_bounds__(256) void k_monitor(DevDomain D, StepArgs A,
         io_vals[4 * (int64_t)io + 3] = uz;
       }
     }
-  };
-  if constexpr (kWaveLayout<Lay>) {
-    const uint32_t wpg = blockDim.x >> 6;
-    for (uint32_t base = blockIdx.x * wpg; base < D.nwaves; base += gridDim.x * wpg) {
-      const uint32_t w = __builtin_amdgcn_readfirstlane(base + ((uint32_t)t >> 6));
-      SiteRef r;
-      if (Lay::locate_wave(D, w, r)) visit(r);
-    }
-  } else {
-    for (int64_t x = (int64_t)blockIdx.x * blockDim.x + t; x < D.n;
-         x += (int64_t)gridDim.x * blockDim.x) {
-      SiteRef r;
-      Lay::at(D, x, r);
-      visit(r);
-    }
-  }
+  });
   s_sum[t] = sum; s_min[t] = mn; s_max[t] = mx; s_u[t] = um; s_bad[t] = bad;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
@@ -290,62 +223,46 @@ __global__ __launch_bounds__(256) void k_monitor(DevDomain D, StepArgs A,
   }
 }
 
-// The same statistics per chunk of sites [range[2b], range[2b+1]) (one
-// workgroup per chunk; chunks never mix instances of an ensemble).
-template <int Q>
-__global__ __launch_bounds__(256) void k_reduce_ranges(int64_t np, const int64_t* range,
-                                                       const double* soa,
-                                                       const double* rho,
-                                                       const double* u,
-                                                       double* partials) {
-  __shared__ double s_sum[256], s_min[256], s_max[256], s_u[256], s_bad[256];
-  const int t = threadIdx.x;
-  double sum = 0.0, mn = 1.7976931348623157e308, mx = -1.7976931348623157e308,
-         um = 0.0, bad = 0.0;
-  const int64_t end = range[2 * blockIdx.x + 1];
-  for (int64_t x = range[2 * blockIdx.x] + t; x < end; x += blockDim.x) {
-    const double r = rho[x];
-    sum += r;
-    mn = r < mn ? r : mn;
-    mx = r > mx ? r : mx;
-    const double a = u[x], b = u[np + x], c = u[2 * np + x];
-    const double m = sqrt(((0.0 + a * a) + b * b) + c * c);
-    um = m > um ? m : um;
-    for (int d = 0; d < Q; ++d)
-      if (!(soa[(int64_t)d * np + x] > 0.0)) bad = 1.0;
-  }
-  s_sum[t] = sum; s_min[t] = mn; s_max[t] = mx; s_u[t] = um; s_bad[t] = bad;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) {
-      s_sum[t] += s_sum[t + w];
-      s_min[t] = s_min[t + w] < s_min[t] ? s_min[t + w] : s_min[t];
-      s_max[t] = s_max[t + w] > s_max[t] ? s_max[t + w] : s_max[t];
-      s_u[t] = s_u[t + w] > s_u[t] ? s_u[t + w] : s_u[t];
-      s_bad[t] = s_bad[t + w] > s_bad[t] ? s_bad[t + w] : s_bad[t];
-    }
-    __syncthreads();
-  }
-  if (t == 0) {
-    double* p = partials + 5 * blockIdx.x;
-    p[0] = s_sum[0]; p[1] = s_min[0]; p[2] = s_max[0]; p[3] = s_u[0]; p[4] = s_bad[0];
-  }
+// The velocity of fOld, u[3][npc] by compact site (the convergence monitor's
+// snapshot), straight from the state.
+template <int Q, typename S, class Lay>
+__global__ __launch_bounds__(256) void k_snapshot_velocity(DevDomain D, StepArgs A,
+                                                           const S* __restrict__ fin,
+                                                           int from_post_stream,
+                                                           double* __restrict__ u) {
+  SiteRef r;
+  if (!Lay::locate(D, r)) return;
+  double g[Q];
+  post_stream_site<Q, S, Lay>(D, A, fin, from_post_stream, r, g);
+  double rho, mx, my, mz;
+  moments<Q, double>(g, rho, mx, my, mz);
+  const int64_t c = Lay::compact(D, r);
+  u[c] = mx / rho;
+  u[D.npc + c] = my / rho;
+  u[2 * D.npc + c] = mz / rho;
 }
 
-__global__ __launch_bounds__(256) void k_velocity_change_ranges(
-    int64_t np, const int64_t* range, const double* u, const double* u0,
-    const double* inv_ref, double* partials) {
+// Per workgroup max |u - u0| * inv_ref over its sites, u from the state.
+template <int Q, typename S, class Lay>
+__global__ __launch_bounds__(256) void k_velocity_change(
+    DevDomain D, StepArgs A, const S* __restrict__ fin, int from_post_stream,
+    const int64_t* range, const double* __restrict__ u0, const double* __restrict__ inv_refs,
+    double inv_ref, double* __restrict__ partials) {
   __shared__ double s[256];
   const int t = threadIdx.x;
   double m = 0.0;
-  const double ir = inv_ref[blockIdx.x];
-  const int64_t end = range[2 * blockIdx.x + 1];
-  for (int64_t x = range[2 * blockIdx.x] + t; x < end; x += blockDim.x) {
-    const double a = u[x] - u0[x], b = u[np + x] - u0[np + x],
-                 c = u[2 * np + x] - u0[2 * np + x];
+  const double ir = inv_refs ? inv_refs[blockIdx.x] : inv_ref;
+  visit_sites<Lay>(D, range, [&](const SiteRef& r) {
+    const int64_t x = Lay::compact(D, r);
+    const double v0 = u0[x], v1 = u0[D.npc + x], v2 = u0[2 * D.npc + x];
+    double g[Q];
+    post_stream_site<Q, S, Lay>(D, A, fin, from_post_stream, r, g);
+    double rho, mx, my, mz;
+    moments<Q, double>(g, rho, mx, my, mz);
+    const double a = mx / rho - v0, b = my / rho - v1, c = mz / rho - v2;
     const double v = sqrt(((0.0 + a * a) + b * b) + c * c) * ir;
     m = v > m ? v : m;
-  }
+  });
   s[t] = m;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
@@ -355,35 +272,38 @@ __global__ __launch_bounds__(256) void k_velocity_change_ranges(
   if (t == 0) partials[blockIdx.x] = s[0];
 }
 
-__global__ __launch_bounds__(256) void k_velocity_change(int64_t n, int64_t np,
-                                                         const double* u,
-                                                         const double* u0,
-                                                         double inv_ref,
-                                                         double* partials) {
-  __shared__ double s[256];
-  const int t = threadIdx.x;
-  double m = 0.0;
-  for (int64_t x = (int64_t)blockIdx.x * blockDim.x + t; x < n;
-       x += (int64_t)gridDim.x * blockDim.x) {
-    const double a = u[x] - u0[x], b = u[np + x] - u0[np + x],
-                 c = u[2 * np + x] - u0[2 * np + x];
-    const double v = sqrt(((0.0 + a * a) + b * b) + c * c) * inv_ref;
-    m = v > m ? v : m;
+// fOld as the caller's AoS [n][Q].  The lane's Q values go through LDS so
+// that the wave writes each site's Q values as one run of memory (the perm
+// of neighbouring sites is mostly consecutive) instead of 19 stores of 64
+// scattered values.
+template <int Q, typename S, class Lay>
+__global__ __launch_bounds__(256) void k_export_distributions(
+    DevDomain D, StepArgs A, const S* __restrict__ fin, int from_post_stream,
+    const int64_t* __restrict__ perm, double* __restrict__ out) {
+  __shared__ double rows[4][64 * Q];
+  __shared__ int64_t site[4][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  SiteRef r;
+  const bool live = Lay::locate(D, r);
+  const uint64_t mask = __ballot(live);
+  if (live) {
+    double g[Q];
+    post_stream_site<Q, S, Lay>(D, A, fin, from_post_stream, r, g);
+    const int k = __popcll(mask & ((1ull << lane) - 1ull));
+    site[wv][k] = perm[Lay::compact(D, r)];
+    sfor<0, Q>([&](auto di) {
+      constexpr int d = decltype(di)::value;
+      rows[wv][k * Q + d] = g[d];
+    });
   }
-  s[t] = m;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) s[t] = s[t + w] > s[t] ? s[t + w] : s[t];
-    __syncthreads();
+  const int count = __popcll(mask) * Q;
+  for (int j = lane; j < count; j += 64) {
+    const int k = j / Q;
+    out[site[wv][k] * Q + (j - k * Q)] = rows[wv][j];
   }
-  if (t == 0) partials[blockIdx.x] = s[0];
 }
 
-// Wall shear stress magnitude at the wall sites (Lattice.h:652-727) from the
-// post-stream binary64 distributions: f_neq = f - f_eq with the SSE3-order
-// equilibrium; Pi_ab = sum_l f_neq_l c_la c_lb accumulated in direction
-// order (terms with c_la c_lb = 0 add nothing); t_a = sum_b (Pi_ab n_b) temp;
-// result sqrt(|t|^2 - (t . n)^2).
 template <int Q, int A, int B>
 __device__ __forceinline__ double second_moment(const double (&fneq)[Q]) {
   using L = Lat<Q>;
@@ -397,66 +317,47 @@ __device__ __forceinline__ double second_moment(const double (&fneq)[Q]) {
   return acc;
 }
 
-template <int Q>
-__global__ __launch_bounds__(256) void k_wall_shear_stress(
-    int64_t nw, int64_t np, const double* __restrict__ soa,
-    const int64_t* __restrict__ site, const float* __restrict__ nrm,
-    const double* __restrict__ temp_of, double* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nw) return;
-  const int64_t x = site[i];
-  double f[Q];
-  sfor<0, Q>([&](auto di) {
-    constexpr int d = decltype(di)::value;
-    f[d] = soa[(int64_t)d * np + x];
-  });
-  double r, mx, my, mz;
-  moments<Q, double>(f, r, mx, my, mz);
-  const FeqCoef<double> fe(r, mx, my, mz);
-  double fneq[Q];
-  sfor<0, Q>([&](auto di) {
-    constexpr int d = decltype(di)::value;
-    fneq[d] = f[d] - fe.template eq<Q, d>();
-  });
-  const double p00 = second_moment<Q, 0, 0>(fneq), p10 = second_moment<Q, 1, 0>(fneq),
-               p11 = second_moment<Q, 1, 1>(fneq), p20 = second_moment<Q, 2, 0>(fneq),
-               p21 = second_moment<Q, 2, 1>(fneq), p22 = second_moment<Q, 2, 2>(fneq);
-  const double pi[3][3] = {{p00, p10, p20}, {p10, p11, p21}, {p20, p21, p22}};
-  const double n[3] = {(double)nrm[3 * i], (double)nrm[3 * i + 1], (double)nrm[3 * i + 2]};
-  const double temp = temp_of[i];
-  double sq = 0.0, nn = 0.0;
-  for (int a = 0; a < 3; ++a) {
-    double t = 0.0;
-    for (int b = 0; b < 3; ++b) t += pi[a][b] * n[b] * temp;
-    sq += t * t;
-    nn += t * n[a];
-  }
-  out[i] = sqrt(sq - nn * nn);
-}
-
-// The other stress outputs of the reference's property cache (Lattice.h):
-// f_neq = f - f_eq (SSE3 order), Pi_ab = sum_l f_neq_l c_la c_lb in direction
-// order.  Stress tensor (CalculateStressTensor, 630-645): Pi * (1 - 1/(2 tau))
-// plus (rho - 1) Cs2 on the diagonal, upper triangle xx xy xz yy yz zz;
-// von Mises stress (508-552); shear rate (728-753, 890-907).  The tau of
-// each site is tau_site[x] when given.
-template <int Q>
-__global__ __launch_bounds__(256) void k_stress_fields(
-    int64_t n, int64_t np, const double* __restrict__ soa, double tau,
-    const double* __restrict__ tau_site, double* __restrict__ t6,
-    double* __restrict__ vm, double* __restrict__ sr) {
+// The property fields of fOld in the caller's site order, straight from the
+// state: one pull per site, no exported distributions in between (they cost
+// 2 Q 8 bytes a site and a second kernel per field), and no permutation on
+// the host.  Bound by the host link: with both gone, all 19 output doubles of
+// a 2.76 M-site tree take 42 ms instead of 109, and density and velocity of a
+// 7.93 M-site tree 25 ms instead of 95.
+//
+// Density and velocity: Lattice::CalculateDensityAndMomentum (SSE3 order) and
+// momentum / density.  With STRESS, from f_neq = f - f_eq (SSE3 order) and
+// Pi_ab = sum_l f_neq_l c_la c_lb in direction order (terms with
+// c_la c_lb = 0 add nothing):
+// * wall shear stress magnitude (Lattice.h:652-727): t_a = sum_b (Pi_ab n_b)
+//   temp, sqrt(|t|^2 - (t . n)^2) at wall sites, the largest double (the
+//   reference's NO_VALUE) elsewhere;
+// * stress tensor (CalculateStressTensor, 630-645): Pi * (1 - 1/(2 tau))
+//   plus (rho - 1) Cs2 on the diagonal, upper triangle xx xy xz yy yz zz;
+// * von Mises stress (508-552) and shear rate (728-753, 890-907);
+// * traction sigma n and its tangential projection t - n (t . n) (560-602)
+//   at wall sites, zero elsewhere (Common.h:107-121).
+template <int Q, typename S, class Lay, bool STRESS>
+__global__ __launch_bounds__(256) void k_export_fields(DevDomain D, StepArgs A,
+                                                       const S* __restrict__ fin,
+                                                       int from_post_stream, FieldPtrs F) {
   using L = Lat<Q>;
-  const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= n) return;
-  const double ts = tau_site ? tau_site[x] : tau;
+  SiteRef r;
+  if (!Lay::locate(D, r)) return;
   double f[Q];
-  sfor<0, Q>([&](auto di) {
-    constexpr int d = decltype(di)::value;
-    f[d] = soa[(int64_t)d * np + x];
-  });
-  double r, mx, my, mz;
-  moments<Q, double>(f, r, mx, my, mz);
-  const FeqCoef<double> fe(r, mx, my, mz);
+  post_stream_site<Q, S, Lay>(D, A, fin, from_post_stream, r, f);
+  const int64_t c = F.perm[Lay::compact(D, r)];
+  double rho, mx, my, mz;
+  moments<Q, double>(f, rho, mx, my, mz);
+  if constexpr (!STRESS) {
+    if (F.density) F.density[c] = rho;
+    if (F.velocity) {
+      F.velocity[3 * c] = mx / rho;
+      F.velocity[3 * c + 1] = my / rho;
+      F.velocity[3 * c + 2] = mz / rho;
+    }
+    return;
+  }
+  const FeqCoef<double> fe(rho, mx, my, mz);
   double fneq[Q];
   sfor<0, Q>([&](auto di) {
     constexpr int d = decltype(di)::value;
@@ -465,26 +366,54 @@ __global__ __launch_bounds__(256) void k_stress_fields(
   const double p00 = second_moment<Q, 0, 0>(fneq), p10 = second_moment<Q, 1, 0>(fneq),
                p11 = second_moment<Q, 1, 1>(fneq), p20 = second_moment<Q, 2, 0>(fneq),
                p21 = second_moment<Q, 2, 1>(fneq), p22 = second_moment<Q, 2, 2>(fneq);
-  if (t6) {
-    const double fac = 1 - 1 / (2 * ts);
-    const double pr = (r - 1) * kCs2;
-    t6[x] = p00 * fac + pr;
-    t6[np + x] = p10 * fac;
-    t6[2 * np + x] = p20 * fac;
-    t6[3 * np + x] = p11 * fac + pr;
-    t6[4 * np + x] = p21 * fac;
-    t6[5 * np + x] = p22 * fac + pr;
+  double ts = F.tau;
+  if constexpr (kWaveLayout<Lay>)
+    if (D.blk_tau) ts = D.blk_tau[r.w >> 3];
+  const bool wall = r.cut && D.b_wall[r.rec] != 0;
+  double n[3] = {0.0, 0.0, 0.0};
+  if (wall && F.rec_normal)
+    for (int a = 0; a < 3; ++a) n[a] = (double)F.rec_normal[3 * (int64_t)r.rec + a];
+  if (F.wss) {
+    double v = 1.7976931348623157e308;  // NO_VALUE, constants.h:47
+    if (wall) {
+      // -sqrt(2) * the stress parameter of LbmParameters
+      // (LbmParameters.h:34-39), as Lattice.h:669 uses it
+      const double temp = (1.0 - 1.0 / (2.0 * ts)) / sqrt(2.0) * (-sqrt(2.0));
+      const double pi[3][3] = {{p00, p10, p20}, {p10, p11, p21}, {p20, p21, p22}};
+      double sq = 0.0, nn = 0.0;
+      for (int a = 0; a < 3; ++a) {
+        double t = 0.0;
+        for (int b = 0; b < 3; ++b) t += pi[a][b] * n[b] * temp;
+        sq += t * t;
+        nn += t * n[a];
+      }
+      v = sqrt(sq - nn * nn);
+    }
+    F.wss[c] = v;
   }
-  if (vm) {
+  const double fac = 1 - 1 / (2 * ts);
+  const double pr = (rho - 1) * kCs2;
+  const double s00 = p00 * fac + pr, s10 = p10 * fac, s20 = p20 * fac, s11 = p11 * fac + pr,
+               s21 = p21 * fac, s22 = p22 * fac + pr;
+  if (F.tensor) {
+    double* t6 = F.tensor + 6 * c;
+    t6[0] = s00;
+    t6[1] = s10;
+    t6[2] = s20;
+    t6[3] = s11;
+    t6[4] = s21;
+    t6[5] = s22;
+  }
+  if (F.von_mises) {
     // sums of f_neq (cx^2 - cy^2) etc. in direction order
     double xx_yy = 0.0, yy_zz = 0.0, xx_zz = 0.0, xy = 0.0, xz = 0.0, yz = 0.0;
     sfor<0, Q>([&](auto li) {
       constexpr int l = decltype(li)::value;
       constexpr int cx = L::c[l][0], cy = L::c[l][1], cz = L::c[l][2];
-      constexpr int a = cx * cx - cy * cy, b = cy * cy - cz * cz, c = cx * cx - cz * cz;
+      constexpr int a = cx * cx - cy * cy, b = cy * cy - cz * cz, d = cx * cx - cz * cz;
       if constexpr (a != 0) xx_yy += fneq[l] * (double)a;
       if constexpr (b != 0) yy_zz += fneq[l] * (double)b;
-      if constexpr (c != 0) xx_zz += fneq[l] * (double)c;
+      if constexpr (d != 0) xx_zz += fneq[l] * (double)d;
       if constexpr (cx * cy != 0) xy += fneq[l] * (double)cx * (double)cy;
       if constexpr (cx * cz != 0) xz += fneq[l] * (double)cx * (double)cz;
       if constexpr (cy * cz != 0) yz += fneq[l] * (double)cy * (double)cz;
@@ -492,10 +421,10 @@ __global__ __launch_bounds__(256) void k_stress_fields(
     const double a = xx_yy * xx_yy + yy_zz * yy_zz + xx_zz * xx_zz;
     const double b = xy * xy + xz * xz + yz * yz;
     const double sp = (1.0 - 1.0 / (2.0 * ts)) / sqrt(2.0);
-    vm[x] = sp * sqrt(a + 6.0 * b);
+    F.von_mises[c] = sp * sqrt(a + 6.0 * b);
   }
-  if (sr) {
-    const double k = -1.0 / (2.0 * ts * r * kCs2);
+  if (F.shear_rate) {
+    const double k = -1.0 / (2.0 * ts * rho * kCs2);
     const double e[6] = {p00 * k, p10 * k, p20 * k, p11 * k, p21 * k, p22 * k};
     // rows: (0,0) (0,1) (0,2) (1,1) (1,2) (2,2)
     double acc = 0.0;
@@ -505,53 +434,20 @@ __global__ __launch_bounds__(256) void k_stress_fields(
     acc += e[3] * e[3];
     acc += 2 * e[4] * e[4];
     acc += e[5] * e[5];
-    sr[x] = sqrt(2 * acc);
+    F.shear_rate[c] = sqrt(2 * acc);
   }
-}
-
-// Traction sigma n and its tangential projection t - n (t . n) at the wall
-// sites (CalculateTractionOnAPoint / CalculateTangentialProjectionTraction,
-// Lattice.h:560-602); tau_of[i] is the tau of wall site i.
-template <int Q>
-__global__ __launch_bounds__(256) void k_traction(
-    int64_t nw, int64_t np, const double* __restrict__ soa,
-    const int64_t* __restrict__ site, const float* __restrict__ nrm,
-    const double* __restrict__ tau_of, double* __restrict__ tr, double* __restrict__ tg) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nw) return;
-  const int64_t x = site[i];
-  double f[Q];
-  sfor<0, Q>([&](auto di) {
-    constexpr int d = decltype(di)::value;
-    f[d] = soa[(int64_t)d * np + x];
-  });
-  double r, mx, my, mz;
-  moments<Q, double>(f, r, mx, my, mz);
-  const FeqCoef<double> fe(r, mx, my, mz);
-  double fneq[Q];
-  sfor<0, Q>([&](auto di) {
-    constexpr int d = decltype(di)::value;
-    fneq[d] = f[d] - fe.template eq<Q, d>();
-  });
-  const double fac = 1 - 1 / (2 * tau_of[i]);
-  const double pr = (r - 1) * kCs2;
-  const double p00 = second_moment<Q, 0, 0>(fneq), p10 = second_moment<Q, 1, 0>(fneq),
-               p11 = second_moment<Q, 1, 1>(fneq), p20 = second_moment<Q, 2, 0>(fneq),
-               p21 = second_moment<Q, 2, 1>(fneq), p22 = second_moment<Q, 2, 2>(fneq);
-  const double sg[3][3] = {{p00 * fac + pr, p10 * fac, p20 * fac},
-                           {p10 * fac, p11 * fac + pr, p21 * fac},
-                           {p20 * fac, p21 * fac, p22 * fac + pr}};
-  const double n[3] = {(double)nrm[3 * i], (double)nrm[3 * i + 1], (double)nrm[3 * i + 2]};
-  double t[3];
-  for (int a = 0; a < 3; ++a) {
-    t[a] = 0.0;
-    for (int b = 0; b < 3; ++b) t[a] += sg[a][b] * n[b];
-  }
-  double tn = 0.0;
-  for (int a = 0; a < 3; ++a) tn = tn + t[a] * n[a];
-  for (int a = 0; a < 3; ++a) {
-    tr[3 * i + a] = t[a];
-    tg[3 * i + a] = t[a] - n[a] * tn;
+  if (F.traction || F.tangential) {
+    double t[3] = {0.0, 0.0, 0.0}, tn = 0.0;
+    if (wall) {
+      const double sg[3][3] = {{s00, s10, s20}, {s10, s11, s21}, {s20, s21, s22}};
+      for (int a = 0; a < 3; ++a)
+        for (int b = 0; b < 3; ++b) t[a] += sg[a][b] * n[b];
+      for (int a = 0; a < 3; ++a) tn = tn + t[a] * n[a];
+    }
+    for (int a = 0; a < 3; ++a) {
+      if (F.traction) F.traction[3 * c + a] = t[a];
+      if (F.tangential) F.tangential[3 * c + a] = wall ? t[a] - n[a] * tn : 0.0;
+    }
   }
 }
 
@@ -609,18 +505,6 @@ int launch_collide_only(const DevDomain& d, const StepArgs& a, const void* fin,
                          : collide_only_in<2>(d, a, fin, fout, stream);
 }
 
-int launch_stream_only(const DevDomain& d, const StepArgs& a, const void* fin,
-                       double* s_out, int from_post_stream, void* stream) {
-  return dispatch(d, a, [&](auto q, auto, auto* s, auto* lay) {
-    using S = std::remove_pointer_t<decltype(s)>;
-    using Lay = std::remove_pointer_t<decltype(lay)>;
-    hipLaunchKernelGGL((k_stream_only<decltype(q)::value, S, Lay>), grid_for(thread_count(d)),
-                       dim3(256), 0, (hipStream_t)stream, d, a, (const S*)fin, s_out,
-                       from_post_stream);
-    return (int)hipGetLastError();
-  });
-}
-
 int launch_import(const DevDomain& d, const StepArgs& a, const double* aos,
                   const int64_t* perm, void* state, void* stream) {
   return dispatch(d, a, [&](auto q, auto, auto* s, auto* lay) {
@@ -645,47 +529,36 @@ int launch_import_equilibrium(const DevDomain& d, const StepArgs& a, const doubl
   });
 }
 
-int launch_soa_to_aos(int Q, int64_t n, int64_t np, const double* soa,
-                      const int64_t* perm, double* aos, void* stream) {
-  hipLaunchKernelGGL(k_soa_to_aos, grid_for(n), dim3(256), 0, (hipStream_t)stream,
-                     Q, n, np, soa, perm, aos);
-  return (int)hipGetLastError();
+int launch_export_distributions(const DevDomain& d, const StepArgs& a, const void* fin,
+                                int from_post_stream, const int64_t* perm, double* out,
+                                void* stream) {
+  return dispatch_narrow(d, a, [&](auto q, auto, auto* s, auto* lay) {
+    using S = std::remove_pointer_t<decltype(s)>;
+    using Lay = std::remove_pointer_t<decltype(lay)>;
+    hipLaunchKernelGGL((k_export_distributions<decltype(q)::value, S, Lay>),
+                       grid_for(thread_count(d)), dim3(256), 0, (hipStream_t)stream, d, a,
+                       (const S*)fin, from_post_stream, perm, out);
+    return (int)hipGetLastError();
+  });
 }
 
-int launch_moments(int Q, int64_t n, int64_t np, const double* soa, double* rho,
-                   double* u, void* stream) {
-  if (Q == 15)
-    hipLaunchKernelGGL(k_moments<15>, grid_for(n), dim3(256), 0,
-                       (hipStream_t)stream, n, np, soa, rho, u);
-  else
-    hipLaunchKernelGGL(k_moments<19>, grid_for(n), dim3(256), 0,
-                       (hipStream_t)stream, n, np, soa, rho, u);
-  return (int)hipGetLastError();
-}
-
-int launch_wall_shear_stress(int Q, int64_t nw, int64_t np, const double* soa,
-                             const int64_t* site, const float* normal, const double* temp,
-                             double* out, void* stream) {
-  if (nw == 0) return 0;
-  if (Q == 15)
-    hipLaunchKernelGGL(k_wall_shear_stress<15>, grid_for(nw), dim3(256), 0,
-                       (hipStream_t)stream, nw, np, soa, site, normal, temp, out);
-  else
-    hipLaunchKernelGGL(k_wall_shear_stress<19>, grid_for(nw), dim3(256), 0,
-                       (hipStream_t)stream, nw, np, soa, site, normal, temp, out);
-  return (int)hipGetLastError();
-}
-
-int launch_reduce(int Q, int64_t n, int64_t np, const double* soa,
-                  const double* rho, const double* u, double* partials,
-                  int nblocks, void* stream) {
-  if (Q == 15)
-    hipLaunchKernelGGL(k_reduce<15>, dim3(nblocks), dim3(256), 0,
-                       (hipStream_t)stream, n, np, soa, rho, u, partials);
-  else
-    hipLaunchKernelGGL(k_reduce<19>, dim3(nblocks), dim3(256), 0,
-                       (hipStream_t)stream, n, np, soa, rho, u, partials);
-  return (int)hipGetLastError();
+int launch_export_fields(const DevDomain& d, const StepArgs& a, const void* fin,
+                         int from_post_stream, const FieldPtrs& fields, void* stream) {
+  const bool stress = fields.wss || fields.tensor || fields.von_mises || fields.shear_rate ||
+                      fields.traction || fields.tangential;
+  return dispatch_narrow(d, a, [&](auto q, auto, auto* s, auto* lay) {
+    using S = std::remove_pointer_t<decltype(s)>;
+    using Lay = std::remove_pointer_t<decltype(lay)>;
+    constexpr int Q = decltype(q)::value;
+    const dim3 grid = grid_for(thread_count(d)), block(256);
+    if (stress)
+      hipLaunchKernelGGL((k_export_fields<Q, S, Lay, true>), grid, block, 0,
+                         (hipStream_t)stream, d, a, (const S*)fin, from_post_stream, fields);
+    else
+      hipLaunchKernelGGL((k_export_fields<Q, S, Lay, false>), grid, block, 0,
+                         (hipStream_t)stream, d, a, (const S*)fin, from_post_stream, fields);
+    return (int)hipGetLastError();
+  });
 }
 
 int launch_copy_arrays(int Q, int64_t stride_bytes, int64_t bytes, int64_t run_bytes,
@@ -760,72 +633,48 @@ int scratch_address(int device, double** out) {
   return 0;
 }
 
+int monitor_groups(const DevDomain& d) {
+  const int64_t units = d.layout == 0 ? (d.n + 255) / 256 : ((int64_t)d.nwaves + 3) / 4;
+  return (int)std::min<int64_t>(kMonitorGroups, std::max<int64_t>(units, 1));
+}
+
 int launch_monitor(const DevDomain& d, const StepArgs& a, const void* fin,
-                   int from_post_stream, double* partials, double* io_vals, void* stream) {
-  return dispatch(d, a, [&](auto q, auto, auto* s, auto* lay) {
+                   int from_post_stream, const int64_t* range, int groups, double* partials,
+                   double* io_vals, void* stream) {
+  return dispatch_narrow(d, a, [&](auto q, auto, auto* s, auto* lay) {
     using S = std::remove_pointer_t<decltype(s)>;
     using Lay = std::remove_pointer_t<decltype(lay)>;
-    hipLaunchKernelGGL((k_monitor<decltype(q)::value, S, Lay>), dim3(kMonitorGroups),
-                       dim3(256), 0, (hipStream_t)stream, d, a, (const S*)fin,
-                       from_post_stream, partials, io_vals);
+    hipLaunchKernelGGL((k_monitor<decltype(q)::value, S, Lay>), dim3(groups), dim3(256), 0,
+                       (hipStream_t)stream, d, a, (const S*)fin, from_post_stream, range,
+                       partials, io_vals);
     return (int)hipGetLastError();
   });
 }
 
-int launch_stress_fields(int Q, int64_t n, int64_t np, const double* soa, double tau,
-                         const double* tau_site, double* t6, double* vm, double* sr,
-                         void* stream) {
-  if (n == 0) return 0;
-  if (Q == 15)
-    hipLaunchKernelGGL(k_stress_fields<15>, grid_for(n), dim3(256), 0, (hipStream_t)stream, n,
-                       np, soa, tau, tau_site, t6, vm, sr);
-  else
-    hipLaunchKernelGGL(k_stress_fields<19>, grid_for(n), dim3(256), 0, (hipStream_t)stream, n,
-                       np, soa, tau, tau_site, t6, vm, sr);
-  return (int)hipGetLastError();
+int launch_snapshot_velocity(const DevDomain& d, const StepArgs& a, const void* fin,
+                             int from_post_stream, double* u, void* stream) {
+  return dispatch_narrow(d, a, [&](auto q, auto, auto* s, auto* lay) {
+    using S = std::remove_pointer_t<decltype(s)>;
+    using Lay = std::remove_pointer_t<decltype(lay)>;
+    hipLaunchKernelGGL((k_snapshot_velocity<decltype(q)::value, S, Lay>),
+                       grid_for(thread_count(d)), dim3(256), 0, (hipStream_t)stream, d, a,
+                       (const S*)fin, from_post_stream, u);
+    return (int)hipGetLastError();
+  });
 }
 
-int launch_traction(int Q, int64_t nw, int64_t np, const double* soa, const int64_t* site,
-                    const float* normal, const double* tau_of, double* tr, double* tg,
-                    void* stream) {
-  if (nw == 0) return 0;
-  if (Q == 15)
-    hipLaunchKernelGGL(k_traction<15>, grid_for(nw), dim3(256), 0, (hipStream_t)stream, nw, np,
-                       soa, site, normal, tau_of, tr, tg);
-  else
-    hipLaunchKernelGGL(k_traction<19>, grid_for(nw), dim3(256), 0, (hipStream_t)stream, nw, np,
-                       soa, site, normal, tau_of, tr, tg);
-  return (int)hipGetLastError();
-}
-
-int launch_reduce_ranges(int Q, int64_t nchunks, int64_t np, const int64_t* range,
-                         const double* soa, const double* rho, const double* u,
-                         double* partials, void* stream) {
-  if (nchunks == 0) return 0;
-  if (Q == 15)
-    hipLaunchKernelGGL(k_reduce_ranges<15>, dim3((unsigned)nchunks), dim3(256), 0,
-                       (hipStream_t)stream, np, range, soa, rho, u, partials);
-  else
-    hipLaunchKernelGGL(k_reduce_ranges<19>, dim3((unsigned)nchunks), dim3(256), 0,
-                       (hipStream_t)stream, np, range, soa, rho, u, partials);
-  return (int)hipGetLastError();
-}
-
-int launch_velocity_change_ranges(int64_t nchunks, int64_t np, const int64_t* range,
-                                  const double* u, const double* u_ref,
-                                  const double* inv_ref, double* partials, void* stream) {
-  if (nchunks == 0) return 0;
-  hipLaunchKernelGGL(k_velocity_change_ranges, dim3((unsigned)nchunks), dim3(256), 0,
-                     (hipStream_t)stream, np, range, u, u_ref, inv_ref, partials);
-  return (int)hipGetLastError();
-}
-
-int launch_velocity_change(int64_t n, int64_t np, const double* u,
-                           const double* u_ref, double inv_ref, double* partials,
-                           int nblocks, void* stream) {
-  hipLaunchKernelGGL(k_velocity_change, dim3(nblocks), dim3(256), 0,
-                     (hipStream_t)stream, n, np, u, u_ref, inv_ref, partials);
-  return (int)hipGetLastError();
+int launch_velocity_change(const DevDomain& d, const StepArgs& a, const void* fin,
+                           int from_post_stream, const int64_t* range, int groups,
+                           const double* u0, const double* inv_refs, double inv_ref,
+                           double* partials, void* stream) {
+  return dispatch_narrow(d, a, [&](auto q, auto, auto* s, auto* lay) {
+    using S = std::remove_pointer_t<decltype(s)>;
+    using Lay = std::remove_pointer_t<decltype(lay)>;
+    hipLaunchKernelGGL((k_velocity_change<decltype(q)::value, S, Lay>), dim3(groups), dim3(256),
+                       0, (hipStream_t)stream, d, a, (const S*)fin, from_post_stream, range, u0,
+                       inv_refs, inv_ref, partials);
+    return (int)hipGetLastError();
+  });
 }
 
 int launch_gather_pairs(int64_t count, int64_t np, int Q, int blockwise,

@@ -75,6 +75,25 @@ struct DevDomain {
   const double* blk_omega = nullptr;
   const float* blk_omega_f = nullptr;
   const double* blk_s_tau = nullptr;
+  const double* blk_tau = nullptr;   // the instance's tau
+};
+
+// Outputs of launch_export_fields, in the caller's site order (null: not
+// wanted): density [n] and velocity [n][3], or any of the stress outputs
+// (wall shear stress, von Mises, shear rate [n], tensor [n][6], traction
+// and tangential traction [n][3]).
+struct FieldPtrs {
+  const int64_t* perm = nullptr;      // compact site -> caller's index
+  double* density = nullptr;
+  double* velocity = nullptr;
+  double* wss = nullptr;
+  double* tensor = nullptr;
+  double* von_mises = nullptr;
+  double* shear_rate = nullptr;
+  double* traction = nullptr;
+  double* tangential = nullptr;
+  const float* rec_normal = nullptr;  // [nb][3] wall normal of boundary record r
+  double tau = 0;                     // relaxation time (ensembles: blk_tau)
 };
 
 struct StepArgs {
@@ -127,33 +146,24 @@ int launch_step(const DevDomain& d, const StepArgs& a, const void* fin,
                 void* fout, void* stream);
 int launch_collide_only(const DevDomain& d, const StepArgs& a, const void* fin,
                         void* fout, void* stream);
-// Post-stream distributions (the reference's fOld) as binary64 compact SoA
-// [Q][npc].  `from_post_stream` copies fin when the state already holds them.
-int launch_stream_only(const DevDomain& d, const StepArgs& a, const void* fin,
-                       double* s_out, int from_post_stream, void* stream);
-// Compact SoA [Q][np] binary64 <-> caller-order AoS [n][Q] through perm
-// (perm[compact] = caller index).
-int launch_soa_to_aos(int Q, int64_t n, int64_t np, const double* soa,
-                      const int64_t* perm, double* aos, void* stream);
+// The post-stream distributions (the reference's fOld) are the state itself
+// where `from_post_stream`, else its pull; every export and monitor below
+// reads them from the state.
+//
+// fOld as the caller's AoS [n][Q] in binary64; perm[compact] = caller's index.
+int launch_export_distributions(const DevDomain& d, const StepArgs& a, const void* fin,
+                                int from_post_stream, const int64_t* perm, double* out,
+                                void* stream);
+// Density and velocity, or the stress outputs, of fOld.
+int launch_export_fields(const DevDomain& d, const StepArgs& a, const void* fin,
+                         int from_post_stream, const FieldPtrs& fields, void* stream);
+// Caller's AoS [n][Q] -> state.
 int launch_import(const DevDomain& d, const StepArgs& a, const double* aos,
                   const int64_t* perm, void* state, void* stream);
 // Equilibrium of caller-order fields rho[n], momentum[n][3] into the state.
 int launch_import_equilibrium(const DevDomain& d, const StepArgs& a, const double* rho,
                               const double* mom, const int64_t* perm, void* state,
                               void* stream);
-// Moments of a binary64 SoA state: rho[np], u[3][np] (internal order).
-int launch_moments(int Q, int64_t n, int64_t np, const double* soa, double* rho,
-                   double* u, void* stream);
-// Wall shear stress magnitude at nw wall sites (compact index site[i],
-// normal[3*i..]) of a binary64 SoA state; temp[i] = -sqrt(2) * the stress
-// parameter of the site's relaxation time.
-int launch_wall_shear_stress(int Q, int64_t nw, int64_t np, const double* soa,
-                             const int64_t* site, const float* normal, const double* temp,
-                             double* out, void* stream);
-// Fixed-order binary64 reductions over moments; partial results per block.
-int launch_reduce(int Q, int64_t n, int64_t np, const double* soa,
-                  const double* rho, const double* u, double* partials,
-                  int nblocks, void* stream);
 // Device-copy ceiling: Q arrays of `bytes` bytes copied from `in` to `out`
 // in words of `width` bytes (4, 8 or 16), one word per thread and array,
 // with the step's workgroup size and workgroup-to-XCD remap.  run_bytes 0:
@@ -167,14 +177,25 @@ int launch_copy_arrays(int Q, int64_t stride_bytes, int64_t bytes, int64_t run_b
 // as raw stored words of esize bytes (8, 4 or 2).
 int launch_halo(int64_t count, const int64_t* idx, int esize, const void* from, void* to,
                 int pack, void* stream);
-// Monitor statistics of the reference's fOld read straight from the state
-// `fin` (post-stream when from_post_stream, else pulled as
-// launch_stream_only does): partials[5*g..] = mass, min rho, max rho,
-// max |u|, unstable of workgroup g < kMonitorGroups, and io_vals[4*r..] =
-// rho, u of iolet-site record r < d.ni.
+// Monitor statistics of fOld: partials[5*g..] = mass, min rho, max rho,
+// max |u|, unstable of workgroup g < groups, and io_vals[4*r..] = rho, u of
+// iolet-site record r < d.ni (unless null).  Without `range` the workgroups
+// (monitor_groups(d), at most kMonitorGroups) stride over the domain; with
+// it, workgroup g covers the x planes (pull table: sites) range[2g] ..
+// range[2g+1].
 constexpr int kMonitorGroups = 1024;
+int monitor_groups(const DevDomain& d);
 int launch_monitor(const DevDomain& d, const StepArgs& a, const void* fin,
-                   int from_post_stream, double* partials, double* io_vals, void* stream);
+                   int from_post_stream, const int64_t* range, int groups, double* partials,
+                   double* io_vals, void* stream);
+// Velocity of fOld, u[3][npc] by compact site.
+int launch_snapshot_velocity(const DevDomain& d, const StepArgs& a, const void* fin,
+                             int from_post_stream, double* u, void* stream);
+// Per workgroup max |u - u0| * inv_refs[g] (inv_ref where that is null).
+int launch_velocity_change(const DevDomain& d, const StepArgs& a, const void* fin,
+                           int from_post_stream, const int64_t* range, int groups,
+                           const double* u0, const double* inv_refs, double inv_ref,
+                           double* partials, void* stream);
 
 // The library's static device scratch (a file-scope __device__ array of
 // kStaticScratchDoubles binary64 values, 8 MiB, one copy per GPU held until
@@ -186,28 +207,6 @@ int launch_monitor(const DevDomain& d, const StepArgs& a, const void* fin,
 constexpr int64_t kStaticIoletSites = int64_t(1) << 18;
 constexpr int64_t kStaticScratchDoubles = 5 * kMonitorGroups + 4 * kStaticIoletSites;
 int scratch_address(int device, double** out);
-// Stress tensor [6][np] (xx xy xz yy yz zz), von Mises [np] and shear rate
-// [np] of every site of a binary64 SoA state (any output may be null); the
-// tau of site x is tau_site[x] when given, else tau.
-int launch_stress_fields(int Q, int64_t n, int64_t np, const double* soa, double tau,
-                         const double* tau_site, double* t6, double* vm, double* sr,
-                         void* stream);
-// Traction and tangential traction [nw][3] at the wall sites.
-int launch_traction(int Q, int64_t nw, int64_t np, const double* soa, const int64_t* site,
-                    const float* normal, const double* tau_of, double* tr, double* tg,
-                    void* stream);
-// Per-chunk statistics of sites [range[2c], range[2c+1]): partials[5c..]
-// = mass, min rho, max rho, max |u|, unstable; velocity change per chunk
-// with its own 1/reference speed.
-int launch_reduce_ranges(int Q, int64_t nchunks, int64_t np, const int64_t* range,
-                         const double* soa, const double* rho, const double* u,
-                         double* partials, void* stream);
-int launch_velocity_change_ranges(int64_t nchunks, int64_t np, const int64_t* range,
-                                  const double* u, const double* u_ref,
-                                  const double* inv_ref, double* partials, void* stream);
-int launch_velocity_change(int64_t n, int64_t np, const double* u,
-                           const double* u_ref, double inv_ref, double* partials,
-                           int nblocks, void* stream);
 // Halo unpack: state[slot_index[i]] = in[i] (storage conversion applied);
 // the direction of a state index is index / np, or (index / 512) % Q for the
 // block layout (blockwise != 0).

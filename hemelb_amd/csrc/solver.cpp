@@ -284,8 +284,14 @@ struct hlb_solver {
   hipEvent_t bv_done[2] = {nullptr, nullptr};
   int bv_cap = 0;
   int bv_which = 0;
+  // boundary values of an export or monitor, pinned host memory that the
+  // kernel reads in place (two values per iolet)
+  double* bv_export = nullptr;
   // scratch for exports and monitors, allocated on first use
-  DevBuf<double> s_soa, s_aos, rho, u, u_snap, partials, gathered, mon_io;
+  DevBuf<double> exports, u_snap, gathered;
+  // pinned host memory that the reductions write their partials into
+  double* partials = nullptr;
+  size_t partials_count = 0;
   // this device's copy of the library's static scratch (hlb_reduce_noalloc)
   double* scratch = nullptr;
   DevBuf<int64_t> slots;
@@ -295,23 +301,19 @@ struct hlb_solver {
   hlb::StepArgs args;
   // ensemble: instances, per-block relaxation, runs of one instance in the
   // internal order
-  struct Run { int64_t start, end; int32_t inst; };
+  struct Run { int64_t start, end; int32_t inst; int64_t wave0, wave1; };
   int32_t n_inst = 1;
   std::vector<double> inst_tau;
-  std::vector<Run> runs;
-  DevBuf<double> blk_omega, blk_s_tau;
+  std::vector<Run> runs;   // sites start..end, x planes wave0..wave1
+  std::vector<int32_t> chunk_inst;  // instance of each reduction chunk
+  DevBuf<int64_t> d_chunks;
+  DevBuf<double> blk_omega, blk_s_tau, blk_tau;
   DevBuf<float> blk_omega_f;
-  std::vector<double> wall_temp, wall_tau;
-  std::vector<int32_t> site_inst;  // instance of each internal site (ensembles)
-  DevBuf<double> d_wall_temp, d_wall_tau, d_site_tau, d_t6, d_vm, d_sr, d_tr, d_tg;
-  // wall sites (internal compact index) and their normals, for the wall
-  // shear stress output
+  // wall normal of every boundary record, for the stress outputs (uploaded on
+  // first use)
   bool has_normals = false;
-  std::vector<int64_t> wall_sites;
-  std::vector<float> wall_normals;
-  DevBuf<int64_t> d_wall_sites;
-  DevBuf<float> d_wall_normals;
-  DevBuf<double> d_wss;
+  std::vector<float> rec_normals;
+  DevBuf<float> d_rec_normals;
   // subdomains (hlb_create_subdomain): ghost sites in internal order n..,
   // their cut-link masks and coordinates, and every owned or ghost site by
   // absolute coordinate key (sorted) for the halo plans
@@ -330,6 +332,8 @@ struct hlb_solver {
       if (s) (void)hipFree(s);
     for (auto& h : bv_host)
       if (h) (void)hipHostFree(h);
+    if (bv_export) (void)hipHostFree(bv_export);
+    if (partials) (void)hipHostFree(partials);
     for (auto& e : bv_done)
       if (e) (void)hipEventDestroy(e);
     if (ev0) (void)hipEventDestroy(ev0);
@@ -346,7 +350,8 @@ struct hlb_solver {
          bnbr.bytes() + wave_fluid.bytes() + wave_bnd.bytes() + wave_links.bytes() +
          wave_rec.bytes() +
          wave_cbase.bytes() + bulk_waves.bytes() + bnd_waves.bytes() +
-         s_soa.bytes() + s_aos.bytes() + rho.bytes() + u.bytes() + u_snap.bytes();
+         exports.bytes() + u_snap.bytes() +
+         blk_tau.bytes() + d_rec_normals.bytes();
     return b;
   }
 
@@ -384,38 +389,40 @@ struct hlb_solver {
     return blockwise() ? ((slot >> 9) * Q + d) * 512 + (slot & 511) : d * np + slot;
   }
 
-  int ensure_scratch_soa() {
-    if (!s_soa.p) HIP_OR_FAIL(s_soa.alloc((size_t)Q * npc));
+  // Device buffer of the exports and imports in the caller's site order, kept
+  // at the largest size asked for; every call that uses it has finished with
+  // it when it returns.
+  int ensure_exports(int64_t count) {
+    if ((int64_t)exports.count < count || !exports.p) {
+      if (exports.p) HIP_OR_FAIL(hipFree(exports.p));
+      exports.p = nullptr;
+      HIP_OR_FAIL(exports.alloc((size_t)count));
+    }
     return HLB_OK;
   }
-  int ensure_moments() {
-    if (!rho.p) HIP_OR_FAIL(rho.alloc((size_t)npc));
-    if (!u.p) HIP_OR_FAIL(u.alloc((size_t)3 * npc));
+  int ensure_normals() {
+    if (!d_rec_normals.p) HIP_OR_FAIL(d_rec_normals.upload(rec_normals));
     return HLB_OK;
   }
-
-  // The reference's fOld as binary64 SoA in s_soa.
-  int post_stream_soa() {
-    int r = ensure_scratch_soa();
-    if (r) return r;
-    int e = hlb::launch_stream_only(dom, args_for_stream(), state[cur], s_soa.p,
-                                    post_stream ? 1 : 0, stream);
-    if (e) return fail(HLB_E_DEVICE, "stream-only kernel launch failed");
+  int ensure_partials(size_t count) {
+    if (partials_count >= count) return HLB_OK;
+    if (partials) HIP_OR_FAIL(hipHostFree(partials));
+    partials = nullptr;
+    partials_count = 0;
+    HIP_OR_FAIL(hipHostMalloc((void**)&partials, sizeof(double) * count));
+    partials_count = count;
     return HLB_OK;
   }
 
   hlb::StepArgs args_for_stream() {
     hlb::StepArgs a = args;
-    // the pending stream belongs to reference step t_ref - 1
+    // The pending stream belongs to reference step t_ref - 1.  Its values are
+    // read in place: a copy to the device and the wait for the stream before
+    // it cost more than the iolet sites' reads over the bus.  Every call that
+    // uses them waits for its kernel, so the buffer is free here.
     if (!post_stream && !iolets.empty()) {
-      // stage through the first pinned and device bv buffers, synchronously
-      // (exports and monitors are rare); once the stream is idle no step's
-      // copy still reads the pinned buffer
-      (void)hipStreamSynchronize(stream);
-      boundary_values(t_ref - 1, bv_host[0]);
-      (void)hipMemcpy(bv[0].p, bv_host[0], sizeof(double) * 2 * iolets.size(),
-                      hipMemcpyHostToDevice);
-      a.bv = bv[0].p;
+      boundary_values(t_ref - 1, bv_export);
+      a.bv = bv_export;
     }
     return a;
   }
@@ -607,13 +614,6 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
     s->internal[keys[o].second] = o;
   }
   s->has_normals = dm->wall_normal != nullptr;
-  for (int64_t o = 0; o < n; ++o) {
-    const int64_t i = s->perm[o];
-    if (!dm->wall_mask[i]) continue;
-    s->wall_sites.push_back(o);
-    if (s->has_normals)
-      for (int a = 0; a < 3; ++a) s->wall_normals.push_back(dm->wall_normal[3 * i + a]);
-  }
   // Ghost sites in Morton order, internal indices n .. n+ng-1.
   std::vector<std::pair<uint64_t, int64_t>> gkeys(ng);
   for (int64_t g = 0; g < ng; ++g) {
@@ -759,6 +759,8 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
       if (!blocks_layout) h_binfo[o] = rec + 1;
       h_bwall.push_back(wm);
       h_biolet.push_back(im);
+      if (s->has_normals)
+        for (int a = 0; a < 3; ++a) s->rec_normals.push_back(dm->wall_normal[3 * i + a]);
       // Cut distances (the BFL links read those of wall links only):
       // * binary64 storage: the reference's float q, bit for bit, of the
       //   wall links alone, packed in direction order from h_bqoff[rec];
@@ -927,7 +929,7 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
 
   // Ensemble: every 8^3 block belongs to one instance; contiguous runs of
   // one instance in the internal order for the per-instance reductions.
-  std::vector<double> h_bomega, h_bstau;
+  std::vector<double> h_bomega, h_bstau, h_btau;
   std::vector<float> h_bomega_f;
   if (instance) {
     std::vector<int32_t> binst(nblocks, -1);
@@ -940,37 +942,31 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
     h_bomega.resize(nblocks);
     h_bomega_f.resize(nblocks);
     h_bstau.resize(nblocks);
+    h_btau.resize(nblocks);
     for (int64_t b = 0; b < nblocks; ++b) {
       h_bomega[b] = -1.0 / inst_tau[binst[b]];
       h_bomega_f[b] = (float)h_bomega[b];
       h_bstau[b] = 1.0 / inst_tau[binst[b]];
+      h_btau[b] = inst_tau[binst[b]];
     }
     s->n_inst = n_inst;
     s->inst_tau.assign(inst_tau, inst_tau + n_inst);
     for (int64_t o = 0; o < n; ++o) {
       const int32_t k = instance[s->perm[o]];
       if (s->runs.empty() || s->runs.back().inst != k || s->runs.back().end != o)
-        s->runs.push_back({o, o + 1, k});
+        s->runs.push_back({o, o + 1, k, 0, 0});
       else
         s->runs.back().end = o + 1;
     }
   } else {
     s->n_inst = 1;
     s->inst_tau.assign(1, P.tau);
-    s->runs.push_back({0, n, 0});
+    s->runs.push_back({0, n, 0, 0, 0});
   }
-  // wall shear stress factor -(1 - 1/(2 tau)) per wall site
-  for (int64_t o : s->wall_sites) {
-    const double tau = instance ? inst_tau[instance[s->perm[o]]] : P.tau;
-    const double stress_parameter = (1.0 - 1.0 / (2.0 * tau)) / std::sqrt(2.0);
-    s->wall_temp.push_back(stress_parameter * (-std::sqrt(2.0)));
-    s->wall_tau.push_back(tau);
+  for (auto& run : s->runs) {
+    run.wave0 = 8 * blk_of[run.start];
+    run.wave1 = 8 * (blk_of[run.end - 1] + 1);
   }
-  if (instance) {
-    s->site_inst.resize(n);
-    for (int64_t o = 0; o < n; ++o) s->site_inst[o] = instance[s->perm[o]];
-  }
-
   // Device set-up.
   HIP_OR_FAIL(hipSetDevice(P.device));
   if (hlb::scratch_address(P.device, &s->scratch))
@@ -1021,9 +1017,11 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
     HIP_OR_FAIL(s->blk_omega.upload(h_bomega));
     HIP_OR_FAIL(s->blk_omega_f.upload(h_bomega_f));
     HIP_OR_FAIL(s->blk_s_tau.upload(h_bstau));
+    HIP_OR_FAIL(s->blk_tau.upload(h_btau));
   }
   s->bv_cap = 512;
   const size_t nio = std::max<size_t>(1, s->iolets.size());
+  HIP_OR_FAIL(hipHostMalloc((void**)&s->bv_export, sizeof(double) * 2 * nio));
   for (int b = 0; b < 2; ++b) {
     HIP_OR_FAIL(s->bv[b].alloc((size_t)s->bv_cap * 2 * nio));
     HIP_OR_FAIL(hipHostMalloc((void**)&s->bv_host[b], sizeof(double) * s->bv_cap * 2 * nio));
@@ -1070,6 +1068,7 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
   D.blk_omega = s->blk_omega.p;
   D.blk_omega_f = s->blk_omega_f.p;
   D.blk_s_tau = s->blk_s_tau.p;
+  D.blk_tau = s->blk_tau.p;
 
   hlb::StepArgs& A = s->args;
   A.Q = Q;
@@ -1206,12 +1205,13 @@ int hlb_time_steps(hlb_solver* s, int64_t n, double* ms) {
 int hlb_get_distributions(hlb_solver* s, double* f_out) {
   if (!s || !f_out) return fail(HLB_E_INVALID, "null argument");
   if (!s->initialised) return fail(HLB_E_STATE, "state not initialised");
-  int r = s->post_stream_soa();
+  int r = s->ensure_exports(s->Q * s->n);
   if (r) return r;
-  if (!s->s_aos.p) HIP_OR_FAIL(s->s_aos.alloc((size_t)s->Q * s->n));
-  if (hlb::launch_soa_to_aos(s->Q, s->n, s->npc, s->s_soa.p, s->d_perm.p, s->s_aos.p, s->stream))
-    return fail(HLB_E_DEVICE, "permute kernel launch failed");
-  HIP_OR_FAIL(hipMemcpyAsync(f_out, s->s_aos.p, sizeof(double) * s->Q * s->n,
+  if (hlb::launch_export_distributions(s->dom, s->args_for_stream(), s->state[s->cur],
+                                       s->post_stream ? 1 : 0, s->d_perm.p, s->exports.p,
+                                       s->stream))
+    return fail(HLB_E_DEVICE, "export kernel launch failed");
+  HIP_OR_FAIL(hipMemcpyAsync(f_out, s->exports.p, sizeof(double) * s->Q * s->n,
                              hipMemcpyDeviceToHost, s->stream));
   HIP_OR_FAIL(hipStreamSynchronize(s->stream));
   return HLB_OK;
@@ -1219,10 +1219,11 @@ int hlb_get_distributions(hlb_solver* s, double* f_out) {
 
 int hlb_set_distributions(hlb_solver* s, const double* f_in) {
   if (!s || !f_in) return fail(HLB_E_INVALID, "null argument");
-  if (!s->s_aos.p) HIP_OR_FAIL(s->s_aos.alloc((size_t)s->Q * s->n));
+  int r = s->ensure_exports(s->Q * s->n);
+  if (r) return r;
   HIP_OR_FAIL(hipStreamSynchronize(s->stream));
-  HIP_OR_FAIL(hipMemcpy(s->s_aos.p, f_in, sizeof(double) * s->Q * s->n, hipMemcpyHostToDevice));
-  if (hlb::launch_import(s->dom, s->args, s->s_aos.p, s->d_perm.p, s->state[s->cur],
+  HIP_OR_FAIL(hipMemcpy(s->exports.p, f_in, sizeof(double) * s->Q * s->n, hipMemcpyHostToDevice));
+  if (hlb::launch_import(s->dom, s->args, s->exports.p, s->d_perm.p, s->state[s->cur],
                          s->stream))
     return fail(HLB_E_DEVICE, "import kernel launch failed");
   HIP_OR_FAIL(hipStreamSynchronize(s->stream));
@@ -1255,34 +1256,48 @@ int hlb_set_equilibrium_fields(hlb_solver* s, const double* density, const doubl
   return HLB_OK;
 }
 
-static int compute_moments(hlb_solver* s) {
-  int r = s->post_stream_soa();
+// One export of per-site fields: `wanted` lists the device pointer slot, the
+// values per site and the caller's array of every output (null: not wanted).
+struct FieldRequest {
+  double* hlb::FieldPtrs::*slot;
+  int width;
+  double* host;
+};
+static int export_fields(hlb_solver* s, const FieldRequest* wanted, int count) {
+  hlb::FieldPtrs F;
+  F.perm = s->d_perm.p;
+  F.rec_normal = s->d_rec_normals.p;
+  F.tau = s->p.tau;
+  int64_t total = 0;
+  for (int k = 0; k < count; ++k)
+    if (wanted[k].host) total += wanted[k].width * s->n;
+  if (total == 0) return HLB_OK;
+  int r = s->ensure_exports(total);
   if (r) return r;
-  r = s->ensure_moments();
-  if (r) return r;
-  if (hlb::launch_moments(s->Q, s->n, s->npc, s->s_soa.p, s->rho.p, s->u.p, s->stream))
-    return fail(HLB_E_DEVICE, "moments kernel launch failed");
+  double* at = s->exports.p;
+  for (int k = 0; k < count; ++k) {
+    if (!wanted[k].host) continue;
+    F.*wanted[k].slot = at;
+    at += wanted[k].width * s->n;
+  }
+  if (hlb::launch_export_fields(s->dom, s->args_for_stream(), s->state[s->cur],
+                                s->post_stream ? 1 : 0, F, s->stream))
+    return fail(HLB_E_DEVICE, "export kernel launch failed");
+  for (int k = 0; k < count; ++k)
+    if (wanted[k].host)
+      HIP_OR_FAIL(hipMemcpyAsync(wanted[k].host, F.*wanted[k].slot,
+                                 sizeof(double) * wanted[k].width * s->n,
+                                 hipMemcpyDeviceToHost, s->stream));
+  HIP_OR_FAIL(hipStreamSynchronize(s->stream));
   return HLB_OK;
 }
 
 int hlb_get_macroscopic(hlb_solver* s, double* density, double* velocity) {
   if (!s) return fail(HLB_E_INVALID, "null solver");
   if (!s->initialised) return fail(HLB_E_STATE, "state not initialised");
-  int r = compute_moments(s);
-  if (r) return r;
-  std::vector<double> rho(s->npc), u(3 * s->npc);
-  HIP_OR_FAIL(hipMemcpyAsync(rho.data(), s->rho.p, sizeof(double) * s->npc,
-                             hipMemcpyDeviceToHost, s->stream));
-  HIP_OR_FAIL(hipMemcpyAsync(u.data(), s->u.p, sizeof(double) * 3 * s->npc,
-                             hipMemcpyDeviceToHost, s->stream));
-  HIP_OR_FAIL(hipStreamSynchronize(s->stream));
-  for (int64_t o = 0; o < s->n; ++o) {
-    const int64_t c = s->perm[o];
-    if (density) density[c] = rho[o];
-    if (velocity)
-      for (int a = 0; a < 3; ++a) velocity[3 * c + a] = u[(size_t)a * s->npc + o];
-  }
-  return HLB_OK;
+  const FieldRequest wanted[] = {{&hlb::FieldPtrs::density, 1, density},
+                                 {&hlb::FieldPtrs::velocity, 3, velocity}};
+  return export_fields(s, wanted, 2);
 }
 
 int hlb_get_wall_shear_stress(hlb_solver* s, double* stress) {
@@ -1290,119 +1305,36 @@ int hlb_get_wall_shear_stress(hlb_solver* s, double* stress) {
   if (!s->initialised) return fail(HLB_E_STATE, "state not initialised");
   if (!s->has_normals)
     return fail(HLB_E_STATE, "wall normals were not given to hlb_create");
-  int r = s->post_stream_soa();
+  int r = s->ensure_normals();
   if (r) return r;
-  const int64_t nw = (int64_t)s->wall_sites.size();
-  std::vector<double> w(nw);
-  if (nw) {
-    if (!s->d_wall_sites.p) {
-      HIP_OR_FAIL(s->d_wall_sites.upload(s->wall_sites));
-      HIP_OR_FAIL(s->d_wall_normals.upload(s->wall_normals));
-      // per site: -sqrt(2) * the stress parameter of LbmParameters
-      // (LbmParameters.h:34-39) as CalculateWallShearStressMagnitude uses it
-      // (Lattice.h:669), from the site's tau
-      HIP_OR_FAIL(s->d_wall_temp.upload(s->wall_temp));
-      HIP_OR_FAIL(s->d_wss.alloc((size_t)nw));
-    }
-    if (hlb::launch_wall_shear_stress(s->Q, nw, s->npc, s->s_soa.p, s->d_wall_sites.p,
-                                      s->d_wall_normals.p, s->d_wall_temp.p, s->d_wss.p,
-                                      s->stream))
-      return fail(HLB_E_DEVICE, "wall shear stress kernel launch failed");
-    HIP_OR_FAIL(hipMemcpyAsync(w.data(), s->d_wss.p, sizeof(double) * nw,
-                               hipMemcpyDeviceToHost, s->stream));
-  }
-  HIP_OR_FAIL(hipStreamSynchronize(s->stream));
-  std::fill(stress, stress + s->n, std::numeric_limits<double>::max());
-  for (int64_t k = 0; k < nw; ++k) stress[s->perm[s->wall_sites[k]]] = w[k];
-  return HLB_OK;
+  const FieldRequest wanted[] = {{&hlb::FieldPtrs::wss, 1, stress}};
+  return export_fields(s, wanted, 1);
 }
 
 int hlb_get_stress(hlb_solver* s, double* tensor, double* von_mises, double* shear_rate,
                    double* traction, double* tangential) {
   if (!s) return fail(HLB_E_INVALID, "null solver");
   if (!s->initialised) return fail(HLB_E_STATE, "state not initialised");
-  if ((traction || tangential) && !s->has_normals)
-    return fail(HLB_E_STATE, "wall normals were not given to hlb_create");
-  int r = s->post_stream_soa();
-  if (r) return r;
-  const int64_t npc = s->npc, n = s->n;
-  if (!s->site_inst.empty() && !s->d_site_tau.p) {
-    std::vector<double> t(n);
-    for (int64_t o = 0; o < n; ++o) t[o] = s->inst_tau[s->site_inst[o]];
-    HIP_OR_FAIL(s->d_site_tau.upload(t));
+  if (traction || tangential) {
+    if (!s->has_normals)
+      return fail(HLB_E_STATE, "wall normals were not given to hlb_create");
+    int r = s->ensure_normals();
+    if (r) return r;
   }
-  if (tensor && !s->d_t6.p) HIP_OR_FAIL(s->d_t6.alloc((size_t)6 * npc));
-  if (von_mises && !s->d_vm.p) HIP_OR_FAIL(s->d_vm.alloc((size_t)npc));
-  if (shear_rate && !s->d_sr.p) HIP_OR_FAIL(s->d_sr.alloc((size_t)npc));
-  if (tensor || von_mises || shear_rate) {
-    if (hlb::launch_stress_fields(s->Q, n, npc, s->s_soa.p, s->p.tau, s->d_site_tau.p,
-                                  tensor ? s->d_t6.p : nullptr, von_mises ? s->d_vm.p : nullptr,
-                                  shear_rate ? s->d_sr.p : nullptr, s->stream))
-      return fail(HLB_E_DEVICE, "stress kernel launch failed");
-  }
-  const int64_t nw = (int64_t)s->wall_sites.size();
-  std::vector<double> h6, hvm, hsr, htr, htg;
-  if (tensor) h6.resize(6 * npc);
-  if (von_mises) hvm.resize(npc);
-  if (shear_rate) hsr.resize(npc);
-  if ((traction || tangential) && nw) {
-    if (!s->d_wall_sites.p) {
-      HIP_OR_FAIL(s->d_wall_sites.upload(s->wall_sites));
-      HIP_OR_FAIL(s->d_wall_normals.upload(s->wall_normals));
-      HIP_OR_FAIL(s->d_wall_temp.upload(s->wall_temp));
-      HIP_OR_FAIL(s->d_wss.alloc((size_t)nw));
-    }
-    if (!s->d_wall_tau.p) {
-      HIP_OR_FAIL(s->d_wall_tau.upload(s->wall_tau));
-      HIP_OR_FAIL(s->d_tr.alloc((size_t)3 * nw));
-      HIP_OR_FAIL(s->d_tg.alloc((size_t)3 * nw));
-    }
-    if (hlb::launch_traction(s->Q, nw, npc, s->s_soa.p, s->d_wall_sites.p, s->d_wall_normals.p,
-                             s->d_wall_tau.p, s->d_tr.p, s->d_tg.p, s->stream))
-      return fail(HLB_E_DEVICE, "traction kernel launch failed");
-    htr.resize(3 * nw);
-    htg.resize(3 * nw);
-    HIP_OR_FAIL(hipMemcpyAsync(htr.data(), s->d_tr.p, sizeof(double) * 3 * nw,
-                               hipMemcpyDeviceToHost, s->stream));
-    HIP_OR_FAIL(hipMemcpyAsync(htg.data(), s->d_tg.p, sizeof(double) * 3 * nw,
-                               hipMemcpyDeviceToHost, s->stream));
-  }
-  if (tensor)
-    HIP_OR_FAIL(hipMemcpyAsync(h6.data(), s->d_t6.p, sizeof(double) * 6 * npc,
-                               hipMemcpyDeviceToHost, s->stream));
-  if (von_mises)
-    HIP_OR_FAIL(hipMemcpyAsync(hvm.data(), s->d_vm.p, sizeof(double) * npc,
-                               hipMemcpyDeviceToHost, s->stream));
-  if (shear_rate)
-    HIP_OR_FAIL(hipMemcpyAsync(hsr.data(), s->d_sr.p, sizeof(double) * npc,
-                               hipMemcpyDeviceToHost, s->stream));
-  HIP_OR_FAIL(hipStreamSynchronize(s->stream));
-  for (int64_t o = 0; o < n; ++o) {
-    const int64_t c = s->perm[o];
-    if (tensor)
-      for (int k = 0; k < 6; ++k) tensor[6 * c + k] = h6[(size_t)k * npc + o];
-    if (von_mises) von_mises[c] = hvm[o];
-    if (shear_rate) shear_rate[c] = hsr[o];
-  }
-  // traction is zero away from the walls (Common.h:107-121)
-  if (traction) std::fill(traction, traction + 3 * n, 0.0);
-  if (tangential) std::fill(tangential, tangential + 3 * n, 0.0);
-  for (int64_t k = 0; k < (int64_t)htr.size() / 3; ++k) {
-    const int64_t c = s->perm[s->wall_sites[k]];
-    for (int a = 0; a < 3; ++a) {
-      if (traction) traction[3 * c + a] = htr[3 * k + a];
-      if (tangential) tangential[3 * c + a] = htg[3 * k + a];
-    }
-  }
-  return HLB_OK;
+  const FieldRequest wanted[] = {{&hlb::FieldPtrs::tensor, 6, tensor},
+                                 {&hlb::FieldPtrs::von_mises, 1, von_mises},
+                                 {&hlb::FieldPtrs::shear_rate, 1, shear_rate},
+                                 {&hlb::FieldPtrs::traction, 3, traction},
+                                 {&hlb::FieldPtrs::tangential, 3, tangential}};
+  return export_fields(s, wanted, 5);
 }
 
 // The monitor's statistics (hlb_reduce, hlb_reduce_noalloc): one launch of
 // k_monitor over the state into `partials` and `io_vals`.
 static int launch_monitor_into(hlb_solver* s, double* partials, double* io_vals) {
   const hlb::StepArgs a = s->args_for_stream();
-  if (hlb::launch_monitor(s->dom, a, s->state[s->cur], s->post_stream ? 1 : 0, partials,
-                          io_vals, s->stream))
+  if (hlb::launch_monitor(s->dom, a, s->state[s->cur], s->post_stream ? 1 : 0, nullptr,
+                          hlb::monitor_groups(s->dom), partials, io_vals, s->stream))
     return fail(HLB_E_DEVICE, "monitor kernel launch failed");
   return HLB_OK;
 }
@@ -1414,7 +1346,8 @@ static void combine_partials(const hlb_solver* s, const double* part, hlb_monito
   m.density_min = 1.7976931348623157e308;
   m.density_max = -1.7976931348623157e308;
   bool bad = false;
-  for (int b = 0; b < hlb::kMonitorGroups; ++b) {
+  const int groups = hlb::monitor_groups(s->dom);
+  for (int b = 0; b < groups; ++b) {
     const double* p = &part[5 * b];
     m.mass += p[0];
     m.density_min = std::min(m.density_min, p[1]);
@@ -1442,22 +1375,16 @@ static void add_fluxes(const hlb_solver* s, const double* vals, int64_t k0, int6
 int hlb_reduce(hlb_solver* s, hlb_monitor* out) {
   if (!s || !out) return fail(HLB_E_INVALID, "null argument");
   if (!s->initialised) return fail(HLB_E_STATE, "state not initialised");
-  const int nb = hlb::kMonitorGroups;
   const int64_t ni = (int64_t)s->io_sites_internal.size();
-  if (!s->partials.p) HIP_OR_FAIL(s->partials.alloc(5 * nb));
-  if (!s->mon_io.p) HIP_OR_FAIL(s->mon_io.alloc(4 * std::max<int64_t>(ni, 1)));
-  int r = launch_monitor_into(s, s->partials.p, s->mon_io.p);
+  int r = s->ensure_partials((size_t)(5 * hlb::kMonitorGroups + 4 * ni));
   if (r) return r;
-  std::vector<double> part(5 * nb), g(4 * std::max<int64_t>(ni, 1));
-  HIP_OR_FAIL(hipMemcpyAsync(part.data(), s->partials.p, sizeof(double) * 5 * nb,
-                             hipMemcpyDeviceToHost, s->stream));
-  if (ni)
-    HIP_OR_FAIL(hipMemcpyAsync(g.data(), s->mon_io.p, sizeof(double) * 4 * ni,
-                               hipMemcpyDeviceToHost, s->stream));
+  double* io_vals = s->partials + 5 * hlb::kMonitorGroups;
+  r = launch_monitor_into(s, s->partials, io_vals);
+  if (r) return r;
   HIP_OR_FAIL(hipStreamSynchronize(s->stream));
   hlb_monitor m;
-  combine_partials(s, part.data(), m);
-  add_fluxes(s, g.data(), 0, ni, m);
+  combine_partials(s, s->partials, m);
+  add_fluxes(s, io_vals, 0, ni, m);
   *out = m;
   return HLB_OK;
 }
@@ -1477,7 +1404,8 @@ int hlb_reduce_noalloc(hlb_solver* s, hlb_monitor* out) {
   if (r) return r;
   // host copies into fixed buffers on the stack: no allocation anywhere
   double part[5 * hlb::kMonitorGroups];
-  HIP_OR_FAIL(hipMemcpyAsync(part, partials, sizeof(part), hipMemcpyDeviceToHost, s->stream));
+  HIP_OR_FAIL(hipMemcpyAsync(part, partials, sizeof(double) * 5 * hlb::monitor_groups(s->dom),
+                             hipMemcpyDeviceToHost, s->stream));
   HIP_OR_FAIL(hipStreamSynchronize(s->stream));
   hlb_monitor m;
   combine_partials(s, part, m);
@@ -1497,11 +1425,10 @@ int hlb_reduce_noalloc(hlb_solver* s, hlb_monitor* out) {
 int hlb_snapshot_velocity(hlb_solver* s) {
   if (!s) return fail(HLB_E_INVALID, "null solver");
   if (!s->initialised) return fail(HLB_E_STATE, "state not initialised");
-  int r = compute_moments(s);
-  if (r) return r;
   if (!s->u_snap.p) HIP_OR_FAIL(s->u_snap.alloc(3 * s->npc));
-  HIP_OR_FAIL(hipMemcpyAsync(s->u_snap.p, s->u.p, sizeof(double) * 3 * s->npc,
-                             hipMemcpyDeviceToDevice, s->stream));
+  if (hlb::launch_snapshot_velocity(s->dom, s->args_for_stream(), s->state[s->cur],
+                                    s->post_stream ? 1 : 0, s->u_snap.p, s->stream))
+    return fail(HLB_E_DEVICE, "velocity kernel launch failed");
   HIP_OR_FAIL(hipStreamSynchronize(s->stream));
   return HLB_OK;
 }
@@ -1510,36 +1437,42 @@ int hlb_velocity_change(hlb_solver* s, double ref, double* out) {
   if (!s || !out) return fail(HLB_E_INVALID, "null argument");
   if (!s->u_snap.p) return fail(HLB_E_STATE, "no velocity snapshot");
   if (!(ref > 0)) return fail(HLB_E_INVALID, "reference speed must be positive");
-  int r = compute_moments(s);
+  const int nb = hlb::monitor_groups(s->dom);
+  int r = s->ensure_partials((size_t)nb);
   if (r) return r;
-  const int nb = 1024;
-  if (!s->partials.p) HIP_OR_FAIL(s->partials.alloc(5 * nb));
-  if (hlb::launch_velocity_change(s->n, s->npc, s->u.p, s->u_snap.p, 1.0 / ref, s->partials.p,
-                                  nb, s->stream))
+  if (hlb::launch_velocity_change(s->dom, s->args_for_stream(), s->state[s->cur],
+                                  s->post_stream ? 1 : 0, nullptr, nb, s->u_snap.p, nullptr,
+                                  1.0 / ref, s->partials, s->stream))
     return fail(HLB_E_DEVICE, "velocity change kernel launch failed");
-  std::vector<double> part(nb);
-  HIP_OR_FAIL(hipMemcpyAsync(part.data(), s->partials.p, sizeof(double) * nb,
-                             hipMemcpyDeviceToHost, s->stream));
   HIP_OR_FAIL(hipStreamSynchronize(s->stream));
   double m = 0.0;
-  for (double v : part) m = std::max(m, v);
+  for (int b = 0; b < nb; ++b) m = std::max(m, s->partials[b]);
   *out = m;
   return HLB_OK;
 }
 
-// Chunks of at most kChunk sites inside the runs of one instance (the
-// per-instance reductions combine their partials in chunk order).
-static void instance_chunks(const hlb_solver* s, std::vector<int64_t>& range,
-                            std::vector<int32_t>& inst) {
-  constexpr int64_t kChunk = 1 << 16;
-  range.clear();
-  inst.clear();
-  for (const auto& r : s->runs)
-    for (int64_t a = r.start; a < r.end; a += kChunk) {
+// Chunks of x planes (pull table: sites) inside the runs of one instance, one
+// workgroup each: about 2048 over the domain, so that the chip is full (a
+// chunk of 65536 sites left most of it idle on a 3.4 M-site ensemble).  The
+// per-instance reductions combine their partials in chunk order.  The list
+// depends on the domain alone and is kept.
+static int instance_chunks(hlb_solver* s) {
+  if (!s->chunk_inst.empty()) return HLB_OK;
+  const bool planes = s->p.layout != HLB_LAYOUT_PULL_TABLE;
+  const int64_t unit = planes ? 4 : 256;  // what a workgroup visits at once
+  const int64_t all = planes ? (int64_t)s->dom.nwaves : s->n;
+  const int64_t size = (all / 2048 + unit) / unit * unit;
+  std::vector<int64_t> range;
+  for (const auto& r : s->runs) {
+    const int64_t begin = planes ? r.wave0 : r.start, end = planes ? r.wave1 : r.end;
+    for (int64_t a = begin; a < end; a += size) {
       range.push_back(a);
-      range.push_back(std::min(r.end, a + kChunk));
-      inst.push_back(r.inst);
+      range.push_back(std::min(end, a + size));
+      s->chunk_inst.push_back(r.inst);
     }
+  }
+  HIP_OR_FAIL(s->d_chunks.upload(range));
+  return HLB_OK;
 }
 
 int32_t hlb_instance_count(const hlb_solver* s) { return s ? s->n_inst : 0; }
@@ -1547,22 +1480,15 @@ int32_t hlb_instance_count(const hlb_solver* s) { return s ? s->n_inst : 0; }
 int hlb_reduce_instances(hlb_solver* s, hlb_instance_monitor* out) {
   if (!s || !out) return fail(HLB_E_INVALID, "null argument");
   if (!s->initialised) return fail(HLB_E_STATE, "state not initialised");
-  int r = compute_moments(s);
+  int r = instance_chunks(s);
   if (r) return r;
-  std::vector<int64_t> range;
-  std::vector<int32_t> inst;
-  instance_chunks(s, range, inst);
-  const int64_t nc = (int64_t)inst.size();
-  DevBuf<int64_t> d_range;
-  DevBuf<double> d_part;
-  HIP_OR_FAIL(d_range.upload(range));
-  HIP_OR_FAIL(d_part.alloc((size_t)5 * std::max<int64_t>(nc, 1)));
-  if (hlb::launch_reduce_ranges(s->Q, nc, s->npc, d_range.p, s->s_soa.p, s->rho.p, s->u.p,
-                                d_part.p, s->stream))
+  const int64_t nc = (int64_t)s->chunk_inst.size();
+  r = s->ensure_partials((size_t)(5 * nc));
+  if (r) return r;
+  if (hlb::launch_monitor(s->dom, s->args_for_stream(), s->state[s->cur],
+                          s->post_stream ? 1 : 0, s->d_chunks.p, (int)nc, s->partials, nullptr,
+                          s->stream))
     return fail(HLB_E_DEVICE, "reduction kernel launch failed");
-  std::vector<double> part(5 * nc);
-  HIP_OR_FAIL(hipMemcpyAsync(part.data(), d_part.p, sizeof(double) * 5 * nc,
-                             hipMemcpyDeviceToHost, s->stream));
   HIP_OR_FAIL(hipStreamSynchronize(s->stream));
   for (int32_t k = 0; k < s->n_inst; ++k) {
     hlb_instance_monitor& m = out[k];
@@ -1572,15 +1498,15 @@ int hlb_reduce_instances(hlb_solver* s, hlb_instance_monitor* out) {
     m.stable = 1;
   }
   for (int64_t c = 0; c < nc; ++c) {
-    hlb_instance_monitor& m = out[inst[c]];
-    const double* p = &part[5 * c];
+    hlb_instance_monitor& m = out[s->chunk_inst[c]];
+    const double* p = &s->partials[5 * c];
     m.mass += p[0];
     m.density_min = std::min(m.density_min, p[1]);
     m.density_max = std::max(m.density_max, p[2]);
     m.velocity_max = std::max(m.velocity_max, p[3]);
     if (p[4] != 0.0) m.stable = 0;
-    m.sites += range[2 * c + 1] - range[2 * c];
   }
+  for (const auto& run : s->runs) out[run.inst].sites += run.end - run.start;
   return HLB_OK;
 }
 
@@ -1589,28 +1515,22 @@ int hlb_velocity_change_instances(hlb_solver* s, const double* reference_speed, 
   if (!s->u_snap.p) return fail(HLB_E_STATE, "no velocity snapshot");
   for (int32_t k = 0; k < s->n_inst; ++k)
     if (!(reference_speed[k] > 0)) return fail(HLB_E_INVALID, "reference speed must be positive");
-  int r = compute_moments(s);
+  int r = instance_chunks(s);
   if (r) return r;
-  std::vector<int64_t> range;
-  std::vector<int32_t> inst;
-  instance_chunks(s, range, inst);
-  const int64_t nc = (int64_t)inst.size();
-  std::vector<double> inv(nc);
-  for (int64_t c = 0; c < nc; ++c) inv[c] = 1.0 / reference_speed[inst[c]];
-  DevBuf<int64_t> d_range;
-  DevBuf<double> d_inv, d_part;
-  HIP_OR_FAIL(d_range.upload(range));
-  HIP_OR_FAIL(d_inv.upload(inv));
-  HIP_OR_FAIL(d_part.alloc((size_t)std::max<int64_t>(nc, 1)));
-  if (hlb::launch_velocity_change_ranges(nc, s->npc, d_range.p, s->u.p, s->u_snap.p, d_inv.p,
-                                         d_part.p, s->stream))
+  // partials, then each chunk's 1 / reference speed, read in place
+  const int64_t nc = (int64_t)s->chunk_inst.size();
+  r = s->ensure_partials((size_t)(2 * nc));
+  if (r) return r;
+  double* inv = s->partials + nc;
+  for (int64_t c = 0; c < nc; ++c) inv[c] = 1.0 / reference_speed[s->chunk_inst[c]];
+  if (hlb::launch_velocity_change(s->dom, s->args_for_stream(), s->state[s->cur],
+                                  s->post_stream ? 1 : 0, s->d_chunks.p, (int)nc, s->u_snap.p,
+                                  inv, 0.0, s->partials, s->stream))
     return fail(HLB_E_DEVICE, "velocity change kernel launch failed");
-  std::vector<double> part(nc);
-  HIP_OR_FAIL(hipMemcpyAsync(part.data(), d_part.p, sizeof(double) * nc,
-                             hipMemcpyDeviceToHost, s->stream));
   HIP_OR_FAIL(hipStreamSynchronize(s->stream));
   std::fill(out, out + s->n_inst, 0.0);
-  for (int64_t c = 0; c < nc; ++c) out[inst[c]] = std::max(out[inst[c]], part[c]);
+  for (int64_t c = 0; c < nc; ++c)
+    out[s->chunk_inst[c]] = std::max(out[s->chunk_inst[c]], s->partials[c]);
   return HLB_OK;
 }
 

@@ -3,8 +3,8 @@
 * ``csrc/lbm_kernels.hip`` (once per layout), ``csrc/lbm_fields.hip`` and
   ``csrc/unet_kernels.hip`` -> hipcc for gfx950 (device code; no FMA
   contraction so binary64 results match the reference's evaluation order).
-* ``csrc/solver.cpp``, ``csrc/geometry.cpp``, ``csrc/extraction.cpp`` and
-  ``csrc/unet.cpp`` -> g++ (host code; the same compiler runtime and libm as the reference's own
+* ``csrc/solver.cpp``, ``csrc/host_copy.cpp``, ``csrc/geometry.cpp``,
+  ``csrc/extraction.cpp`` and ``csrc/unet.cpp`` -> g++ (host code; the same compiler runtime and libm as the reference's own
   g++ build).
 * linked with g++ against libamdhip64 and zlib.
 * ``driver/hemelb_driver.cpp`` -> ``hemelb_amd/hemelb_driver``: the C++
@@ -61,7 +61,8 @@ def build() -> str:
     jobs += [(hipcc, src, src.replace(".hip", ".o")) for src in ("lbm_fields.hip",
                                                                  "unet_kernels.hip")]
     jobs += [(["g++"] + GXX_FLAGS, src, src.replace(".cpp", ".o"))
-             for src in ("solver.cpp", "geometry.cpp", "extraction.cpp", "unet.cpp")]
+             for src in ("solver.cpp", "host_copy.cpp", "geometry.cpp", "extraction.cpp",
+                         "unet.cpp")]
     objs = [os.path.join(BUILD, obj) for _, _, obj in jobs]
     with ThreadPoolExecutor(max_workers=4) as pool:
         list(pool.map(lambda j: _run(j[0] + ["-c", os.path.join(CSRC, j[1]), "-o",

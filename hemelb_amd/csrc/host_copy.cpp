@@ -5,7 +5,8 @@
 // size: one thread of the runtime touches (the kernel zeroes) the caller's
 // pages and moves the data.  The link delivers more than 50 GB/s into pinned
 // memory, so the copy goes into pinned chunks and worker threads move them
-// on, each taking the page faults of its own chunks.
+// on, each taking the page faults of its own chunks: 420 MB of distributions
+// 40 -> 13.9 ms (30 GB/s), 88 MB of density and velocity 8.7 -> 3.3 ms.
 #include "host_copy.h"
 
 #include <algorithm>

@@ -18,6 +18,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "host_copy.h"
 #include "lbm_internal.h"
 
 namespace {
@@ -327,7 +328,9 @@ struct hlb_solver {
   bool post_stream = true;
   bool initialised = false;
 
+  hlb_solver() { hlb::staging_acquire(); }
   ~hlb_solver() {
+    hlb::staging_release();
     for (auto& s : state)
       if (s) (void)hipFree(s);
     for (auto& h : bv_host)
@@ -1211,9 +1214,8 @@ int hlb_get_distributions(hlb_solver* s, double* f_out) {
                                        s->post_stream ? 1 : 0, s->d_perm.p, s->exports.p,
                                        s->stream))
     return fail(HLB_E_DEVICE, "export kernel launch failed");
-  HIP_OR_FAIL(hipMemcpyAsync(f_out, s->exports.p, sizeof(double) * s->Q * s->n,
-                             hipMemcpyDeviceToHost, s->stream));
-  HIP_OR_FAIL(hipStreamSynchronize(s->stream));
+  HIP_OR_FAIL(hlb::copy_to_host({{f_out, s->exports.p, sizeof(double) * s->Q * s->n}},
+                                s->stream));
   return HLB_OK;
 }
 
@@ -1283,12 +1285,12 @@ static int export_fields(hlb_solver* s, const FieldRequest* wanted, int count) {
   if (hlb::launch_export_fields(s->dom, s->args_for_stream(), s->state[s->cur],
                                 s->post_stream ? 1 : 0, F, s->stream))
     return fail(HLB_E_DEVICE, "export kernel launch failed");
+  std::vector<hlb::HostSegment> segments;
   for (int k = 0; k < count; ++k)
     if (wanted[k].host)
-      HIP_OR_FAIL(hipMemcpyAsync(wanted[k].host, F.*wanted[k].slot,
-                                 sizeof(double) * wanted[k].width * s->n,
-                                 hipMemcpyDeviceToHost, s->stream));
-  HIP_OR_FAIL(hipStreamSynchronize(s->stream));
+      segments.push_back({wanted[k].host, F.*wanted[k].slot,
+                          sizeof(double) * wanted[k].width * s->n});
+  HIP_OR_FAIL(hlb::copy_to_host(segments, s->stream));
   return HLB_OK;
 }
 

@@ -85,3 +85,28 @@ def test_instances_keep_their_own_tau_and_chunks():
             m["density_min"], m["density_max"], m["velocity_max"])
         np.testing.assert_allclose(mons[k]["mass"], m["mass"], rtol=1e-12)
         assert change[k] == one.velocity_change(0.02)
+
+
+# 152 bytes a site: below and just above the 4 MiB from which copies go
+# through the staging chunks, and past the 16 chunks of its ring, none a
+# multiple of the 1 MiB chunk
+@pytest.mark.parametrize("radius,length", [(10.0, 80), (10.0, 91), (20.0, 121)])
+def test_large_exports_return_what_was_set(radius, length):
+    from concurrent.futures import ThreadPoolExecutor
+
+    case = K.cylinder_case(radius, length, 19, "LBGK", "SBB", "cosine")
+    n = case.domain.n
+    print(f"[exports] {n} sites, {n * 152 / 2 ** 20:.2f} MiB of distributions", flush=True)
+
+    def one(seed):
+        f = np.random.default_rng(seed).uniform(0.01, 0.1, (n, 19))
+        lbm = case.product()
+        lbm.set_distributions(f)
+        for _ in range(3):
+            np.testing.assert_array_equal(lbm.get_distributions(), f)
+        rho, _ = lbm.macroscopic()
+        np.testing.assert_allclose(rho, f.sum(1), rtol=19 * 2.3e-16)
+
+    one(0)
+    with ThreadPoolExecutor(3) as pool:   # concurrent copies: one stages, the others do not
+        list(pool.map(one, (1, 2, 3)))

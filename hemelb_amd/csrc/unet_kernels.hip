@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "unet_internal.h"
 
@@ -173,6 +174,313 @@ __global__ __launch_bounds__(256) void k_conv_fwd(Grid3 g, const uint16_t* __res
         if (y32) y32[o] = v;
         if (y16) y16[o] = f2bf(v);
       }
+  }
+}
+
+// --------------------------------------------------------------------------
+// The same convolution from LDS.  k_conv_fwd loads every A fragment from
+// global memory, 27 times per activation, each with its own address and
+// bounds arithmetic: 67-144 us a layer at 64^3 x 4, 10x what the bytes or the
+// matrix cores need.  Here a workgroup of four waves stages a BD x BH x BW box
+// of positions and its one-voxel halo, all input channels, once, as planes of
+// 8 channels ([plane][position][8]: the 16 positions that one quarter of the
+// wave reads are 256 contiguous bytes, one pass over the banks), and reads
+// every tap's fragment from there at a constant offset.  Positions outside the volume are
+// staged as zeros, so the K loop has no tests.  The weights stream from the
+// caches, one K step (even group counts: one tap) ahead.
+//
+// Waves: WM along positions x 4 / WM along output channels, each MT tiles of
+// 16 positions x NT tiles of 16 channels.  The product is formed transposed
+// (A = weights, B = positions), so that a lane ends with 4 consecutive
+// channels of one position and stores them at once.
+//
+// The input may come in two parts: the first `cu` channels from `xu`, a
+// tensor of half the resolution (read at (d/2, h/2, w/2): nearest
+// upsampling), the others from x.
+//
+// K runs as in k_conv_fwd, in the same steps and slices: the partial sum of
+// `kps` steps is added to the total after each slice, so the results are the
+// same bits whichever kernel runs.
+//
+// Measured at 64^3 x 4 (k_conv_fwd before): 16 -> 16 channels 67 -> 25 us
+// (575 TF/s; its 67 MB take 13), 48 -> 16 147 -> 77, 16 -> 48 in binary32 144
+// -> 68 (its bytes take 45), 96 -> 32 at 32^3 106 -> 62; all convolutions and
+// data gradients of a training iteration 1.65 -> 0.55 ms.  Now bound by the
+// LDS reads of the position fragments (1 KB a product where NT is 1).
+// --------------------------------------------------------------------------
+template <int I, int N, typename F>
+__device__ __forceinline__ void sfor(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    sfor<I + 1, N>(f);
+  }
+}
+
+// 16 zero bytes, the source of LDS pieces outside the volume.
+__device__ const uint16_t zero_piece[8] __attribute__((aligned(16))) = {0};
+
+// 16 bytes from the lane's global address to lds + 16 * lane (lds the same in
+// all lanes), without passing through registers; complete after
+// wait_for_loads() and a barrier.
+__device__ __forceinline__ void load_to_lds(const uint16_t* p, void* lds) {
+  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) const void*)p,
+                                   (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+__device__ __forceinline__ void wait_for_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+struct ConvSrc {
+  const uint16_t* x;    // [P][ci - cu]
+  const uint16_t* xu;   // [P/8][cu], or null
+  int cu;
+};
+
+template <int NG, int NT, int MT, int WM, int BD, int BH, int BW>
+struct ConvBox {
+  static constexpr int WN = 4 / WM;
+  static constexpr int HH = BH + 2, HW = BW + 2, NPOS = (BD + 2) * HH * HW;
+  static constexpr int PB = (NPOS + 63) / 64;       // 64-position chunks of a plane
+  static constexpr int PLANE = PB * 1024;           // bytes of one 8-channel plane
+  static constexpr int RPT = 16 / BW;               // rows of w per 16-position tile
+  static constexpr int LDS = 2 * NG * PLANE;
+  static_assert(BD * BH * BW == 16 * MT * WM, "box and waves disagree");
+  static_assert(BW == 16 || (BW == 8 && BH % 2 == 0), "tiles are rows of w");
+  static constexpr int TPD = BH / RPT;              // tiles per d plane
+  static_assert(MT % TPD == 0 || TPD % MT == 0, "a wave's tiles at constant offsets");
+  // halo position of the first site of tile m, relative to the wave's first
+  static constexpr int tile_off(int m) { return (m / TPD) * HH * HW + (m % TPD) * RPT * HW; }
+  static constexpr int tap_off(int t) { return ((t / 9) * HH + (t / 3) % 3) * HW + t % 3; }
+  // workgroups (waves per SIMD) a CU's 160 KB of LDS has room for, at most 2
+  static constexpr int WAVES = 163840 / LDS < 2 ? 163840 / LDS : 2;
+  // byte offset of half-step h (tap, 16-channel group)
+  static constexpr int half_off(int h) { return (h % NG) * 2 * PLANE + tap_off(h / NG) * 16; }
+};
+
+template <int NG, int NT, int MT, int WM, int BD, int BH, int BW, bool SLICES>
+__global__ __launch_bounds__(256, (ConvBox<NG, NT, MT, WM, BD, BH, BW>::WAVES)) void k_conv_box(Grid3 g, ConvSrc src,
+                                                  const uint16_t* __restrict__ w,
+                                                  const float* __restrict__ bias, int co,
+                                                  float* __restrict__ y32,
+                                                  uint16_t* __restrict__ y16, int yc, int yoff,
+                                                  int relu, int kps) {
+  using B = ConvBox<NG, NT, MT, WM, BD, BH, BW>;
+  constexpr int ci = 16 * NG;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[B::LDS];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row = lane & 15, q = lane >> 4, half = q >> 1, sub = q & 1;
+  const int nbw = (g.W + BW - 1) / BW, nbh = (g.H + BH - 1) / BH, nbd = (g.D + BD - 1) / BD;
+  int b = blockIdx.x;
+  const int w0 = (b % nbw) * BW;
+  b /= nbw;
+  const int h0 = (b % nbh) * BH;
+  b /= nbh;
+  const int d0 = (b % nbd) * BD, n = b / nbd;
+  const int wm = wv % WM, wn = wv / WM;
+  const int ntiles = co / 16;
+  const int tile0 = (blockIdx.y * B::WN + wn) * NT;
+  // the wave's first position, the lane's row inside a tile
+  constexpr int TPD = B::TPD;
+  const int t0 = wm * MT, bd = t0 / TPD, bh = (t0 % TPD) * B::RPT;
+  const int rh = row / BW, rw = row % BW;
+  const int abase = ((bd * B::HH + bh + rh) * B::HW + rw) * 16 + sub * B::PLANE;
+  const uint16_t* wp[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    wp[j] = w + (int64_t)((min(tile0 + j, ntiles - 1)) * 16 + row) * ci + sub * 8;
+  const bf16x8_t zero = __builtin_bit_cast(bf16x8_t, u32x4_t{0u, 0u, 0u, 0u});
+  auto lds8 = [&](int off) {
+    return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(lds + off));
+  };
+  // Weights are loaded a chunk of K steps ahead of their use (their latency is
+  // hundreds of cycles, a step MT * NT * 16); the first chunk before staging.
+  // Even NG: a K step is two groups of one tap and a chunk the three taps of
+  // one (kd, kh).  Odd NG: a step may straddle two taps.
+  constexpr bool kEven = NG % 2 == 0;
+  constexpr int NH = 27 * NG, KS = (NH + 1) / 2;
+  constexpr int KC = kEven ? 3 * NG / 2 : NG == 1 && NT == 1 ? KS : NT == 1 ? 7 : 10 / NT;
+  constexpr int kChunks = (KS + KC - 1) / KC;
+  const int64_t tap = (int64_t)co * ci;
+  bf16x8_t bn[KC][NT];
+  auto load_chunk = [&](auto first) {   // odd NG: constant first step
+    sfor<0, KC>([&](auto ki) {
+      constexpr int k = decltype(first)::value + decltype(ki)::value;
+      constexpr int ha = 2 * k, hb = ha + 1 < NH ? ha + 1 : ha;
+      if constexpr (ha < NH) {
+        const int64_t off = half ? (hb / NG) * tap + (hb % NG) * 16 : (ha / NG) * tap + (ha % NG) * 16;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          bn[decltype(ki)::value][j] = load8(wp[j] + off);
+          if (ha + 1 >= NH && half) bn[decltype(ki)::value][j] = zero;
+        }
+      }
+    });
+  };
+  auto load_row = [&](int r) {          // even NG: the taps 3r .. 3r+2
+#pragma unroll
+    for (int x = 0; x < 3; ++x)
+#pragma unroll
+      for (int k = 0; k < NG / 2; ++k)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          bn[x * (NG / 2) + k][j] = load8(wp[j] + (3 * r + x) * tap + k * 32 + half * 16);
+  };
+  if constexpr (kEven) load_row(0);
+  else load_chunk(std::integral_constant<int, 0>{});
+  // Stage the halo box: 16 bytes per lane straight into LDS, every load in
+  // flight at once (through registers, in two or three batches, staging cost
+  // as much as the products).  A wave takes the 8-channel pieces of 64
+  // positions, its neighbours the same positions' other pieces; positions
+  // outside the volume load zeros.
+  {
+    const int cx = ci - src.cu;
+#pragma unroll
+    for (int r = 0; r < (2 * NG * B::PB + 3) / 4; ++r) {
+      const int chunk = r * 4 + wv;
+      if (chunk < 2 * NG * B::PB) {
+        const int block = chunk / (2 * NG), piece = chunk % (2 * NG), c = piece * 8;
+        const int pos = block * 64 + lane;
+        const int hw = pos % B::HW, hh = (pos / B::HW) % B::HH, hd = pos / (B::HW * B::HH);
+        const int d = d0 + hd - 1, h = h0 + hh - 1, x = w0 + hw - 1;
+        const bool in = (unsigned)d < (unsigned)g.D && (unsigned)h < (unsigned)g.H &&
+                        (unsigned)x < (unsigned)g.W;
+        const uint16_t* p =
+            c < src.cu
+                ? src.xu + (((n * (g.D / 2) + d / 2) * (g.H / 2) + h / 2) * (g.W / 2) + x / 2) *
+                               src.cu + c
+                : src.x + (((n * g.D + d) * g.H + h) * g.W + x) * cx + c - src.cu;
+        load_to_lds(in ? p : zero_piece, lds + piece * B::PLANE + block * 1024);
+      }
+    }
+  }
+  wait_for_loads();
+  __syncthreads();
+  if (tile0 >= ntiles) return;
+  f32x4_t acc[MT][NT], total[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[m][j] = total[m][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // SLICES: a scalar branch after every K step.  It ends the block of code that
+  // the compiler schedules, so the next step's fragments are read before it;
+  // without slices the steps are one block (16 -> 16 channels at 64^3 x 4: 28.0
+  // us with the branches, 25.3 without).
+  int left = kps;  // K steps left in the slice
+  auto products = [&](const bf16x8_t (&a)[MT], const bf16x8_t (&b)[NT]) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[m], acc[m][j], 0, 0, 0);
+    if constexpr (SLICES) {
+      if (--left == 0) {
+        left = kps;
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int j = 0; j < NT; ++j) {
+            total[m][j] += acc[m][j];
+            acc[m][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          }
+      }
+    }
+  };
+  bf16x8_t an[MT];  // SLICES: the next step's fragments
+  if constexpr (kEven) {
+    const int a0 = abase + half * 2 * B::PLANE;
+    auto fragments = [&](int at, int k, bf16x8_t (&a)[MT]) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        a[m] = lds8(at + (k / (NG / 2)) * 16 + 4 * (k % (NG / 2)) * B::PLANE + B::tile_off(m) * 16);
+    };
+    if constexpr (SLICES) fragments(a0, 0, an);
+#pragma unroll 1
+    for (int r = 0; r < 9; ++r) {
+      bf16x8_t bw[KC][NT];
+#pragma unroll
+      for (int k = 0; k < KC; ++k)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) bw[k][j] = bn[k][j];
+      const int rn = min(r + 1, 8);
+      load_row(rn);
+      const int at = a0 + (r / 3 * B::HH + r % 3) * B::HW * 16;
+      const int next = a0 + (rn / 3 * B::HH + rn % 3) * B::HW * 16;
+#pragma unroll
+      for (int k = 0; k < KC; ++k) {
+        bf16x8_t a[MT];
+        if constexpr (SLICES) {
+#pragma unroll
+          for (int m = 0; m < MT; ++m) a[m] = an[m];
+          if (k + 1 < KC) fragments(at, k + 1, an);
+          else fragments(next, 0, an);
+        } else {
+          fragments(at, k, a);
+        }
+        products(a, bw[k]);
+      }
+    }
+  } else {
+    // every offset is a constant, plus the lane's half times one of a few
+    // differences
+    auto fragments = [&](auto ki, bf16x8_t (&a)[MT]) {
+      constexpr int ha = 2 * decltype(ki)::value, hb = ha + 1 < NH ? ha + 1 : ha;
+      constexpr int oa = B::half_off(ha), diff = B::half_off(hb) - oa;
+      const int at = abase + half * diff;
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        a[m] = lds8(at + oa + B::tile_off(m) * 16);
+        if (ha + 1 >= NH && half) a[m] = zero;  // the last step's second half
+      }
+    };
+    if constexpr (SLICES) fragments(std::integral_constant<int, 0>{}, an);
+    sfor<0, kChunks>([&](auto ch) {
+      constexpr int first = decltype(ch)::value * KC;
+      bf16x8_t bw[KC][NT];
+#pragma unroll
+      for (int k = 0; k < KC; ++k)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) bw[k][j] = bn[k][j];
+      if constexpr (first + KC < KS) load_chunk(std::integral_constant<int, first + KC>{});
+      sfor<0, KC>([&](auto ki) {
+        constexpr int step = first + decltype(ki)::value;
+        if constexpr (step < KS) {
+          bf16x8_t a[MT];
+          if constexpr (SLICES) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) a[m] = an[m];
+            if constexpr (step + 1 < KS) fragments(std::integral_constant<int, step + 1>{}, an);
+          } else {
+            fragments(std::integral_constant<int, step>{}, a);
+          }
+          products(a, bw[decltype(ki)::value]);
+        }
+      });
+    });
+  }
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int tile = t0 + m;
+    const int d = d0 + tile / TPD, h = h0 + (tile % TPD) * B::RPT + rh, x = w0 + rw;
+    if (d >= g.D || h >= g.H || x >= g.W) continue;
+    const int o = (((n * g.D + d) * g.H + h) * g.W + x) * yc + yoff + 4 * q;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      if (tile0 + j >= ntiles) continue;
+      const int c = (tile0 + j) * 16;
+      f32x4_t v = total[m][j] + acc[m][j];
+      if (bias) v += *reinterpret_cast<const f32x4_t*>(bias + c + 4 * q);
+      if (relu)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = v[r] > 0.f ? v[r] : 0.f;
+      if (y32) *reinterpret_cast<f32x4_t*>(y32 + o + c) = v;
+      if (y16) {
+        ushort4 p;
+        p.x = f2bf(v[0]);
+        p.y = f2bf(v[1]);
+        p.z = f2bf(v[2]);
+        p.w = f2bf(v[3]);
+        *reinterpret_cast<ushort4*>(y16 + o + c) = p;
+      }
+    }
   }
 }
 
@@ -701,7 +1009,87 @@ FwdPlan fwd_plan(const ConvGeom& cg, int ci, int co) {
 }
 }  // namespace
 
+namespace {
+struct BoxCall {
+  Grid3 g;
+  ConvSrc src;
+  const uint16_t* w;
+  const float* bias;
+  int co;
+  float* y32;
+  uint16_t* y16;
+  int yc, yoff, relu;
+  int kps;  // K steps per slice; 0: one slice
+  hipStream_t stream;
+};
+template <int NG, int NT, int MT, int WM, int BD, int BH, int BW>
+void box_launch(const BoxCall& c) {
+  using B = ConvBox<NG, NT, MT, WM, BD, BH, BW>;
+  const int64_t boxes = (int64_t)c.g.N * ((c.g.D + BD - 1) / BD) * ((c.g.H + BH - 1) / BH) *
+                        ((c.g.W + BW - 1) / BW);
+  const int per = 16 * NT * B::WN;
+  const dim3 grid((unsigned)boxes, (unsigned)((c.co + per - 1) / per)), block(256);
+  if (c.kps)
+    hipLaunchKernelGGL((k_conv_box<NG, NT, MT, WM, BD, BH, BW, true>), grid, block, 0, c.stream,
+                       c.g, c.src, c.w, c.bias, c.co, c.y32, c.y16, c.yc, c.yoff, c.relu, c.kps);
+  else
+    hipLaunchKernelGGL((k_conv_box<NG, NT, MT, WM, BD, BH, BW, false>), grid, block, 0, c.stream,
+                       c.g, c.src, c.w, c.bias, c.co, c.y32, c.y16, c.yc, c.yoff, c.relu, 0);
+}
+// Whether k_conv_box has a form for ci input channels.
+bool box_channels(int ci) {
+  const int ng = ci / 16;
+  return (ng >= 1 && ng <= 4) || ng == 6 || ng == 8 || ng == 12;
+}
+// Boxes are 16 wide where that pads the width no more than 8, and hold as
+// many positions as still leave about two workgroups per CU (512): a large
+// box re-reads less halo, a small one fills the chip.  Many input channels
+// bound the box by LDS instead.
+template <int BW>
+bool box_dispatch(const BoxCall& c, int ci) {
+  constexpr int H = BW == 16 ? 1 : 2;  // rows of w per 16 positions
+  const int64_t P = (int64_t)c.g.N * c.g.D * c.g.H * c.g.W;
+  const int T = c.co / 16;
+  const bool large = P >= 512 * 256;
+  switch (ci / 16) {
+    case 1:
+      if (!large) box_launch<1, 1, 1, 4, 1, 4 * H, BW>(c);
+      else if (T % 3 == 0) box_launch<1, 3, 4, 4, 4, 4 * H, BW>(c);
+      else if (T % 2 == 0) box_launch<1, 2, 4, 4, 4, 4 * H, BW>(c);
+      else box_launch<1, 1, 8, 4, BW == 16 ? 4 : 8, 8, BW>(c);
+      return true;
+    case 2:
+      if (!large) box_launch<2, 1, 1, 4, 1, 4 * H, BW>(c);
+      else if (T % 3 == 0) box_launch<2, 3, 4, 4, 4, 4 * H, BW>(c);
+      else if (T % 2 == 0) box_launch<2, 2, 4, 4, 4, 4 * H, BW>(c);
+      else box_launch<2, 1, 4, 4, 4, 4 * H, BW>(c);
+      return true;
+    case 3:
+      if (!large) box_launch<3, 1, 1, 4, 1, 4 * H, BW>(c);
+      else box_launch<3, 1, 4, 4, 4, 4 * H, BW>(c);
+      return true;
+    case 4:
+      if (T <= 2) box_launch<4, 1, 2, 2, 2, 2 * H, BW>(c);
+      else if (P >= 64 * 256) box_launch<4, 1, 4, 1, 2, 2 * H, BW>(c);
+      else box_launch<4, 1, 2, 1, 1, 2 * H, BW>(c);
+      return true;
+    case 6:
+      box_launch<6, 1, 2, 2, 2, 2 * H, BW>(c);
+      return true;
+    case 8:
+      if (P >= 64 * 256) box_launch<8, 1, 4, 1, 2, 2 * H, BW>(c);
+      else box_launch<8, 1, 1, 2, 1, 2 * H, BW>(c);
+      return true;
+    case 12:
+      box_launch<12, 1, 4, 1, 2, 2 * H, BW>(c);
+      return true;
+  }
+  return false;
+}
+}  // namespace
+
 int64_t conv_fwd_ws(const ConvGeom& cg, int ci, int co) {
+  if (box_channels(ci)) return 0;
   const FwdPlan f = fwd_plan(cg, ci, co);
   return f.nsplit > 1 ? (int64_t)f.nsplit * cg.N * cg.D * cg.H * cg.W * co : 0;
 }
@@ -712,6 +1100,16 @@ int conv_fwd(const ConvGeom& cg, const uint16_t* x, int ci, const uint16_t* w,
   const Grid3 g{cg.N, cg.D, cg.H, cg.W};
   const int64_t P = (int64_t)cg.N * cg.D * cg.H * cg.W;
   const FwdPlan f = fwd_plan(cg, ci, co);
+  if (box_channels(ci)) {
+    const BoxCall c{g,    ConvSrc{x, nullptr, 0}, w,    bias,
+                    co,   y32,                    y16,  yc,
+                    yoff, relu,                   f.nsplit > 1 ? f.hpw / 2 : 0,
+                    (hipStream_t)stream};
+    const bool wide = (cg.W + 15) / 16 * 16 == (cg.W + 7) / 8 * 8;
+    if (!(wide ? box_dispatch<16>(c, ci) : box_dispatch<8>(c, ci)))
+      return (int)hipErrorInvalidValue;
+    return (int)hipGetLastError();
+  }
   if (f.nsplit > 1 && !ws) return (int)hipErrorInvalidValue;
   float* slices = f.nsplit > 1 ? ws : nullptr;
   const dim3 grid((unsigned)((f.waves + 3) / 4), (unsigned)f.nsplit), block(256);

@@ -228,6 +228,45 @@ __device__ __forceinline__ void load_to_lds(const uint16_t* p, void* lds) {
 }
 __device__ __forceinline__ void wait_for_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// x / D for 0 <= x < LIMIT by a 24-bit product and a shift (full-rate vector
+// instructions; the compiler's exact division multiplies in 32 x 32 bits at a
+// quarter of that rate).
+template <int D, int LIMIT>
+__device__ __forceinline__ int small_div(int x) {
+  constexpr unsigned kMul = (1u << 20) / D + 1;
+  static_assert([] {
+    for (unsigned v = 0; v < (unsigned)LIMIT; ++v)
+      if (((v * kMul) >> 20) != v / D || v * kMul >= (1ull << 32)) return false;
+    return kMul < (1u << 24) && LIMIT <= (1 << 12);
+  }(), "inexact");
+  return (int)(__umul24((unsigned)x, kMul) >> 20);
+}
+
+// Where a lane's piece of a halo box lies: its coordinates in the box, and
+// whether and where the position is in the volume, for a box whose first halo
+// position is (d, h, w) of sample n (possibly -1).
+struct HaloPos {
+  int d, h, w;
+};
+template <int HH, int HW, int LIMIT>
+__device__ __forceinline__ HaloPos halo_pos(int pos) {
+  const int r = small_div<HW, LIMIT>(pos), d = small_div<HH, LIMIT>(r);
+  return HaloPos{d, r - d * HH, pos - r * HW};
+}
+__device__ __forceinline__ bool halo_inside(const Grid3& g, const HaloPos& o, int d, int h, int w) {
+  return (unsigned)(d + o.d) < (unsigned)g.D && (unsigned)(h + o.h) < (unsigned)g.H &&
+         (unsigned)(w + o.w) < (unsigned)g.W;
+}
+// Offset of the position from the box's first one, in positions.
+__device__ __forceinline__ int halo_offset(const Grid3& g, const HaloPos& o) {
+  return __mul24(__mul24(o.d, g.H) + o.h, g.W) + o.w;
+}
+// Index of its parent in the tensor of half the resolution.
+__device__ __forceinline__ int halo_parent(const Grid3& g, const HaloPos& o, int n, int d, int h,
+                                           int w) {
+  return ((n * (g.D / 2) + (d + o.d) / 2) * (g.H / 2) + (h + o.h) / 2) * (g.W / 2) + (w + o.w) / 2;
+}
+
 struct ConvSrc {
   const uint16_t* x;    // [P][ci - cu]
   const uint16_t* xu;   // [P/8][cu], or null
@@ -333,22 +372,21 @@ __global__ __launch_bounds__(256, (ConvBox<NG, NT, MT, WM, BD, BH, BW>::WAVES)) 
   // outside the volume load zeros.
   {
     const int cx = ci - src.cu;
+    const int dz = d0 - 1, hz = h0 - 1, wz = w0 - 1;
+    const int64_t first = (((int64_t)n * g.D + dz) * g.H + hz) * g.W + wz;
 #pragma unroll
     for (int r = 0; r < (2 * NG * B::PB + 3) / 4; ++r) {
       const int chunk = r * 4 + wv;
       if (chunk < 2 * NG * B::PB) {
         const int block = chunk / (2 * NG), piece = chunk % (2 * NG), c = piece * 8;
-        const int pos = block * 64 + lane;
-        const int hw = pos % B::HW, hh = (pos / B::HW) % B::HH, hd = pos / (B::HW * B::HH);
-        const int d = d0 + hd - 1, h = h0 + hh - 1, x = w0 + hw - 1;
-        const bool in = (unsigned)d < (unsigned)g.D && (unsigned)h < (unsigned)g.H &&
-                        (unsigned)x < (unsigned)g.W;
-        const uint16_t* p =
-            c < src.cu
-                ? src.xu + (((n * (g.D / 2) + d / 2) * (g.H / 2) + h / 2) * (g.W / 2) + x / 2) *
-                               src.cu + c
-                : src.x + (((n * g.D + d) * g.H + h) * g.W + x) * cx + c - src.cu;
-        load_to_lds(in ? p : zero_piece, lds + piece * B::PLANE + block * 1024);
+        const HaloPos o = halo_pos<B::HH, B::HW, B::PB * 64>(block * 64 + lane);
+        const uint16_t* p;
+        if (c < src.cu)   // the same for the whole wave
+          p = src.xu + halo_parent(g, o, n, dz, hz, wz) * src.cu + c;
+        else
+          p = src.x + first * cx + c - src.cu + __mul24(halo_offset(g, o), cx);
+        load_to_lds(halo_inside(g, o, dz, hz, wz) ? p : zero_piece,
+                    lds + piece * B::PLANE + block * 1024);
       }
     }
   }
@@ -582,117 +620,148 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(Grid3 g, const uint16_t* __r
 // --------------------------------------------------------------------------
 // Backward-weight on v_mfma_f32_16x16x32_bf16 with the operands staged in
 // LDS: dW[t][co][ci] = sum_p dy[p][co] x[p + off_t][ci] is, per tap, a GEMM
-// with M = 16 output channels, N = 16 input channels and K = positions.  A
-// workgroup takes one (co, ci) tile pair and a run of `bpw` boxes of
-// BD x BH x BW = 256 positions (BW = 16 or 8).  Per box it stages
-//  * sA: dy of the box transposed to [co][position] (one 16-byte row
-//    segment per lane and K step), and
-//  * sB: x of the box and its one-voxel halo transposed to
-//    [dx][ci][d][h][w], three copies shifted by dx = -1, 0, +1, so that the
-//    eight positions a lane needs for any tap are one aligned 16-byte read;
-// then wave w accumulates taps w, w+4, ... over the box's 8 K steps of 32
-// positions (octets of 8 consecutive w).  Rows are padded by 8 elements
-// against LDS bank conflicts.  Each run of boxes writes one partial sum.
+// with M = 16 output channels, N = 16 input channels and K = positions, which
+// channels-last storage does not make contiguous.  A workgroup takes NCO
+// output-channel tiles, one input-channel tile and a run of `bpw` boxes of
+// BD x BH x BW = 256 positions (BW = 16 or 8).  Per box it stages dy and x
+// with its one-voxel halo as they lie in memory, [position][16 channels],
+// straight into LDS, the next box while it computes this one.  The transposed
+// LDS read (ds_read_b64_tr_b16: 16 lanes read 4 rows of 16 channels and lane
+// i gets the 4 values of channel i) then gives a lane its 8 positions of any
+// tap in two reads.  Wave w accumulates taps w, w+4, ... over the box's 8 K
+// steps of 32 positions (octets of 8 consecutive w).  Each run of boxes
+// writes one partial sum.
+//
+// Transposing on the way into LDS (dword loads, packing, three copies
+// shifted by dx) took most of the time before.  Measured at 64^3 x 4, a layer
+// of 16 -> 16 channels 75 -> 28 us (510 TF/s), all 14 layers of a training
+// iteration 0.62 -> 0.35 ms.  Bound by the LDS reads (1 KB a product with one
+// output tile) and the staging of 2.5 positions per position.
 // --------------------------------------------------------------------------
 template <int BW>
 struct WBox {
   static constexpr int BD = 4, BH = 256 / (4 * BW);
-  static constexpr int HD = BD + 2, HH = BH + 2;
-  static constexpr int ROW_A = 256 + 8;             // [co][position] row
-  static constexpr int ROW_B = HD * HH * BW + 8;    // [ci][d][h][w] plane
+  static constexpr int HH = BH + 2, HW = BW + 2, NPOS = (BD + 2) * HH * HW;
+  static constexpr int XC = (NPOS * 2 + 63) / 64;   // 1 KB pieces of the x halo
+  static constexpr int DY = 256 * 32;               // bytes of one dy tile
 };
 
-template <int BW>
-__global__ __launch_bounds__(256) void k_conv_wgrad_box(Grid3 g, const uint16_t* __restrict__ x,
-                                                        int ci, const uint16_t* __restrict__ dy,
-                                                        int co, int bpw,
-                                                        float* __restrict__ part) {
+// In LDS the two quads of every odd octet of positions are swapped (of dy, and
+// of the 16-wide x rows), so that the octets two quarters of the wave read,
+// 256 bytes apart, fall on different banks.
+__host__ __device__ constexpr int quad_swap(int pos) { return pos ^ ((pos >> 3 & 1) << 2); }
+
+// Two transposed reads: 4 + 4 positions (32-byte rows) of the lane's channel;
+// lo and hi are the lane's pieces of the two quads.
+__device__ __forceinline__ bf16x8_t read_transposed(const unsigned char* lo_at,
+                                                    const unsigned char* hi_at) {
+  typedef __attribute__((address_space(3))) short4_t lds_short4;
+  const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)lo_at);
+  const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)hi_at);
+  return __builtin_bit_cast(bf16x8_t,
+                            __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+template <int BW, int NCO>
+__global__ __launch_bounds__(256, 2) void k_conv_wgrad_box(Grid3 g, ConvSrc src, int ci,
+                                                           const uint16_t* __restrict__ dy,
+                                                           int co, int bpw,
+                                                           float* __restrict__ part) {
   using B = WBox<BW>;
-  __shared__ __attribute__((aligned(16))) uint16_t sA[16 * B::ROW_A];
-  __shared__ __attribute__((aligned(16))) uint16_t sB[3 * 16 * B::ROW_B];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  __shared__ __attribute__((aligned(16))) unsigned char s_dy[2][NCO * B::DY];
+  __shared__ __attribute__((aligned(16))) unsigned char s_x[2][B::XC * 1024];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row = lane & 15, q = lane >> 4;
-  const int nct = co / 16, nit = ci / 16;
-  const int tile = blockIdx.x % (nct * nit);
-  const int chunk = blockIdx.x / (nct * nit);
-  const int co0 = (tile / nit) * 16, ci0 = (tile % nit) * 16;
+  const int nct = co / (16 * NCO), nit = ci / 16;
+  const int tile = blockIdx.x % (nct * nit), chunk = blockIdx.x / (nct * nit);
+  const int co0 = (tile / nit) * 16 * NCO, ci0 = (tile % nit) * 16;
   const int nbd = g.D / B::BD, nbh = g.H / B::BH, nbw = g.W / BW;
   const int nboxes = g.N * nbd * nbh * nbw;
-  f32x4_t acc[7];
+  const bool upper = ci0 < src.cu;   // the tile's channels come from the coarse tensor
+  const int cx = ci - src.cu;
+  // The lane's pieces, the same in every box: dy positions as offsets in
+  // elements, halo positions as coordinates and offsets.
+  int dy_off[2 * NCO], x_off[(B::XC + 3) / 4];
+  HaloPos x_pos[(B::XC + 3) / 4];
+  const int c8 = (lane & 1) * 8;
 #pragma unroll
-  for (int k = 0; k < 7; ++k) acc[k] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int b_end = min(nboxes, (chunk + 1) * bpw);
-  for (int b = chunk * bpw; b < b_end; ++b) {
+  for (int r = 0; r < 2 * NCO; ++r) {
+    const int piece = r * 4 + wv, pos = quad_swap((piece % 8) * 32 + (lane >> 1));
+    dy_off[r] = ((pos / (BW * B::BH) * g.H + pos / BW % B::BH) * g.W + pos % BW) * co + co0 +
+                (piece / 8) * 16 + c8;
+  }
+#pragma unroll
+  for (int r = 0; r < (B::XC + 3) / 4; ++r) {
+    x_pos[r] = halo_pos<B::HH, B::HW, (B::XC + 3) / 4 * 128>((r * 4 + wv) * 32 + (lane >> 1));
+    if (BW == 16) x_pos[r].w = quad_swap(x_pos[r].w);
+    x_off[r] = halo_offset(g, x_pos[r]) * cx + ci0 - src.cu + c8;
+  }
+  auto stage = [&](int b, int buf) {
     const int bw0 = (b % nbw) * BW, bh0 = ((b / nbw) % nbh) * B::BH;
     const int bd0 = ((b / (nbw * nbh)) % nbd) * B::BD, n = b / (nbw * nbh * nbd);
-    __syncthreads();  // the previous box's reads are done
-    {
-      // dy: thread = (octet o of 8 positions, co pair j)
-      const int o = tid >> 3, j = tid & 7;
-      const int od = o / (B::BH * BW / 8), oh = (o / (BW / 8)) % B::BH, ow = (o % (BW / 8)) * 8;
-      const int64_t p = (((int64_t)n * g.D + bd0 + od) * g.H + bh0 + oh) * g.W + bw0 + ow;
-      uint32_t v[8];
+    const int dz = bd0 - 1, hz = bh0 - 1, wz = bw0 - 1;
+    const uint16_t* dy0 = dy + ((((int64_t)n * g.D + bd0) * g.H + bh0) * g.W + bw0) * co;
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        v[i] = *reinterpret_cast<const uint32_t*>(dy + (p + i) * co + co0 + 2 * j);
-      u32x4_t lo, hi;
+    for (int r = 0; r < 2 * NCO; ++r) load_to_lds(dy0 + dy_off[r], &s_dy[buf][(r * 4 + wv) * 1024]);
+    const uint16_t* x0 = src.x + ((((int64_t)n * g.D + dz) * g.H + hz) * g.W + wz) * cx;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        lo[i] = (v[2 * i] & 0xFFFFu) | (v[2 * i + 1] << 16);
-        hi[i] = (v[2 * i] >> 16) | (v[2 * i + 1] & 0xFFFF0000u);
-      }
-      *reinterpret_cast<u32x4_t*>(&sA[(2 * j) * B::ROW_A + o * 8]) = lo;
-      *reinterpret_cast<u32x4_t*>(&sA[(2 * j + 1) * B::ROW_A + o * 8]) = hi;
-    }
-    // x halo: task = (halo row (hd, hh), w octet, ci pair)
-    constexpr int ntask = B::HD * B::HH * (BW / 8) * 8;
-    for (int task = tid; task < ntask; task += 256) {
-      const int j = task & 7, rest = task >> 3;
-      const int wo = rest % (BW / 8), r2 = rest / (BW / 8);
-      const int hh = r2 % B::HH, hd = r2 / B::HH;
-      const int d = bd0 + hd - 1, h = bh0 + hh - 1;
-      const bool rowin = (unsigned)d < (unsigned)g.D && (unsigned)h < (unsigned)g.H;
-      const int64_t rbase = (((int64_t)n * g.D + d) * g.H + h) * g.W;
-      uint32_t v[10];
-#pragma unroll
-      for (int i = 0; i < 10; ++i) {
-        const int w = bw0 + wo * 8 + i - 1;
-        v[i] = (rowin && (unsigned)w < (unsigned)g.W)
-                   ? *reinterpret_cast<const uint32_t*>(x + (rbase + w) * ci + ci0 + 2 * j)
-                   : 0u;
-      }
-#pragma unroll
-      for (int sh = 0; sh < 3; ++sh) {
-        u32x4_t lo, hi;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t a = v[sh + 2 * i], c = v[sh + 2 * i + 1];
-          lo[i] = (a & 0xFFFFu) | (c << 16);
-          hi[i] = (a >> 16) | (c & 0xFFFF0000u);
-        }
-        const int base = ((hd * B::HH + hh) * BW) + wo * 8;
-        *reinterpret_cast<u32x4_t*>(&sB[(sh * 16 + 2 * j) * B::ROW_B + base]) = lo;
-        *reinterpret_cast<u32x4_t*>(&sB[(sh * 16 + 2 * j + 1) * B::ROW_B + base]) = hi;
+    for (int r = 0; r < (B::XC + 3) / 4; ++r) {
+      const int piece = r * 4 + wv;
+      if (piece < B::XC) {
+        const HaloPos& o = x_pos[r];
+        const uint16_t* p = x0 + x_off[r];
+        if (upper) p = src.xu + halo_parent(g, o, n, dz, hz, wz) * src.cu + ci0 + c8;
+        load_to_lds(halo_inside(g, o, dz, hz, wz) ? p : zero_piece, &s_x[buf][piece * 1024]);
       }
     }
-    __syncthreads();
-#pragma unroll 2
+  };
+  f32x4_t acc[7][NCO];
+#pragma unroll
+  for (int k = 0; k < 7; ++k)
+#pragma unroll
+    for (int j = 0; j < NCO; ++j) acc[k][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // byte offsets of the lane's octet of K step 0 (a step is two rows of 16 or
+  // four of 8 positions: the others are at constant distances)
+  const int oh = BW == 16 ? q >> 1 : q, ow = BW == 16 ? (q & 1) * 8 : 0;
+  const int r4 = row >> 2, piece = (row & 3) * 8;
+  const int dy_pos = oh * BW + ow + r4;
+  const int dy_lo = quad_swap(dy_pos) * 32 + piece, dy_hi = quad_swap(dy_pos + 4) * 32 + piece;
+  int x_lo[7], x_hi[7];
+#pragma unroll
+  for (int k = 0; k < 7; ++k) {
+    // (there is no tap 27: wave 3 computes tap 26 again and drops it, cheaper
+    // than a branch that splits every K step for the scheduler)
+    const int t = min(wv + 4 * k, 26), x = t % 3 + ow + r4;
+    const int at = (t / 9 * B::HH + t / 3 % 3 + oh) * B::HW;
+    x_lo[k] = (at + (BW == 16 ? quad_swap(x) : x)) * 32 + piece;
+    x_hi[k] = (at + (BW == 16 ? quad_swap(x + 4) : x + 4)) * 32 + piece;
+  }
+  const int b_begin = chunk * bpw, b_end = min(nboxes, b_begin + bpw);
+  stage(b_begin, 0);
+  for (int b = b_begin; b < b_end; ++b) {
+    const int buf = (b - b_begin) & 1;
+    wait_for_loads();
+    __syncthreads();  // this box is there, the other buffer's reads are done
+    if (b + 1 < b_end) stage(b + 1, buf ^ 1);
+    const unsigned char* pdy = s_dy[buf];
+    const unsigned char* px = s_x[buf];
+#pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      const int o = 4 * ks + q;
-      const int od = o / (B::BH * BW / 8), oh = (o / (BW / 8)) % B::BH, ow = (o % (BW / 8)) * 8;
-      const bf16x8_t a = __builtin_bit_cast(
-          bf16x8_t, *reinterpret_cast<const u32x4_t*>(&sA[row * B::ROW_A + o * 8]));
+      constexpr int kRows = 32 / BW;   // rows of w per K step
+      const int xo = ((ks / 2) * B::HH + (ks % 2) * kRows) * B::HW * 32;
+      bf16x8_t a[NCO];
+#pragma unroll
+      for (int j = 0; j < NCO; ++j) {
+        const unsigned char* at = pdy + j * B::DY + ks * 1024;
+        a[j] = read_transposed(at + dy_lo, at + dy_hi);
+      }
 #pragma unroll
       for (int k = 0; k < 7; ++k) {
-        const int t = wv + 4 * k;
-        if (t < 27) {
-          const int dz = t / 9, dyy = (t / 3) % 3, dx = t % 3;  // offsets + 1
-          const bf16x8_t bb = __builtin_bit_cast(
-              bf16x8_t, *reinterpret_cast<const u32x4_t*>(
-                            &sB[(dx * 16 + row) * B::ROW_B + ((od + dz) * B::HH + oh + dyy) * BW +
-                                ow]));
-          acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bb, acc[k], 0, 0, 0);
-        }
+        const bf16x8_t bb = read_transposed(px + x_lo[k] + xo, px + x_hi[k] + xo);
+#pragma unroll
+        for (int j = 0; j < NCO; ++j)
+          acc[k][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j], bb, acc[k][j], 0, 0, 0);
       }
     }
   }
@@ -702,7 +771,10 @@ __global__ __launch_bounds__(256) void k_conv_wgrad_box(Grid3 g, const uint16_t*
     if (t >= 27) continue;
     float* out = part + ((int64_t)chunk * 27 + t) * co * ci;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) out[(int64_t)(co0 + 4 * q + r) * ci + ci0 + row] = acc[k][r];
+    for (int j = 0; j < NCO; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        out[(int64_t)(co0 + j * 16 + 4 * q + r) * ci + ci0 + row] = acc[k][j][r];
   }
 }
 
@@ -1182,13 +1254,20 @@ int conv_wgrad(const ConvGeom& cg, const uint16_t* x, int ci, const uint16_t* dy
   if (bw) {
     const int64_t bpw = wgrad_boxes_per_group(cg, ci, co);
     const int64_t nchunks = (P / 256 + bpw - 1) / bpw;
-    const dim3 grid((unsigned)(nchunks * (co / 16) * (ci / 16))), block(256);
-    if (bw == 16)
-      hipLaunchKernelGGL(k_conv_wgrad_box<16>, grid, block, 0, s, g, x, ci, dy, co, (int)bpw,
-                         part);
-    else
-      hipLaunchKernelGGL(k_conv_wgrad_box<8>, grid, block, 0, s, g, x, ci, dy, co, (int)bpw,
-                         part);
+    // two output-channel tiles per workgroup where they come in pairs: each
+    // read of x then serves two products
+    const ConvSrc src{x, nullptr, 0};
+    auto go = [&](auto width, auto tiles) {
+      constexpr int BW = decltype(width)::value, NCO = decltype(tiles)::value;
+      hipLaunchKernelGGL((k_conv_wgrad_box<BW, NCO>),
+                         dim3((unsigned)(nchunks * (co / (16 * NCO)) * (ci / 16))), dim3(256), 0, s,
+                         g, src, ci, dy, co, (int)bpw, part);
+    };
+    using std::integral_constant;
+    if (bw == 16 && co % 32 == 0) go(integral_constant<int, 16>{}, integral_constant<int, 2>{});
+    else if (bw == 16) go(integral_constant<int, 16>{}, integral_constant<int, 1>{});
+    else if (co % 32 == 0) go(integral_constant<int, 8>{}, integral_constant<int, 2>{});
+    else go(integral_constant<int, 8>{}, integral_constant<int, 1>{});
     sum_chunks(part, nchunks, n, dw, s);
     return (int)hipGetLastError();
   }

@@ -77,10 +77,12 @@ struct hlbn_net {
   Buf<float> out, in32, tgt32, lterm, dout;
   Buf<uint8_t> mask8;
   // gradients (binary32) of each activation and of the concat buffers
-  Buf<float> g[14], gcat[3], gpool[3], genc[3];
+  // (of the layers that feed a convolution; the others' are formed in place)
+  Buf<float> g[14], gcat[3], gpool[3];
+  Buf<float> gtmp;  // an output gradient of a layer that hlbn::dpre does not take
   Buf<uint16_t> dpre16;
   Buf<float> dpre32, part;
-  Buf<float> wc;
+  Buf<float> wc, loss_sums;
   int64_t head_chunk = 0;
 
   ~hlbn_net() {
@@ -100,108 +102,137 @@ int refresh_weights(hlbn_net* n) {
   return 0;
 }
 
-// One 3x3x3 convolution + ReLU layer of the forward pass.
-int conv_layer(hlbn_net* n, int L, const uint16_t* x, uint16_t* y) {
+// The input of a layer: x, or [up(xu), x] of a decoder's first convolution,
+// read in place where the kernels can, else from the concatenated copy.
+struct Input {
+  const uint16_t* x;
+  const uint16_t* xu = nullptr;
+  int cu = 0;
+};
+Input decoder_input(hlbn_net* n, int L, int up_layer, int skip_layer) {
   const Conv& c = n->conv[L];
-  KERN(hlbn::conv_fwd(n->geo[c.level], x, c.ci, c.w16.p, n->params.p + c.boff, c.co, nullptr,
-                      y, c.co, 0, 1, n->part.p, n->stream));
+  if (hlbn::conv_takes_parts(n->geo[c.level], c.ci))
+    return Input{n->a[skip_layer].p, n->a[up_layer].p, n->conv[up_layer].co};
+  return Input{n->cat[c.level].p};
+}
+// Builds the concatenated copy of a decoder level that needs it.
+int concat(hlbn_net* n, int L, int up_layer, int skip_layer) {
+  const int lv = n->conv[L].level, cu = n->conv[up_layer].co, cs = n->conv[skip_layer].co;
+  if (hlbn::conv_takes_parts(n->geo[lv], cu + cs)) return 0;
+  KERN(hlbn::up(n->geo[lv + 1], cu, n->a[up_layer].p, n->cat[lv].p, cu + cs, 0, n->stream));
+  KERN(hlbn::copy_channels(n->P[lv], cs, n->a[skip_layer].p, n->cat[lv].p, cu + cs, cu,
+                           n->stream));
   return 0;
 }
 
-// Backward of layer L: dpost = gradient of its (post-ReLU) output; writes
-// its parameter gradients and, when dx != nullptr, the input gradient.
-int conv_layer_back(hlbn_net* n, int L, const uint16_t* x, const float* dpost, float* dx) {
+// One 3x3x3 convolution + ReLU layer of the forward pass.
+int conv_layer(hlbn_net* n, int L, const Input& in) {
+  const Conv& c = n->conv[L];
+  KERN(hlbn::conv_fwd(n->geo[c.level], in.x, in.xu, in.cu, c.ci, c.w16.p, n->params.p + c.boff,
+                      c.co, nullptr, n->a[L].p, c.co, 0, 1, n->part.p, n->stream));
+  return 0;
+}
+
+// The gradient of a layer's (post-ReLU) output, by where the output went
+// (hlbn::dpre's kinds): the next convolution's data gradient `a`; the head
+// (a = dout, b = W, n outputs); the decoder level above (a = its concatenated
+// gradient, n channels wide); or a skip connection (a as before, channels
+// from off) together with the pooled gradient b.
+struct OutGrad {
+  int kind;
+  hlbn::DpreSrc src;
+};
+
+// ReLU backward of layer L into dpre16, and its bias gradient.
+int relu_layer_back(hlbn_net* n, int L, const OutGrad& g) {
   const Conv& c = n->conv[L];
   const hlbn::ConvGeom& G = n->geo[c.level];
   const int64_t P = n->P[c.level];
+  if (hlbn::dpre_fused(c.co)) {
+    KERN(hlbn::dpre(G, c.co, g.kind, g.src, n->a[L].p, n->dpre16.p, n->part.p,
+                    n->grads.p + c.boff, n->stream));
+    return 0;
+  }
+  const float* dpost = g.src.a;
+  if (g.kind != hlbn::kDprePlain) {
+    dpost = n->gtmp.p;
+    if (g.kind == hlbn::kDpreHead)
+      KERN(hlbn::head_bwd_data(P, c.co, g.src.n, g.src.a, g.src.b, n->gtmp.p, n->stream));
+    else if (g.kind == hlbn::kDpreUp)
+      KERN(hlbn::up_bwd(G, c.co, g.src.a, g.src.n, 0, n->gtmp.p, n->stream));
+    else {
+      KERN(hlbn::take_channels(P, c.co, g.src.a, g.src.n, g.src.off, n->gtmp.p, 0, n->stream));
+      KERN(hlbn::pool_bwd_add(G, c.co, g.src.b, n->gtmp.p, n->stream));
+    }
+  }
   KERN(hlbn::relu_bwd(dpost, n->a[L].p, P * c.co, n->dpre16.p, n->dpre32.p, n->stream));
-  KERN(hlbn::conv_wgrad(G, x, c.ci, n->dpre16.p, c.co, n->part.p, n->grads.p + c.woff,
-                        n->stream));
   KERN(hlbn::channel_sum(n->dpre32.p, P, c.co, n->part.p, hlbn::wgrad_chunk(G),
                          n->grads.p + c.boff, n->stream));
+  return 0;
+}
+
+// Backward of layer L: writes its parameter gradients and, when dx !=
+// nullptr, the gradient of its input.
+int conv_layer_back(hlbn_net* n, int L, const Input& in, const OutGrad& g, float* dx) {
+  const Conv& c = n->conv[L];
+  const hlbn::ConvGeom& G = n->geo[c.level];
+  if (relu_layer_back(n, L, g)) return 1;
+  KERN(hlbn::conv_wgrad(G, in.x, in.xu, in.cu, c.ci, n->dpre16.p, c.co, n->part.p,
+                        n->grads.p + c.woff, n->stream));
   if (dx)
-    KERN(hlbn::conv_fwd(G, n->dpre16.p, c.co, c.wt16.p, nullptr, c.ci, dx, nullptr, c.ci, 0, 0,
-                        n->part.p, n->stream));
+    KERN(hlbn::conv_fwd(G, n->dpre16.p, nullptr, 0, c.co, c.wt16.p, nullptr, c.ci, dx, nullptr,
+                        c.ci, 0, 0, n->part.p, n->stream));
   return 0;
 }
 
 int forward_impl(hlbn_net* n) {
-  const int C1 = n->C[0], C2 = n->C[1], C3 = n->C[2], C4 = n->C[3];
-  if (conv_layer(n, E1A, n->xin.p, n->a[E1A].p) || conv_layer(n, E1B, n->a[E1A].p, n->a[E1B].p))
-    return 1;
-  KERN(hlbn::pool(n->geo[0], C1, n->a[E1B].p, n->pooled[0].p, n->stream));
-  if (conv_layer(n, E2A, n->pooled[0].p, n->a[E2A].p) ||
-      conv_layer(n, E2B, n->a[E2A].p, n->a[E2B].p))
-    return 1;
-  KERN(hlbn::pool(n->geo[1], C2, n->a[E2B].p, n->pooled[1].p, n->stream));
-  if (conv_layer(n, E3A, n->pooled[1].p, n->a[E3A].p) ||
-      conv_layer(n, E3B, n->a[E3A].p, n->a[E3B].p))
-    return 1;
-  KERN(hlbn::pool(n->geo[2], C3, n->a[E3B].p, n->pooled[2].p, n->stream));
-  if (conv_layer(n, E4A, n->pooled[2].p, n->a[E4A].p) ||
-      conv_layer(n, E4B, n->a[E4A].p, n->a[E4B].p))
-    return 1;
-  // decoder: cat[k] = [up(coarser), skip] at level k
-  KERN(hlbn::up(n->geo[3], C4, n->a[E4B].p, n->cat[2].p, C4 + C3, 0, n->stream));
-  KERN(hlbn::copy_channels(n->P[2], C3, n->a[E3B].p, n->cat[2].p, C4 + C3, C4, n->stream));
-  if (conv_layer(n, D3A, n->cat[2].p, n->a[D3A].p) ||
-      conv_layer(n, D3B, n->a[D3A].p, n->a[D3B].p))
-    return 1;
-  KERN(hlbn::up(n->geo[2], C3, n->a[D3B].p, n->cat[1].p, C3 + C2, 0, n->stream));
-  KERN(hlbn::copy_channels(n->P[1], C2, n->a[E2B].p, n->cat[1].p, C3 + C2, C3, n->stream));
-  if (conv_layer(n, D2A, n->cat[1].p, n->a[D2A].p) ||
-      conv_layer(n, D2B, n->a[D2A].p, n->a[D2B].p))
-    return 1;
-  KERN(hlbn::up(n->geo[1], C2, n->a[D2B].p, n->cat[0].p, C2 + C1, 0, n->stream));
-  KERN(hlbn::copy_channels(n->P[0], C1, n->a[E1B].p, n->cat[0].p, C2 + C1, C2, n->stream));
-  if (conv_layer(n, D1A, n->cat[0].p, n->a[D1A].p) ||
-      conv_layer(n, D1B, n->a[D1A].p, n->a[D1B].p))
-    return 1;
-  KERN(hlbn::head_fwd(n->P[0], C1, n->cout, n->a[D1B].p, n->params.p + n->head_w,
+  const int enc[4][2] = {{E1A, E1B}, {E2A, E2B}, {E3A, E3B}, {E4A, E4B}};
+  for (int k = 0; k < 4; ++k) {
+    const uint16_t* x = k ? n->pooled[k - 1].p : n->xin.p;
+    if (conv_layer(n, enc[k][0], {x}) || conv_layer(n, enc[k][1], {n->a[enc[k][0]].p})) return 1;
+    if (k < 3)
+      KERN(hlbn::pool(n->geo[k], n->C[k], n->a[enc[k][1]].p, n->pooled[k].p, n->stream));
+  }
+  // decoder: [up(coarser), skip]
+  const int dec[3][4] = {{D3A, D3B, E4B, E3B}, {D2A, D2B, D3B, E2B}, {D1A, D1B, D2B, E1B}};
+  for (const auto& d : dec)
+    if (concat(n, d[0], d[2], d[3]) ||
+        conv_layer(n, d[0], decoder_input(n, d[0], d[2], d[3])) ||
+        conv_layer(n, d[1], {n->a[d[0]].p}))
+      return 1;
+  KERN(hlbn::head_fwd(n->P[0], n->C[0], n->cout, n->a[D1B].p, n->params.p + n->head_w,
                       n->params.p + n->head_b, n->out.p, n->stream));
   return 0;
 }
 
 int backward_impl(hlbn_net* n) {
-  const int C1 = n->C[0], C2 = n->C[1], C3 = n->C[2], C4 = n->C[3];
-  hipStream_t s = n->stream;
-  KERN(hlbn::head_bwd(n->P[0], C1, n->cout, n->dout.p, n->a[D1B].p, n->params.p + n->head_w,
-                      n->g[D1B].p, n->part.p, n->head_chunk, n->grads.p + n->head_w,
-                      n->grads.p + n->head_b, s));
-  // decoder level 0
-  if (conv_layer_back(n, D1B, n->a[D1A].p, n->g[D1B].p, n->g[D1A].p) ||
-      conv_layer_back(n, D1A, n->cat[0].p, n->g[D1A].p, n->gcat[0].p))
-    return 1;
-  KERN(hlbn::up_bwd(n->geo[1], C2, n->gcat[0].p, C2 + C1, 0, n->g[D2B].p, s));
-  KERN(hlbn::take_channels(n->P[0], C1, n->gcat[0].p, C2 + C1, C2, n->genc[0].p, 0, s));
-  // decoder level 1
-  if (conv_layer_back(n, D2B, n->a[D2A].p, n->g[D2B].p, n->g[D2A].p) ||
-      conv_layer_back(n, D2A, n->cat[1].p, n->g[D2A].p, n->gcat[1].p))
-    return 1;
-  KERN(hlbn::up_bwd(n->geo[2], C3, n->gcat[1].p, C3 + C2, 0, n->g[D3B].p, s));
-  KERN(hlbn::take_channels(n->P[1], C2, n->gcat[1].p, C3 + C2, C3, n->genc[1].p, 0, s));
-  // decoder level 2
-  if (conv_layer_back(n, D3B, n->a[D3A].p, n->g[D3B].p, n->g[D3A].p) ||
-      conv_layer_back(n, D3A, n->cat[2].p, n->g[D3A].p, n->gcat[2].p))
-    return 1;
-  KERN(hlbn::up_bwd(n->geo[3], C4, n->gcat[2].p, C4 + C3, 0, n->g[E4B].p, s));
-  KERN(hlbn::take_channels(n->P[2], C3, n->gcat[2].p, C4 + C3, C4, n->genc[2].p, 0, s));
+  KERN(hlbn::head_wgrad(n->P[0], n->C[0], n->cout, n->dout.p, n->a[D1B].p, n->part.p,
+                        n->head_chunk, n->grads.p + n->head_w, n->grads.p + n->head_b,
+                        n->stream));
+  // decoder, finest level first: a level's output went to the head or, through
+  // the upsampling, into the concatenated gradient of the level above it
+  OutGrad g{hlbn::kDpreHead, {n->dout.p, n->params.p + n->head_w, n->cout, 0}};
+  const int dec[3][4] = {{D1A, D1B, D2B, E1B}, {D2A, D2B, D3B, E2B}, {D3A, D3B, E4B, E3B}};
+  for (int k = 0; k < 3; ++k) {
+    const int* d = dec[k];
+    if (conv_layer_back(n, d[1], {n->a[d[0]].p}, g, n->g[d[0]].p) ||
+        conv_layer_back(n, d[0], decoder_input(n, d[0], d[2], d[3]),
+                        {hlbn::kDprePlain, {n->g[d[0]].p, nullptr, 0, 0}}, n->gcat[k].p))
+      return 1;
+    g = {hlbn::kDpreUp, {n->gcat[k].p, nullptr, n->C[k + 1] + n->C[k], 0}};
+  }
   // bottleneck and encoder
-  if (conv_layer_back(n, E4B, n->a[E4A].p, n->g[E4B].p, n->g[E4A].p) ||
-      conv_layer_back(n, E4A, n->pooled[2].p, n->g[E4A].p, n->gpool[2].p))
-    return 1;
-  KERN(hlbn::pool_bwd_add(n->geo[2], C3, n->gpool[2].p, n->genc[2].p, s));
-  if (conv_layer_back(n, E3B, n->a[E3A].p, n->genc[2].p, n->g[E3A].p) ||
-      conv_layer_back(n, E3A, n->pooled[1].p, n->g[E3A].p, n->gpool[1].p))
-    return 1;
-  KERN(hlbn::pool_bwd_add(n->geo[1], C2, n->gpool[1].p, n->genc[1].p, s));
-  if (conv_layer_back(n, E2B, n->a[E2A].p, n->genc[1].p, n->g[E2A].p) ||
-      conv_layer_back(n, E2A, n->pooled[0].p, n->g[E2A].p, n->gpool[0].p))
-    return 1;
-  KERN(hlbn::pool_bwd_add(n->geo[0], C1, n->gpool[0].p, n->genc[0].p, s));
-  if (conv_layer_back(n, E1B, n->a[E1A].p, n->genc[0].p, n->g[E1A].p) ||
-      conv_layer_back(n, E1A, n->xin.p, n->g[E1A].p, nullptr))
-    return 1;
+  const int enc[4][2] = {{E1A, E1B}, {E2A, E2B}, {E3A, E3B}, {E4A, E4B}};
+  for (int k = 3; k >= 0; --k) {
+    if (k < 3)
+      g = {hlbn::kDpreSkip, {n->gcat[k].p, n->gpool[k].p, n->C[k + 1] + n->C[k], n->C[k + 1]}};
+    const int A = enc[k][0], B = enc[k][1];
+    if (conv_layer_back(n, B, {n->a[A].p}, g, n->g[A].p) ||
+        conv_layer_back(n, A, {k ? n->pooled[k - 1].p : n->xin.p},
+                        {hlbn::kDprePlain, {n->g[A].p, nullptr, 0, 0}},
+                        k ? n->gpool[k - 1].p : nullptr))
+      return 1;
+  }
   return 0;
 }
 
@@ -275,7 +306,7 @@ int hlbn_create(int32_t side, int32_t batch, int32_t in_channels, int32_t out_ch
   HIPN(hipMemset(n->grads.p, 0, sizeof(float) * n->nparam));
   HIPN(hipMemset(n->adam_m.p, 0, sizeof(float) * n->nparam));
   HIPN(hipMemset(n->adam_v.p, 0, sizeof(float) * n->nparam));
-  int64_t max_part = 0, max_pc = 0;
+  int64_t max_part = 0, max_pc = 0, unfused_pc = 0;
   for (auto& c : n->conv) {
     HIPN(c.w16.alloc((size_t)27 * c.co * c.ci));
     HIPN(c.wt16.alloc((size_t)27 * c.co * c.ci));
@@ -287,6 +318,7 @@ int hlbn_create(int32_t side, int32_t batch, int32_t in_channels, int32_t out_ch
     max_part = std::max(max_part, hlbn::conv_fwd_ws(n->geo[c.level], c.co, c.ci));
     max_part = std::max(max_part, (P + ch - 1) / ch * c.co);
     max_pc = std::max(max_pc, P * c.co);
+    if (!hlbn::dpre_fused(c.co)) unfused_pc = std::max(unfused_pc, P * c.co);
   }
   // positions per partial sum of the head's weight gradient and of the
   // per-channel sums at full resolution: 16384 chunks of 64 at a 64^3 x 4
@@ -296,20 +328,25 @@ int hlbn_create(int32_t side, int32_t batch, int32_t in_channels, int32_t out_ch
                                     (int64_t)out_channels * C1);
   HIPN(n->part.alloc(max_part));
   HIPN(n->dpre16.alloc(max_pc));
-  HIPN(n->dpre32.alloc(max_pc));
+  if (unfused_pc) {
+    HIPN(n->dpre32.alloc(unfused_pc));
+    HIPN(n->gtmp.alloc(unfused_pc));
+  }
+  HIPN(n->loss_sums.alloc(out_channels));
   const int64_t P0 = n->P[0];
   HIPN(n->xin.alloc(P0 * n->cinp));
   HIPN(n->in32.alloc(P0 * in_channels));
   for (int L = 0; L < 14; ++L) {
     HIPN(n->a[L].alloc(n->P[n->conv[L].level] * n->conv[L].co));
-    HIPN(n->g[L].alloc(n->P[n->conv[L].level] * n->conv[L].co));
+    if (L == E1A || L == E2A || L == E3A || L == E4A || L == D3A || L == D2A || L == D1A)
+      HIPN(n->g[L].alloc(n->P[n->conv[L].level] * n->conv[L].co));
   }
   for (int k = 0; k < 3; ++k) {
     HIPN(n->pooled[k].alloc(n->P[k + 1] * chans[k]));
     HIPN(n->gpool[k].alloc(n->P[k + 1] * chans[k]));
-    HIPN(n->cat[k].alloc(n->P[k] * (chans[k + 1] + chans[k])));
+    if (!hlbn::conv_takes_parts(n->geo[k], chans[k + 1] + chans[k]))
+      HIPN(n->cat[k].alloc(n->P[k] * (chans[k + 1] + chans[k])));
     HIPN(n->gcat[k].alloc(n->P[k] * (chans[k + 1] + chans[k])));
-    HIPN(n->genc[k].alloc(n->P[k] * chans[k]));
   }
   HIPN(n->out.alloc(P0 * out_channels));
   HIPN(n->dout.alloc(P0 * out_channels));
@@ -335,8 +372,9 @@ int64_t hlbn_device_bytes(const hlbn_net* n) {
   for (int L = 0; L < 14; ++L) b += 2 * (int64_t)n->a[L].n + 4 * (int64_t)n->g[L].n;
   for (int k = 0; k < 3; ++k)
     b += 2 * (int64_t)(n->pooled[k].n + n->cat[k].n) +
-         4 * (int64_t)(n->gpool[k].n + n->gcat[k].n + n->genc[k].n);
-  b += 4 * (int64_t)(n->out.n + n->dout.n + n->lterm.n + n->tgt32.n + n->part.n + n->dpre32.n);
+         4 * (int64_t)(n->gpool[k].n + n->gcat[k].n);
+  b += 4 * (int64_t)(n->out.n + n->dout.n + n->lterm.n + n->tgt32.n + n->part.n + n->dpre32.n +
+            n->gtmp.n);
   b += 2 * (int64_t)n->dpre16.n + (int64_t)n->mask8.n;
   return b;
 }
@@ -376,7 +414,7 @@ int hlbn_forward(hlbn_net* n, const float* input, float* output, int32_t device)
     in = n->in32.p;
   }
   HIPN(hipEventRecord(n->ev[0], n->stream));
-  KERN(hlbn::pack_input(P0, n->cin, n->cinp, in, n->xin.p, n->stream));
+  KERN(hlbn::pack_input(P0, n->cin, in, n->xin.p, n->stream));
   if (forward_impl(n)) return 1;
   HIPN(hipEventRecord(n->ev[1], n->stream));
   if (output) {
@@ -411,12 +449,11 @@ int hlbn_backward(hlbn_net* n, const float* target, const uint8_t* mask,
   HIPN(hipEventRecord(n->ev[2], n->stream));
   if (loss) {
     // loss terms summed per channel in a fixed order, then on the host
-    Buf<float> sums;
-    HIPN(sums.alloc(n->cout));
-    KERN(hlbn::channel_sum(n->lterm.p, P0, n->cout, n->part.p, n->head_chunk, sums.p,
+    KERN(hlbn::channel_sum(n->lterm.p, P0, n->cout, n->part.p, n->head_chunk,
+                           n->loss_sums.p,
                            n->stream));
     std::vector<float> h(n->cout);
-    HIPN(hipMemcpyAsync(h.data(), sums.p, sizeof(float) * n->cout, hipMemcpyDeviceToHost,
+    HIPN(hipMemcpyAsync(h.data(), n->loss_sums.p, sizeof(float) * n->cout, hipMemcpyDeviceToHost,
                         n->stream));
     HIPN(hipStreamSynchronize(n->stream));
     double l = 0;

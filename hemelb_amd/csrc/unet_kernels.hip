@@ -823,6 +823,73 @@ __global__ __launch_bounds__(256) void k_channel_sum_block(const float* __restri
   if ((int)threadIdx.x < C) part[k * C + threadIdx.x] = sh[threadIdx.x];
 }
 
+// dpre = dpost where post > 0, else 0 (ReLU backward), as bf16, and the
+// per-channel sums of its binary32 values (the bias gradient) in one pass;
+// dpost is formed on the way from where the layer's output went:
+//   kDprePlain  the data gradient of the next convolution
+//   kDpreHead   sum_o dout[p][o] W[o][c] of the 1x1x1 head
+//   kDpreUp     the sum of the 8 children in channels [0, C) of the concatenated
+//           gradient one level up (nearest upsampling)
+//   kDpreSkip   channels [off, off + C) of the concatenated gradient plus the
+//           parent's share of the pooled gradient
+// Bound by the bytes: one read of each operand, one bf16 write.  Before, the
+// gradient was written out in binary32 by each of these operations, masked by
+// a second kernel into a bf16 and a binary32 copy, and read again for the
+// sums.  A block per chunk adds elements in k_channel_sum_block's order, so
+// the sums are the same bits.
+template <int SRC>
+__global__ __launch_bounds__(256) void k_dpre(Grid3 g, int C, DpreSrc s,
+                                              const uint16_t* __restrict__ post, int chunk,
+                                              uint16_t* __restrict__ dpre16,
+                                              float* __restrict__ part) {
+  __shared__ float sh[256];
+  const int t = threadIdx.x, c = t % C, step = 256 / C;
+  const int P = (int)g.P(), p0 = blockIdx.x * chunk, pend = min(P, p0 + chunk);
+  float wh[16];
+  if constexpr (SRC == kDpreHead)
+#pragma unroll
+    for (int o = 0; o < 16; ++o) wh[o] = o < s.n ? s.b[o * C + c] : 0.f;
+  float sum = 0.f;
+#pragma unroll 4
+  for (int p = p0 + t / C; p < pend; p += step) {
+    const int e = p * C + c;
+    float v;
+    if constexpr (SRC == kDprePlain) {
+      v = s.a[e];
+    } else if constexpr (SRC == kDpreHead) {
+      v = 0.f;
+#pragma unroll
+      for (int o = 0; o < 16; ++o)
+        if (o < s.n) v += s.a[p * s.n + o] * wh[o];
+    } else if constexpr (SRC == kDpreUp) {
+      // row of (n, d, h) and its first child; the fine tensor is 2H x 2W
+      const int r1 = p / g.W, w = p - r1 * g.W, r2 = r1 / g.H, h = r1 - r2 * g.H;
+      const int child = ((2 * r2) * (2 * g.H) + 2 * h) * (2 * g.W) + 2 * w;
+      v = 0.f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        v += s.a[(child + ((k >> 2) * (2 * g.H) + (k >> 1 & 1)) * (2 * g.W) + (k & 1)) * s.n + c];
+    } else {
+      const int r1 = p / g.W, w = p - r1 * g.W, r2 = r1 / g.H, h = r1 - r2 * g.H;
+      const int parent = ((r2 >> 1) * (g.H / 2) + (h >> 1)) * (g.W / 2) + (w >> 1);
+      v = s.a[p * s.n + s.off + c];
+      v += s.b[parent * C + c] * 0.125f;
+    }
+    if (!(bf2f(post[e]) > 0.f)) v = 0.f;
+    dpre16[e] = f2bf(v);
+    sum += v;
+  }
+  sh[t] = sum;
+  __syncthreads();
+  for (int stride = 128; stride >= C; stride >>= 1) {
+    if (t < stride) sh[t] += sh[t + stride];
+    __syncthreads();
+  }
+  if (t < C) part[blockIdx.x * C + t] = sh[t];
+}
+
+// The same in three steps for channel counts that do not divide 256: dpost in
+// binary32 (kDpreHead, kDpreUp and kDpreSkip), the mask, and the sums.
 // Per-channel sums for any C: one thread per (chunk, channel).
 __global__ void k_channel_sum_part(const float* __restrict__ a, int64_t P, int C,
                                    int64_t chunk, float* __restrict__ part) {
@@ -946,26 +1013,49 @@ __global__ void k_take_channels(int64_t P, int C, const float* __restrict__ dy, 
   dx[i] = add ? dx[i] + v : v;
 }
 
-// Input packing: float [P][cin] -> bf16 [P][cpad] with zero padding.
-__global__ void k_pack_input(int64_t P, int cin, int cpad, const float* __restrict__ in,
+// Input packing: float [P][cin] -> bf16 [P][16] with zero padding, a position
+// per thread (an element per thread with its division took 40 us at
+// 64^3 x 4, this 12).
+__global__ void k_pack_input(int64_t P, int cin, const float* __restrict__ in,
                              uint16_t* __restrict__ x) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= P * cpad) return;
-  const int c = (int)(i % cpad);
-  x[i] = c < cin ? f2bf(in[(i / cpad) * cin + c]) : (uint16_t)0;
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= P) return;
+  uint32_t v[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const uint32_t lo = 2 * k < cin ? f2bf(in[p * cin + 2 * k]) : 0u;
+    const uint32_t hi = 2 * k + 1 < cin ? f2bf(in[p * cin + 2 * k + 1]) : 0u;
+    v[k] = lo | (hi << 16);
+  }
+  u32x4_t* out = reinterpret_cast<u32x4_t*>(x + p * 16);
+  out[0] = u32x4_t{v[0], v[1], v[2], v[3]};
+  out[1] = u32x4_t{v[4], v[5], v[6], v[7]};
 }
 
-// 1x1x1 head: out[p][o] = sum_k h[p][k] W[o][k] + b[o]   (binary32)
+// 1x1x1 head: out[p][o] = sum_k h[p][k] W[o][k] + b[o]   (binary32), a
+// position per thread: h is read once, 16 bytes at a time, instead of once
+// per output in 2-byte loads (42 -> 27 us at 64^3 x 4).
 __global__ void k_head_fwd(int64_t P, int K, int O, const uint16_t* __restrict__ h,
                            const float* __restrict__ W, const float* __restrict__ b,
                            float* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= P * O) return;
-  const int o = (int)(i % O);
-  const int64_t p = i / O;
-  float s = b[o];
-  for (int k = 0; k < K; ++k) s += bf2f(h[p * K + k]) * W[o * K + k];
-  out[i] = s;
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= P) return;
+  float s[16];
+#pragma unroll
+  for (int o = 0; o < 16; ++o) s[o] = o < O ? b[o] : 0.f;
+  for (int k0 = 0; k0 < K; k0 += 8) {
+    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(h + p * K + k0);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float x = __uint_as_float(k & 1 ? v[k >> 1] & 0xFFFF0000u : v[k >> 1] << 16);
+#pragma unroll
+      for (int o = 0; o < 16; ++o)
+        if (o < O) s[o] += x * W[o * K + k0 + k];
+    }
+  }
+#pragma unroll
+  for (int o = 0; o < 16; ++o)
+    if (o < O) out[p * O + o] = s[o];
 }
 
 // dh[p][k] = sum_o dout[p][o] W[o][k]
@@ -992,6 +1082,7 @@ __global__ void k_head_wgrad_part(int64_t P, int K, int O, const float* __restri
   const int o = ok / K, k = ok % K;
   const int64_t end = min(P, (c + 1) * chunk);
   float s = 0.f;
+#pragma unroll 8
   for (int64_t p = c * chunk; p < end; ++p) s += dout[p * O + o] * bf2f(h[p * K + k]);
   part[i] = s;
 }
@@ -1166,22 +1257,43 @@ int64_t conv_fwd_ws(const ConvGeom& cg, int ci, int co) {
   return f.nsplit > 1 ? (int64_t)f.nsplit * cg.N * cg.D * cg.H * cg.W * co : 0;
 }
 
-int conv_fwd(const ConvGeom& cg, const uint16_t* x, int ci, const uint16_t* w,
+namespace {
+// Box width of the LDS-staged weight gradient for this level (0: the level
+// does not tile into 4 x BH x BW boxes and takes the direct kernel).
+int wgrad_box_width(const ConvGeom& cg) {
+  if (cg.D % 4) return 0;
+  if (cg.W % 16 == 0 && cg.H % 4 == 0) return 16;
+  if (cg.W % 8 == 0 && cg.H % 8 == 0) return 8;
+  return 0;
+}
+// Boxes per workgroup: at least about 1024 workgroups over the tile pairs.
+int64_t wgrad_boxes_per_group(const ConvGeom& cg, int ci, int co) {
+  const int64_t nboxes = (int64_t)cg.N * cg.D * cg.H * cg.W / 256;
+  const int64_t tiles = (int64_t)(co / 16) * (ci / 16);
+  return std::max<int64_t>(1, nboxes * tiles / 1024);
+}
+}  // namespace
+
+bool conv_takes_parts(const ConvGeom& cg, int ci) {
+  return box_channels(ci) && wgrad_box_width(cg) != 0;
+}
+
+int conv_fwd(const ConvGeom& cg, const uint16_t* x, const uint16_t* xu, int cu, int ci,
+             const uint16_t* w,
              const float* bias, int co, float* y32, uint16_t* y16, int yc, int yoff, int relu,
              float* ws, void* stream) {
   const Grid3 g{cg.N, cg.D, cg.H, cg.W};
   const int64_t P = (int64_t)cg.N * cg.D * cg.H * cg.W;
   const FwdPlan f = fwd_plan(cg, ci, co);
   if (box_channels(ci)) {
-    const BoxCall c{g,    ConvSrc{x, nullptr, 0}, w,    bias,
-                    co,   y32,                    y16,  yc,
-                    yoff, relu,                   f.nsplit > 1 ? f.hpw / 2 : 0,
-                    (hipStream_t)stream};
+    const BoxCall c{g, ConvSrc{x, xu, xu ? cu : 0}, w, bias, co, y32, y16, yc, yoff, relu,
+                    f.nsplit > 1 ? f.hpw / 2 : 0, (hipStream_t)stream};
     const bool wide = (cg.W + 15) / 16 * 16 == (cg.W + 7) / 8 * 8;
     if (!(wide ? box_dispatch<16>(c, ci) : box_dispatch<8>(c, ci)))
       return (int)hipErrorInvalidValue;
     return (int)hipGetLastError();
   }
+  if (xu) return (int)hipErrorInvalidValue;
   if (f.nsplit > 1 && !ws) return (int)hipErrorInvalidValue;
   float* slices = f.nsplit > 1 ? ws : nullptr;
   const dim3 grid((unsigned)((f.waves + 3) / 4), (unsigned)f.nsplit), block(256);
@@ -1214,23 +1326,6 @@ int64_t wgrad_chunk(const ConvGeom& cg) {
   return chunk < 256 ? 256 : chunk;
 }
 
-namespace {
-// Box width of the LDS-staged weight gradient for this level (0: the level
-// does not tile into 4 x BH x BW boxes and takes the direct kernel).
-int wgrad_box_width(const ConvGeom& cg) {
-  if (cg.D % 4) return 0;
-  if (cg.W % 16 == 0 && cg.H % 4 == 0) return 16;
-  if (cg.W % 8 == 0 && cg.H % 8 == 0) return 8;
-  return 0;
-}
-// Boxes per workgroup: at least about 1024 workgroups over the tile pairs.
-int64_t wgrad_boxes_per_group(const ConvGeom& cg, int ci, int co) {
-  const int64_t nboxes = (int64_t)cg.N * cg.D * cg.H * cg.W / 256;
-  const int64_t tiles = (int64_t)(co / 16) * (ci / 16);
-  return std::max<int64_t>(1, nboxes * tiles / 1024);
-}
-}  // namespace
-
 int64_t wgrad_parts(const ConvGeom& cg, int ci, int co) {
   const int64_t P = (int64_t)cg.N * cg.D * cg.H * cg.W;
   int64_t nchunks;
@@ -1244,7 +1339,8 @@ int64_t wgrad_parts(const ConvGeom& cg, int ci, int co) {
   return nchunks * 27 * co * ci;
 }
 
-int conv_wgrad(const ConvGeom& cg, const uint16_t* x, int ci, const uint16_t* dy, int co,
+int conv_wgrad(const ConvGeom& cg, const uint16_t* x, const uint16_t* xu, int cu, int ci,
+               const uint16_t* dy, int co,
                float* part, float* dw, void* stream) {
   const Grid3 g{cg.N, cg.D, cg.H, cg.W};
   const int64_t P = g.P();
@@ -1256,7 +1352,7 @@ int conv_wgrad(const ConvGeom& cg, const uint16_t* x, int ci, const uint16_t* dy
     const int64_t nchunks = (P / 256 + bpw - 1) / bpw;
     // two output-channel tiles per workgroup where they come in pairs: each
     // read of x then serves two products
-    const ConvSrc src{x, nullptr, 0};
+    const ConvSrc src{x, xu, xu ? cu : 0};
     auto go = [&](auto width, auto tiles) {
       constexpr int BW = decltype(width)::value, NCO = decltype(tiles)::value;
       hipLaunchKernelGGL((k_conv_wgrad_box<BW, NCO>),
@@ -1271,6 +1367,7 @@ int conv_wgrad(const ConvGeom& cg, const uint16_t* x, int ci, const uint16_t* dy
     sum_chunks(part, nchunks, n, dw, s);
     return (int)hipGetLastError();
   }
+  if (xu) return (int)hipErrorInvalidValue;
   const int64_t chunk = wgrad_chunk(cg);
   const int64_t nchunks = (P + chunk - 1) / chunk;
   constexpr int TG = 9;
@@ -1298,6 +1395,31 @@ int channel_sum(const float* a, int64_t P, int C, float* part, int64_t chunk, fl
 int flip_transpose(const float* w, int co, int ci, uint16_t* w16, uint16_t* wt16, void* stream) {
   hipLaunchKernelGGL(k_flip_transpose, blocks_for((int64_t)27 * co * ci), dim3(256), 0,
                      (hipStream_t)stream, w, co, ci, w16, wt16);
+  return (int)hipGetLastError();
+}
+
+bool dpre_fused(int C) { return C <= 256 && 256 % C == 0; }
+
+namespace {
+template <int SRC>
+void dpre_launch(const ConvGeom& cg, int C, const DpreSrc& src, const uint16_t* post,
+                 int64_t chunk, uint16_t* dpre16, float* part, hipStream_t s) {
+  const Grid3 g{cg.N, cg.D, cg.H, cg.W};
+  hipLaunchKernelGGL(k_dpre<SRC>, dim3((unsigned)((g.P() + chunk - 1) / chunk)), dim3(256), 0, s,
+                     g, C, src, post, (int)chunk, dpre16, part);
+}
+}  // namespace
+
+int dpre(const ConvGeom& cg, int C, int kind, const DpreSrc& src, const uint16_t* post,
+         uint16_t* dpre16, float* part, float* db, void* stream) {
+  hipStream_t s = (hipStream_t)stream;
+  const int64_t chunk = wgrad_chunk(cg), P = (int64_t)cg.N * cg.D * cg.H * cg.W;
+  if (!dpre_fused(C)) return (int)hipErrorInvalidValue;
+  if (kind == kDprePlain) dpre_launch<kDprePlain>(cg, C, src, post, chunk, dpre16, part, s);
+  else if (kind == kDpreHead) dpre_launch<kDpreHead>(cg, C, src, post, chunk, dpre16, part, s);
+  else if (kind == kDpreUp) dpre_launch<kDpreUp>(cg, C, src, post, chunk, dpre16, part, s);
+  else dpre_launch<kDpreSkip>(cg, C, src, post, chunk, dpre16, part, s);
+  sum_chunks(part, (P + chunk - 1) / chunk, (int64_t)C, db, s);
   return (int)hipGetLastError();
 }
 
@@ -1352,23 +1474,29 @@ int take_channels(int64_t P, int C, const float* dy, int dyc, int dyoff, float* 
   return (int)hipGetLastError();
 }
 
-int pack_input(int64_t P, int cin, int cpad, const float* in, uint16_t* x, void* stream) {
-  hipLaunchKernelGGL(k_pack_input, blocks_for(P * cpad), dim3(256), 0, (hipStream_t)stream, P,
-                     cin, cpad, in, x);
+int pack_input(int64_t P, int cin, const float* in, uint16_t* x, void* stream) {
+  hipLaunchKernelGGL(k_pack_input, blocks_for(P), dim3(256), 0, (hipStream_t)stream, P, cin, in,
+                     x);
   return (int)hipGetLastError();
 }
 
 int head_fwd(int64_t P, int K, int O, const uint16_t* h, const float* W, const float* b,
              float* out, void* stream) {
-  hipLaunchKernelGGL(k_head_fwd, blocks_for(P * O), dim3(256), 0, (hipStream_t)stream, P, K, O,
+  hipLaunchKernelGGL(k_head_fwd, blocks_for(P), dim3(256), 0, (hipStream_t)stream, P, K, O,
                      h, W, b, out);
   return (int)hipGetLastError();
 }
 
-int head_bwd(int64_t P, int K, int O, const float* dout, const uint16_t* h, const float* W,
-             float* dh, float* part, int64_t chunk, float* dW, float* db, void* stream) {
+int head_bwd_data(int64_t P, int K, int O, const float* dout, const float* W, float* dh,
+                  void* stream) {
+  hipLaunchKernelGGL(k_head_bwd_data, blocks_for(P * K), dim3(256), 0, (hipStream_t)stream, P, K,
+                     O, dout, W, dh);
+  return (int)hipGetLastError();
+}
+
+int head_wgrad(int64_t P, int K, int O, const float* dout, const uint16_t* h, float* part,
+               int64_t chunk, float* dW, float* db, void* stream) {
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_head_bwd_data, blocks_for(P * K), dim3(256), 0, s, P, K, O, dout, W, dh);
   const int64_t nchunks = (P + chunk - 1) / chunk;
   hipLaunchKernelGGL(k_head_wgrad_part, blocks_for(nchunks * O * K), dim3(256), 0, s, P, K, O,
                      dout, h, chunk, part);

@@ -97,8 +97,12 @@ namespace {
 enum { E1A, E1B, E2A, E2B, E3A, E3B, E4A, E4B, D3A, D3B, D2A, D2B, D1A, D1B };
 
 int refresh_weights(hlbn_net* n) {
-  for (auto& c : n->conv)
-    KERN(hlbn::flip_transpose(n->params.p + c.woff, c.co, c.ci, c.w16.p, c.wt16.p, n->stream));
+  hlbn::WeightLayers layers;
+  for (int L = 0; L < hlbn::WeightLayers::kCount; ++L) {
+    const Conv& c = n->conv[L];
+    layers.layer[L] = {c.woff, c.co, c.ci, c.w16.p, c.wt16.p};
+  }
+  KERN(hlbn::refresh_weights(layers, n->params.p, n->stream));
   return 0;
 }
 

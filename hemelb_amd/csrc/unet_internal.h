@@ -36,10 +36,17 @@ int64_t wgrad_parts(const ConvGeom& g, int ci, int co);
 // out[c] = sum_p a[p][c] (chunked, fixed order); part holds ceil(P/chunk)*C.
 int channel_sum(const float* a, int64_t P, int C, float* part, int64_t chunk, float* out,
                 void* stream);
-// bfloat16 copies of w [27][co][ci] and of its flipped transpose
-// wt[26 - t][ci][co] (the weights of the backward-data convolution).
-int flip_transpose(const float* w, int co, int ci, uint16_t* w16, uint16_t* wt16,
-                   void* stream);
+// bfloat16 copies of every layer's weights w [27][co][ci] and of their flipped
+// transposes wt[26 - t][ci][co] (the weights of the backward-data convolution).
+struct WeightLayers {
+  static constexpr int kCount = 14;
+  struct Layer {
+    int64_t woff;   // first weight in the parameter vector
+    int co, ci;
+    uint16_t *w16, *wt16;
+  } layer[kCount];
+};
+int refresh_weights(const WeightLayers& layers, const float* params, void* stream);
 // ReLU backward with the bias gradient: dpre16 = bf16 of dpost where post > 0,
 // db[c] = sum_p of its binary32 values (part: ceil(P / wgrad_chunk) * C), for
 // C dividing 256 (dpre_fused).  dpost by kind:

@@ -792,6 +792,7 @@ __global__ __launch_bounds__(256) void k_sum_chunks(const float* __restrict__ pa
   const int64_t i = (int64_t)blockIdx.x * kOut + j;
   float s = 0.f;
   if (i < n)
+#pragma unroll 8
     for (int64_t k = q; k < nchunks; k += kPhases) s += part[k * n + i];
   sh[threadIdx.x] = s;
   __syncthreads();
@@ -837,7 +838,8 @@ __global__ __launch_bounds__(256) void k_channel_sum_block(const float* __restri
 // a second kernel into a bf16 and a binary32 copy, and read again for the
 // sums.  A block per chunk adds elements in k_channel_sum_block's order, so
 // the sums are the same bits.
-template <int SRC>
+// (NO: the head's outputs, or 16 for any number of them.)
+template <int SRC, int NO>
 __global__ __launch_bounds__(256) void k_dpre(Grid3 g, int C, DpreSrc s,
                                               const uint16_t* __restrict__ post, int chunk,
                                               uint16_t* __restrict__ dpre16,
@@ -845,10 +847,10 @@ __global__ __launch_bounds__(256) void k_dpre(Grid3 g, int C, DpreSrc s,
   __shared__ float sh[256];
   const int t = threadIdx.x, c = t % C, step = 256 / C;
   const int P = (int)g.P(), p0 = blockIdx.x * chunk, pend = min(P, p0 + chunk);
-  float wh[16];
+  float wh[NO];
   if constexpr (SRC == kDpreHead)
 #pragma unroll
-    for (int o = 0; o < 16; ++o) wh[o] = o < s.n ? s.b[o * C + c] : 0.f;
+    for (int o = 0; o < NO; ++o) wh[o] = o < s.n ? s.b[o * C + c] : 0.f;
   float sum = 0.f;
 #pragma unroll 4
   for (int p = p0 + t / C; p < pend; p += step) {
@@ -859,8 +861,8 @@ __global__ __launch_bounds__(256) void k_dpre(Grid3 g, int C, DpreSrc s,
     } else if constexpr (SRC == kDpreHead) {
       v = 0.f;
 #pragma unroll
-      for (int o = 0; o < 16; ++o)
-        if (o < s.n) v += s.a[p * s.n + o] * wh[o];
+      for (int o = 0; o < NO; ++o)
+        if (NO == 4 || o < s.n) v += s.a[p * s.n + o] * wh[o];
     } else if constexpr (SRC == kDpreUp) {
       // row of (n, d, h) and its first child; the fine tensor is 2H x 2W
       const int r1 = p / g.W, w = p - r1 * g.W, r2 = r1 / g.H, h = r1 - r2 * g.H;
@@ -904,17 +906,19 @@ __global__ void k_channel_sum_part(const float* __restrict__ a, int64_t P, int C
   part[k * C + c] = s;
 }
 
-// Weights for backward-data: wt[26 - t][ci][co] = w[t][co][ci] (bf16).
-__global__ void k_flip_transpose(const float* __restrict__ w, int co, int ci,
-                                 uint16_t* __restrict__ w16, uint16_t* __restrict__ wt16) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = (int64_t)27 * co * ci;
-  if (i >= n) return;
-  const int t = (int)(i / ((int64_t)co * ci));
-  const int o = (int)((i / ci) % co), c = (int)(i % ci);
-  const uint16_t b = f2bf(w[i]);
-  w16[i] = b;
-  wt16[((int64_t)(26 - t) * ci + c) * co + o] = b;
+// bf16 copies of the weights for the forward pass, w16[t][co][ci], and for
+// backward-data, wt16[26 - t][ci][co], of every layer (blockIdx.y): one launch
+// instead of one per layer, most of which lasted no longer than a launch.
+__global__ __launch_bounds__(256) void k_refresh_weights(WeightLayers layers,
+                                                         const float* __restrict__ params) {
+  const WeightLayers::Layer& l = layers.layer[blockIdx.y];
+  const int n = l.co * l.ci, total = 27 * n;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+    const int t = i / n, r = i - t * n, o = r / l.ci, c = r - o * l.ci;
+    const uint16_t b = f2bf(params[l.woff + i]);
+    l.w16[i] = b;
+    l.wt16[((26 - t) * l.ci + c) * l.co + o] = b;
+  }
 }
 
 // dpre_bf16[i] = dpost[i] if post[i] > 0 else 0  (ReLU backward)
@@ -1034,28 +1038,35 @@ __global__ void k_pack_input(int64_t P, int cin, const float* __restrict__ in,
 
 // 1x1x1 head: out[p][o] = sum_k h[p][k] W[o][k] + b[o]   (binary32), a
 // position per thread: h is read once, 16 bytes at a time, instead of once
-// per output in 2-byte loads (42 -> 27 us at 64^3 x 4).
-__global__ void k_head_fwd(int64_t P, int K, int O, const uint16_t* __restrict__ h,
-                           const float* __restrict__ W, const float* __restrict__ b,
-                           float* __restrict__ out) {
+// per output in 2-byte loads.  NO: O, or 16 for any O.
+template <int NO>
+__global__ __launch_bounds__(256) void k_head_fwd(int64_t P, int K, int O,
+                                                  const uint16_t* __restrict__ h,
+                                                  const float* __restrict__ W,
+                                                  const float* __restrict__ b,
+                                                  float* __restrict__ out) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= P) return;
-  float s[16];
+  float s[NO];
 #pragma unroll
-  for (int o = 0; o < 16; ++o) s[o] = o < O ? b[o] : 0.f;
+  for (int o = 0; o < NO; ++o) s[o] = NO == 4 || o < O ? b[o] : 0.f;
   for (int k0 = 0; k0 < K; k0 += 8) {
     const u32x4_t v = *reinterpret_cast<const u32x4_t*>(h + p * K + k0);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const float x = __uint_as_float(k & 1 ? v[k >> 1] & 0xFFFF0000u : v[k >> 1] << 16);
 #pragma unroll
-      for (int o = 0; o < 16; ++o)
-        if (o < O) s[o] += x * W[o * K + k0 + k];
+      for (int o = 0; o < NO; ++o)
+        if (NO == 4 || o < O) s[o] += x * W[o * K + k0 + k];
     }
   }
+  if constexpr (NO == 4) {
+    *reinterpret_cast<f32x4_t*>(out + p * 4) = f32x4_t{s[0], s[1], s[2], s[3]};
+  } else {
 #pragma unroll
-  for (int o = 0; o < 16; ++o)
-    if (o < O) out[p * O + o] = s[o];
+    for (int o = 0; o < NO; ++o)
+      if (o < O) out[p * O + o] = s[o];
+  }
 }
 
 // dh[p][k] = sum_o dout[p][o] W[o][k]
@@ -1392,20 +1403,20 @@ int channel_sum(const float* a, int64_t P, int C, float* part, int64_t chunk, fl
   return (int)hipGetLastError();
 }
 
-int flip_transpose(const float* w, int co, int ci, uint16_t* w16, uint16_t* wt16, void* stream) {
-  hipLaunchKernelGGL(k_flip_transpose, blocks_for((int64_t)27 * co * ci), dim3(256), 0,
-                     (hipStream_t)stream, w, co, ci, w16, wt16);
+int refresh_weights(const WeightLayers& layers, const float* params, void* stream) {
+  hipLaunchKernelGGL(k_refresh_weights, dim3(128, WeightLayers::kCount), dim3(256), 0,
+                     (hipStream_t)stream, layers, params);
   return (int)hipGetLastError();
 }
 
 bool dpre_fused(int C) { return C <= 256 && 256 % C == 0; }
 
 namespace {
-template <int SRC>
+template <int SRC, int NO = 1>
 void dpre_launch(const ConvGeom& cg, int C, const DpreSrc& src, const uint16_t* post,
                  int64_t chunk, uint16_t* dpre16, float* part, hipStream_t s) {
   const Grid3 g{cg.N, cg.D, cg.H, cg.W};
-  hipLaunchKernelGGL(k_dpre<SRC>, dim3((unsigned)((g.P() + chunk - 1) / chunk)), dim3(256), 0, s,
+  hipLaunchKernelGGL((k_dpre<SRC, NO>), dim3((unsigned)((g.P() + chunk - 1) / chunk)), dim3(256), 0, s,
                      g, C, src, post, (int)chunk, dpre16, part);
 }
 }  // namespace
@@ -1416,7 +1427,10 @@ int dpre(const ConvGeom& cg, int C, int kind, const DpreSrc& src, const uint16_t
   const int64_t chunk = wgrad_chunk(cg), P = (int64_t)cg.N * cg.D * cg.H * cg.W;
   if (!dpre_fused(C)) return (int)hipErrorInvalidValue;
   if (kind == kDprePlain) dpre_launch<kDprePlain>(cg, C, src, post, chunk, dpre16, part, s);
-  else if (kind == kDpreHead) dpre_launch<kDpreHead>(cg, C, src, post, chunk, dpre16, part, s);
+  else if (kind == kDpreHead && src.n == 4)
+    dpre_launch<kDpreHead, 4>(cg, C, src, post, chunk, dpre16, part, s);
+  else if (kind == kDpreHead)
+    dpre_launch<kDpreHead, 16>(cg, C, src, post, chunk, dpre16, part, s);
   else if (kind == kDpreUp) dpre_launch<kDpreUp>(cg, C, src, post, chunk, dpre16, part, s);
   else dpre_launch<kDpreSkip>(cg, C, src, post, chunk, dpre16, part, s);
   sum_chunks(part, (P + chunk - 1) / chunk, (int64_t)C, db, s);
@@ -1482,8 +1496,12 @@ int pack_input(int64_t P, int cin, const float* in, uint16_t* x, void* stream) {
 
 int head_fwd(int64_t P, int K, int O, const uint16_t* h, const float* W, const float* b,
              float* out, void* stream) {
-  hipLaunchKernelGGL(k_head_fwd, blocks_for(P), dim3(256), 0, (hipStream_t)stream, P, K, O,
-                     h, W, b, out);
+  if (O == 4)
+    hipLaunchKernelGGL(k_head_fwd<4>, blocks_for(P), dim3(256), 0, (hipStream_t)stream, P, K, O,
+                       h, W, b, out);
+  else
+    hipLaunchKernelGGL(k_head_fwd<16>, blocks_for(P), dim3(256), 0, (hipStream_t)stream, P, K, O,
+                       h, W, b, out);
   return (int)hipGetLastError();
 }
 

@@ -57,14 +57,16 @@ __global__ __launch_bounds__(256) void k_step(DevDomain D, StepArgs A,
                                               S* __restrict__ fout) {
   step_wave<Q, KERNEL, S, Lay>(D, A, fin, fout);
 }
-// The same step for binary16 storage, held to 7 waves per SIMD (at most 72
-// VGPRs instead of the 78 it would take, 6 waves): binary16 is bound by the
-// issue and latency of its vector instructions rather than by bytes, and
-// the seventh wave measured 3 % faster on the vessel tree (binary32 1 %
-// slower, binary64 spills).
+// The same step held to WAVES waves per SIMD, without spills: binary16 to 7
+// (at most 72 VGPRs; it is bound by the issue and latency of its vector
+// instructions rather than by bytes, and the seventh wave measured 3 % faster
+// on the vessel tree), binary32 to 6 (80 VGPRs; left to itself it takes 86, 5
+// waves, and the step of a 4 M-site tree 168.5 instead of 163.2 us).
+// Binary64 takes its natural 4: held to 5 it spills.
+template <typename S> constexpr int kStepWaves = sizeof(S) == 2 ? 7 : 6;
 template <int Q, int KERNEL, typename S, class Lay>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7)))
-void k_step_w7(DevDomain D, StepArgs A, const S* __restrict__ fin, S* __restrict__ fout) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStepWaves<S>)))
+void k_step_held(DevDomain D, StepArgs A, const S* __restrict__ fin, S* __restrict__ fout) {
   step_wave<Q, KERNEL, S, Lay>(D, A, fin, fout);
 }
 
@@ -177,8 +179,8 @@ int step_launch(const DevDomain& d, const StepArgs& a, const void* fin, void* fo
     }
     const dim3 grid((unsigned)std::max<uint64_t>(groups, 1)), block(a.threads);
     if (one_pass) {
-      if constexpr (std::is_same<S, _Float16>::value)
-        hipLaunchKernelGGL((k_step_w7<Q, K, S, Lay>), grid,
+      if constexpr (kShifted<S>)
+        hipLaunchKernelGGL((k_step_held<Q, K, S, Lay>), grid,
                            block, 0, (hipStream_t)stream, d, a, (const S*)fin, (S*)fout);
       else
         hipLaunchKernelGGL((k_step<Q, K, S, Lay>), grid,

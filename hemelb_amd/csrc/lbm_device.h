@@ -587,10 +587,33 @@ struct SiteRef {
   int64_t x;      // index into every per-direction array
   uint32_t cut;   // wall|iolet link mask of the site (0: bulk site)
   uint32_t rec;   // boundary record (valid when cut != 0)
+  uint32_t wall, iolet;  // the record's words (0 for a bulk site)
+  int32_t io;
+  uint32_t qoff;
   uint32_t w;     // block layout: wave index (block * 8 + x plane)
   uint32_t lane;  // block layout: lane = y * 8 + z inside the plane
   int32_t tb[27]; // block layout: neighbour blocks of this wave's block
 };
+
+// The site's boundary record, or none: one load, so that the cut distances,
+// the iolet's values and the pulls all start from here instead of one after
+// the other.  A launch is as long as its slowest wave's chain of loads: with
+// the neighbour table loaded beside the masks and the stash formed after the
+// stores, a step of 43 k sites (D3Q19 BFL) takes 9.0 instead of 9.7 us, of the
+// 7.93 M-site tree 507, 285 and 183 instead of 513, 290 and 190 us (binary64,
+// 32, 16).
+__device__ __forceinline__ void load_record(const DevDomain& D, bool boundary, SiteRef& r) {
+  r.wall = r.iolet = r.qoff = 0;
+  r.io = -1;
+  if (boundary) {
+    const uint4 v = *reinterpret_cast<const uint4*>(D.b_rec + r.rec);
+    r.wall = v.x;
+    r.iolet = v.y;
+    r.io = (int32_t)v.z;
+    r.qoff = v.w;
+  }
+  r.cut = r.wall | (r.iolet & BoundaryRecord::kLinks);
+}
 
 __device__ __forceinline__ uint32_t logical_workgroup() {
   // XCD-aware remap: hardware dispatches workgroup b to XCD b % 8; give
@@ -632,8 +655,8 @@ struct SparseLayout {
   static __device__ __forceinline__ void at(const DevDomain& D, int64_t x, SiteRef& r) {
     r.x = x;
     const uint32_t bi = D.binfo[x];
-    r.cut = bi != 0 ? 1u : 0u;  // only "is boundary" is needed here
     r.rec = bi - 1;
+    load_record(D, bi != 0, r);
   }
   // State index of direction d of slot x, and of the value streaming into
   // slot E of the lane's site.
@@ -714,16 +737,16 @@ struct BlockLayout {
     const uint64_t fm = D.wave_fluid[r.w];
     const uint64_t bm = D.wave_bnd[r.w];
     const uint32_t rb = D.wave_rec[r.w];
-    if (!((fm >> r.lane) & 1ull)) return false;
+    // (before the exit of the lanes without a site, so that the table is on
+    // its way while the masks are)
     const int32_t* nbt = D.bnbr + (int64_t)(r.w >> 3) * 27;
     sfor<0, 27>([&](auto ii) {
       constexpr int i = decltype(ii)::value;
       r.tb[i] = nbt[i];
     });
-    // A lane's cut-link mask comes from its boundary record (the gather
-    // reads the same two words again for the wall and iolet formulas).
+    if (!((fm >> r.lane) & 1ull)) return false;
     r.rec = rb + (uint32_t)__popcll(bm & ((1ull << r.lane) - 1ull));
-    r.cut = ((bm >> r.lane) & 1ull) ? (D.b_wall[r.rec] | D.b_iolet[r.rec]) : 0u;
+    load_record(D, (bm >> r.lane) & 1ull, r);
     return true;
   }
   template <int Q>
@@ -801,7 +824,7 @@ struct CompactBlockLayout {
       r.tb[i] = nbt[i];
     });
     r.rec = rb + (uint32_t)__popcll(bm & ((1ull << r.lane) - 1ull));
-    r.cut = ((bm >> r.lane) & 1ull) ? (D.b_wall[r.rec] | D.b_iolet[r.rec]) : 0u;
+    load_record(D, (bm >> r.lane) & 1ull, r);
     return true;
   }
   // Fluid mask and compact base of x plane px of block nb (nb < 0: absent,
@@ -1102,7 +1125,7 @@ __device__ __forceinline__ void bfl_stream_links(const float (&q)[kQS16<Q>], uin
   });
 }
 
-// Iolet links of boundary record `rec`: the Nash ghost equilibrium or the
+// Iolet links of a boundary site: the Nash ghost equilibrium or the
 // Ladd correction of the bounce-back value.  What a site's links share (the
 // iolet's values, the ghost's two divisions) is formed once: with all of it
 // in each link's own branch, these waves were the last of every step, and the
@@ -1110,11 +1133,12 @@ __device__ __forceinline__ void bfl_stream_links(const float (&q)[kQS16<Q>], uin
 // with, 6.3 without; an 819 k-site tree 69.1 and 67.3 us in binary64, 32.3 and
 // 30.3 in binary16).
 template <int Q, typename S, typename T>
-__device__ __forceinline__ void iolet_links(const DevDomain& D, const StepArgs& A, uint32_t rec,
-                                            uint32_t im, T (&f)[Q]) {
-  const int io = D.b_io[rec];
-  const int k = D.io_iolet[io];
-  if (D.io_bc[io] == 0) {
+__device__ __forceinline__ void iolet_links(const DevDomain& D, const StepArgs& A,
+                                            const SiteRef& r, T (&f)[Q]) {
+  const int io = r.io;
+  const uint32_t im = r.iolet;
+  const int k = (int)(r.iolet >> BoundaryRecord::kIndexBit);
+  if (!((r.iolet >> BoundaryRecord::kBcBit) & 1u)) {
     const FeqCoef<double> ghost = nash_ghost(D, A, io, k);
     sfor<1, Q>([&](auto ei) {
       constexpr int e = decltype(ei)::value;
@@ -1197,8 +1221,7 @@ __device__ __forceinline__ void gather_early(const DevDomain& D, const StepArgs&
     constexpr int dp = inv_dir(e);
     if ((r.cut >> (dp - 1)) & 1u) f[e] = own[dp];
   });
-  const uint32_t rec = r.rec;
-  const uint32_t wm = D.b_wall[rec], im = D.b_iolet[rec];
+  const uint32_t wm = r.wall, im = r.iolet & BoundaryRecord::kLinks;
   // the plane's BFL links: formulas of links no lane has are skipped
   const uint64_t wl = D.wave_links[r.w];
   float q[kQS16<Q>];
@@ -1206,7 +1229,7 @@ __device__ __forceinline__ void gather_early(const DevDomain& D, const StepArgs&
     decode_q16<Q>(qv, q);
     bfl_stream_links<Q, S, T>(q, pair_swap(wm) & ~pair_swap(im) & ~wm, own, f, (uint32_t)wl);
   }
-  if (im) iolet_links<Q, S, T>(D, A, rec, im, f);
+  if (im) iolet_links<Q, S, T>(D, A, r, f);
   if (A.wall == 1 && wm) bfl_post_links<Q, S, T>(q, wm, f, (uint32_t)(wl >> 32));
 }
 
@@ -1231,15 +1254,14 @@ __device__ __forceinline__ void gather(const DevDomain& D, const StepArgs& A,
   });
   if constexpr (BULK) return;  // a wave without boundary sites
   if (!r.cut) return;
-  const uint32_t rec = r.rec;
-  const uint32_t wm = D.b_wall[rec], im = D.b_iolet[rec];
+  const uint32_t wm = r.wall, im = r.iolet & BoundaryRecord::kLinks;
   // cut distances of links 1..Q-1 (only the wall links' are read): 16-bit
   // fixed-point records for the shifted forms, binary32 values of the wall
   // links alone, packed, for binary64 storage
   float q[kQS16<Q>];
   if (A.wall == 1 && wm) {
     if constexpr (kShifted<S>) {
-      const uint4* q8 = reinterpret_cast<const uint4*>(D.b_q16 + (int64_t)rec * kQS16<Q>);
+      const uint4* q8 = reinterpret_cast<const uint4*>(D.b_q16 + (int64_t)r.rec * kQS16<Q>);
       uint4 qv[kQS16<Q> / 8];
       sfor<0, kQS16<Q> / 8>([&](auto ii) {
         constexpr int i = decltype(ii)::value;
@@ -1249,13 +1271,19 @@ __device__ __forceinline__ void gather(const DevDomain& D, const StepArgs& A,
     } else {
       // 4.6 wall links per wall site on the vessel tree: 18 bytes instead
       // of an 80-byte record of every link
-      const float* qp = D.b_q + D.b_qoff[rec];
+      const float* qp = D.b_q + r.qoff;
       sfor<0, Q - 1>([&](auto kk) {
         constexpr int k = decltype(kk)::value;
         q[k] = -1.0f;
         if ((wm >> k) & 1u) q[k] = qp[__popc(wm & ((1u << k) - 1u))];
       });
     }
+  }
+  // The iolet links of a site and its interpolated wall links write different
+  // slots, so the iolet ones go first, while the cut distances are on their
+  // way.
+  if (im) iolet_links<Q, S, T>(D, A, r, f);
+  if (A.wall == 1 && wm) {
     // The links that take the interpolated form need the site's own f*_e.
     // Binary64 and binary32: only those lanes load (the rest are masked
     // off; measured 0.3-0.6 % faster on the vessel tree).  Binary16 (64-bit
@@ -1276,22 +1304,20 @@ __device__ __forceinline__ void gather(const DevDomain& D, const StepArgs& A,
       }
     });
     bfl_stream_links<Q, S, T>(q, cand, opp, f);
+    bfl_post_links<Q, S, T>(q, wm, f);
   }
-  if (im) iolet_links<Q, S, T>(D, A, rec, im, f);
-  if (A.wall == 1 && wm) bfl_post_links<Q, S, T>(q, wm, f);
 }
 
 template <int Q, typename T, bool BULK = false>
 __device__ __forceinline__ void update_stash(const DevDomain& D, const SiteRef& r,
                                              const Hydro<Q, T>& h) {
   if constexpr (BULK) return;
-  if (!r.cut) return;
-  const int io = D.b_io[r.rec];
+  const int io = r.io;
   if (io < 0) return;
   const double rho = (double)h.rho;
-  if (D.io_bc[io] == 0) {
+  if (!((r.iolet >> BoundaryRecord::kBcBit) & 1u)) {
     // component = Dot(momentum, n_float) / density (NashZerothOrderPressure.h:43)
-    const int k = D.io_iolet[io];
+    const int k = (int)(r.iolet >> BoundaryRecord::kIndexBit);
     double acc = 0.0;
     acc = acc + (double)h.mx * (double)D.iolet_nf[3 * k];
     acc = acc + (double)h.my * (double)D.iolet_nf[3 * k + 1];

@@ -195,8 +195,8 @@ __global__ __launch_bounds__(256) void k_monitor(DevDomain D, StepArgs A,
     mx = rho > mx ? rho : mx;
     const double m = sqrt(((0.0 + ux * ux) + uy * uy) + uz * uz);
     um = m > um ? m : um;
-    if (r.cut && io_vals) {
-      const int io = D.b_io[r.rec];
+    if (io_vals) {
+      const int io = r.io;
       if (io >= 0) {
         io_vals[4 * (int64_t)io] = rho;
         io_vals[4 * (int64_t)io + 1] = ux;
@@ -369,7 +369,7 @@ __global__ __launch_bounds__(256) void k_export_fields(DevDomain D, StepArgs A,
   double ts = F.tau;
   if constexpr (kWaveLayout<Lay>)
     if (D.blk_tau) ts = D.blk_tau[r.w >> 3];
-  const bool wall = r.cut && D.b_wall[r.rec] != 0;
+  const bool wall = r.wall != 0;
   double n[3] = {0.0, 0.0, 0.0};
   if (wall && F.rec_normal)
     for (int a = 0; a < 3; ++a) n[a] = (double)F.rec_normal[3 * (int64_t)r.rec + a];

@@ -11,6 +11,18 @@ namespace hlb {
 constexpr int kMaxMoments = 15;
 constexpr int kMaxQ = 19;
 
+// A boundary site's record: one 16-byte load gives the kernels all that its
+// later loads depend on.
+struct alignas(16) BoundaryRecord {
+  uint32_t wall;    // wall link mask
+  uint32_t iolet;   // bits 0-17: iolet link mask; bit 18: hlb_iolet_bc; from
+                    // bit 19: global iolet index (inlets first)
+  int32_t io;       // iolet-site record or -1
+  uint32_t qoff;    // first entry in b_q (binary64 storage)
+  static constexpr uint32_t kLinks = (1u << 18) - 1;
+  static constexpr int kBcBit = 18, kIndexBit = 19;
+};
+
 // Device-side description of one solver's domain in the library's own
 // layout.  Sites are ordered by 8^3 block in Morton order, z-fastest inside a
 // block ("compact" order).  Distributions are structure-of-arrays with stride
@@ -49,19 +61,14 @@ struct DevDomain {
   // boundary mask.
   const uint32_t* binfo = nullptr;
   int64_t nb = 0;                  // boundary records
-  const uint32_t* b_wall = nullptr;   // [nb] wall link mask
-  const uint32_t* b_iolet = nullptr;  // [nb] iolet link mask
-  const int32_t* b_io = nullptr;      // [nb] iolet-site record or -1
+  const BoundaryRecord* b_rec = nullptr;  // [nb]
   const float* b_q = nullptr;         // binary64 storage: the cut distances
                                       // of each record's wall links, packed
-                                      // in direction order
-  const uint32_t* b_qoff = nullptr;   // [nb] first entry of record r in b_q
+                                      // in direction order from rec.qoff
   const uint16_t* b_q16 = nullptr;    // [nb][QS16] the same as q * 65535,
                                       // QS16 = Q-1 rounded up to a multiple of 8
                                       // (reduced-precision storage)
   int64_t ni = 0;                  // iolet-site records
-  const int32_t* io_iolet = nullptr;  // [ni] global iolet index (inlets first)
-  const int32_t* io_bc = nullptr;     // [ni] hlb_iolet_bc of the site's group
   const int32_t* io_site = nullptr;   // [ni] internal site index
   double* io_stash = nullptr;         // [ni] Nash: m.n/rho ; Ladd: rho
   const double* io_ladd = nullptr;    // [ni][Q-1][2] per-link velocity coeffs

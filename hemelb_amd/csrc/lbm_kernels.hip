@@ -22,7 +22,9 @@ __device__ __forceinline__ void step_site(const DevDomain& D, const StepArgs& A,
   StepArgs a = A;
   Lay::relax(D, r, a);
   const Hydro<Q, T> h = collide<Q, KERNEL, S>(f, a);
-  update_stash<Q, T, BULK>(D, r, h);
+  // The stash's loads and division come after the stores, which need not wait
+  // for them (binary16: before, where its registers suffice; 4 % faster).
+  if constexpr (sizeof(S) == 2) update_stash<Q, T, BULK>(D, r, h);
   sfor<0, Q>([&](auto di) {
     constexpr int d = decltype(di)::value;
     if constexpr (std::is_same<Lay, BlockLayout32>::value)
@@ -30,6 +32,7 @@ __device__ __forceinline__ void step_site(const DevDomain& D, const StepArgs& A,
     else
       store_out<S>(own_ptr<Q, Lay>(D, r, fout, d), f[d]);
   });
+  if constexpr (sizeof(S) != 2) update_stash<Q, T, BULK>(D, r, h);
 }
 
 // One timestep, one site per thread.  Block layout: one x plane per wave,
@@ -87,7 +90,7 @@ __global__ __launch_bounds__(256) void k_step_list(DevDomain D, StepArgs A,
   const uint32_t w = __builtin_amdgcn_readfirstlane(waves[i]);
   SiteRef r;
   if (!Lay::locate_wave(D, w, r)) return;
-  if constexpr (BULK) r.cut = 0;  // known: no cut links in these planes
+  if constexpr (BULK) r.cut = 0;  // known: no boundary sites in these planes
   step_site<Q, KERNEL, S, Lay, BULK>(D, A, fin, fout, r);
 }
 

@@ -267,10 +267,10 @@ struct hlb_solver {
   int n_inlets = 0;
   // device data
   DevBuf<int32_t> src;
-  DevBuf<uint32_t> binfo, b_wall, b_iolet;
-  DevBuf<int32_t> b_io, io_iolet, io_bc, io_site, iolet_kind;
+  DevBuf<uint32_t> binfo;
+  DevBuf<hlb::BoundaryRecord> b_rec;
+  DevBuf<int32_t> io_site, iolet_kind;
   DevBuf<float> b_q, iolet_nf;
-  DevBuf<uint32_t> b_qoff;
   DevBuf<uint16_t> b_q16;
   DevBuf<double> io_stash, io_ladd, iolet_n, weights;
   DevBuf<int32_t> bnbr;
@@ -346,9 +346,8 @@ struct hlb_solver {
 
   int64_t device_bytes() const {
     int64_t b = 2 * (int64_t)storage_bytes(p.storage) * Q * np;
-    b += src.bytes() + binfo.bytes() + b_wall.bytes() + b_iolet.bytes() +
-         b_io.bytes() + io_iolet.bytes() + io_bc.bytes() + io_site.bytes() +
-         iolet_kind.bytes() + b_q.bytes() + b_qoff.bytes() + b_q16.bytes() + iolet_nf.bytes() + io_stash.bytes() +
+    b += src.bytes() + binfo.bytes() + b_rec.bytes() + io_site.bytes() +
+         iolet_kind.bytes() + b_q.bytes() + b_q16.bytes() + iolet_nf.bytes() + io_stash.bytes() +
          io_ladd.bytes() + iolet_n.bytes() + weights.bytes() + d_perm.bytes() +
          bnbr.bytes() + wave_fluid.bytes() + wave_bnd.bytes() + wave_links.bytes() +
          wave_rec.bytes() +
@@ -718,10 +717,10 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
     h_src.assign((size_t)(Q - 1) * np, 0);
     h_binfo.assign(np, 0);
   }
-  std::vector<uint32_t> h_bwall, h_biolet;
-  std::vector<int32_t> h_bio, h_io_iolet, h_io_bc, h_io_site;
+  static_assert(kMaxIolets <= 1 << (32 - hlb::BoundaryRecord::kIndexBit), "iolet index bits");
+  std::vector<hlb::BoundaryRecord> h_brec;
+  std::vector<int32_t> h_io_site;
   std::vector<float> h_bq;        // binary64: the wall links' cut distances, packed
-  std::vector<uint32_t> h_bqoff;  // binary64: first entry of each record in h_bq
   std::vector<uint16_t> h_bq16;  // reduced-precision storage: q * 65535
   std::vector<double> h_ladd;
   for (int64_t o = 0; o < n; ++o) {
@@ -758,15 +757,13 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
         h_src[(size_t)(e - 1) * np + o] = own ? (int32_t)(o + (int64_t)(dp - e) * np) : (int32_t)j;
     }
     if (wm | im) {
-      const uint32_t rec = (uint32_t)h_bwall.size();
-      if (!blocks_layout) h_binfo[o] = rec + 1;
-      h_bwall.push_back(wm);
-      h_biolet.push_back(im);
+      if (!blocks_layout) h_binfo[o] = (uint32_t)h_brec.size() + 1;
+      hlb::BoundaryRecord rec{wm, im, -1, 0};
       if (s->has_normals)
         for (int a = 0; a < 3; ++a) s->rec_normals.push_back(dm->wall_normal[3 * i + a]);
       // Cut distances (the BFL links read those of wall links only):
       // * binary64 storage: the reference's float q, bit for bit, of the
-      //   wall links alone, packed in direction order from h_bqoff[rec];
+      //   wall links alone, packed in direction order from rec.qoff;
       // * reduced-precision forms: q * 65535 rounded to 16 bits for every
       //   link, in 16-byte aligned records (a wall position error below 8e-6
       //   lattice units).
@@ -779,7 +776,7 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
                                                  65535.0));
         }
       } else {
-        h_bqoff.push_back((uint32_t)h_bq.size());
+        rec.qoff = (uint32_t)h_bq.size();
         for (int d = 1; d < Q; ++d)
           if ((wm >> (d - 1)) & 1u)
             h_bq.push_back(dm->cut_distance ? dm->cut_distance[i * (Q - 1) + d - 1] : -1.0f);
@@ -787,10 +784,9 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
       if (im) {
         const int g = dm->site_type[i] == HLB_SITE_OUTLET ? 1 : 0;
         const int k = (g ? n_inlets : 0) + dm->iolet_id[i];
-        const int32_t io_rec = (int32_t)h_io_iolet.size();
-        h_bio.push_back(io_rec);
-        h_io_iolet.push_back(k);
-        h_io_bc.push_back(s->iolets[k].bc);
+        rec.io = (int32_t)h_io_site.size();
+        rec.iolet |= (uint32_t)s->iolets[k].bc << hlb::BoundaryRecord::kBcBit |
+                     (uint32_t)k << hlb::BoundaryRecord::kIndexBit;
         h_io_site.push_back((int32_t)o);
         s->io_sites_internal.push_back(o);
         s->io_sites_iolet.push_back(k);
@@ -812,9 +808,8 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
           h_ladd.push_back(c0);
           h_ladd.push_back(c1);
         }
-      } else {
-        h_bio.push_back(-1);
       }
+      h_brec.push_back(rec);
     }
   }
 
@@ -989,18 +984,13 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
   HIP_OR_FAIL(s->wave_cbase.upload(h_wc));
   HIP_OR_FAIL(s->bulk_waves.upload(h_bulkw));
   HIP_OR_FAIL(s->bnd_waves.upload(h_bndw));
-  HIP_OR_FAIL(s->b_wall.upload(h_bwall));
-  HIP_OR_FAIL(s->b_iolet.upload(h_biolet));
-  HIP_OR_FAIL(s->b_io.upload(h_bio));
+  HIP_OR_FAIL(s->b_rec.upload(h_brec));
   HIP_OR_FAIL(s->b_q.upload(h_bq));
-  HIP_OR_FAIL(s->b_qoff.upload(h_bqoff));
   HIP_OR_FAIL(s->b_q16.upload(h_bq16));
-  HIP_OR_FAIL(s->io_iolet.upload(h_io_iolet));
-  HIP_OR_FAIL(s->io_bc.upload(h_io_bc));
   HIP_OR_FAIL(s->io_site.upload(h_io_site));
   HIP_OR_FAIL(s->io_ladd.upload(h_ladd));
-  HIP_OR_FAIL(s->io_stash.alloc(h_io_iolet.size()));
-  HIP_OR_FAIL(hipMemset(s->io_stash.p, 0, sizeof(double) * (h_io_iolet.empty() ? 1 : h_io_iolet.size())));
+  HIP_OR_FAIL(s->io_stash.alloc(h_io_site.size()));
+  HIP_OR_FAIL(hipMemset(s->io_stash.p, 0, sizeof(double) * (h_io_site.empty() ? 1 : h_io_site.size())));
   std::vector<float> h_nf;
   std::vector<double> h_n;
   std::vector<int32_t> h_kind;
@@ -1051,16 +1041,11 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
   }
   D.src = s->src.p;
   D.binfo = s->binfo.p;
-  D.nb = (int64_t)h_bwall.size();
-  D.b_wall = s->b_wall.p;
-  D.b_iolet = s->b_iolet.p;
-  D.b_io = s->b_io.p;
+  D.nb = (int64_t)h_brec.size();
+  D.b_rec = s->b_rec.p;
   D.b_q = s->b_q.p;
-  D.b_qoff = s->b_qoff.p;
   D.b_q16 = s->b_q16.p;
-  D.ni = (int64_t)h_io_iolet.size();
-  D.io_iolet = s->io_iolet.p;
-  D.io_bc = s->io_bc.p;
+  D.ni = (int64_t)h_io_site.size();
   D.io_site = s->io_site.p;
   D.io_stash = s->io_stash.p;
   D.io_ladd = s->io_ladd.p;

@@ -1216,30 +1216,37 @@ bool box_channels(int ci) {
   return (ng >= 1 && ng <= 4) || ng == 6 || ng == 8 || ng == 12;
 }
 // Boxes are 16 wide where that pads the width no more than 8, and hold as
-// many positions as still leave about two workgroups per CU (512): a large
-// box re-reads less halo, a small one fills the chip.  Many input channels
-// bound the box by LDS instead.
+// many positions as still leave about two workgroups per CU: a large box
+// re-reads less halo, a small one fills the chip (32 -> 32 channels at
+// 2 x 32^3: 21 us in boxes of 64 positions and one output tile, 13 in boxes
+// of 128 and two).  Many input channels bound the box by LDS instead; there
+// half the box (12 groups) and twice (6) measured the same within 3 %.
 template <int BW>
 bool box_dispatch(const BoxCall& c, int ci) {
   constexpr int H = BW == 16 ? 1 : 2;  // rows of w per 16 positions
   const int64_t P = (int64_t)c.g.N * c.g.D * c.g.H * c.g.W;
   const int T = c.co / 16;
-  const bool large = P >= 512 * 256;
+  const bool large = P >= 512 * 256, medium = P >= 256 * 128;
   switch (ci / 16) {
     case 1:
-      if (!large) box_launch<1, 1, 1, 4, 1, 4 * H, BW>(c);
+      if (!medium) box_launch<1, 1, 1, 4, 1, 4 * H, BW>(c);
+      else if (!large && T % 2 == 0) box_launch<1, 2, 2, 4, 2, 4 * H, BW>(c);
+      else if (!large) box_launch<1, 1, 2, 4, 2, 4 * H, BW>(c);
       else if (T % 3 == 0) box_launch<1, 3, 4, 4, 4, 4 * H, BW>(c);
       else if (T % 2 == 0) box_launch<1, 2, 4, 4, 4, 4 * H, BW>(c);
       else box_launch<1, 1, 8, 4, BW == 16 ? 4 : 8, 8, BW>(c);
       return true;
     case 2:
-      if (!large) box_launch<2, 1, 1, 4, 1, 4 * H, BW>(c);
+      if (!medium) box_launch<2, 1, 1, 4, 1, 4 * H, BW>(c);
+      else if (!large && T % 2 == 0) box_launch<2, 2, 2, 4, 2, 4 * H, BW>(c);
+      else if (!large) box_launch<2, 1, 2, 4, 2, 4 * H, BW>(c);
       else if (T % 3 == 0) box_launch<2, 3, 4, 4, 4, 4 * H, BW>(c);
       else if (T % 2 == 0) box_launch<2, 2, 4, 4, 4, 4 * H, BW>(c);
       else box_launch<2, 1, 4, 4, 4, 4 * H, BW>(c);
       return true;
     case 3:
-      if (!large) box_launch<3, 1, 1, 4, 1, 4 * H, BW>(c);
+      if (!medium) box_launch<3, 1, 1, 4, 1, 4 * H, BW>(c);
+      else if (!large) box_launch<3, 1, 2, 4, 2, 4 * H, BW>(c);
       else box_launch<3, 1, 4, 4, 4, 4 * H, BW>(c);
       return true;
     case 4:

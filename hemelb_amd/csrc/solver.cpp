@@ -1250,6 +1250,9 @@ struct FieldRequest {
   int width;
   double* host;
 };
+// Up to this many values the kernel writes pinned host memory itself (256 KiB):
+// a copy after it costs a launch and a wait of its own for each array.
+constexpr int64_t kSmallExport = 32768;
 static int export_fields(hlb_solver* s, const FieldRequest* wanted, int count) {
   hlb::FieldPtrs F;
   F.perm = s->d_perm.p;
@@ -1259,9 +1262,10 @@ static int export_fields(hlb_solver* s, const FieldRequest* wanted, int count) {
   for (int k = 0; k < count; ++k)
     if (wanted[k].host) total += wanted[k].width * s->n;
   if (total == 0) return HLB_OK;
-  int r = s->ensure_exports(total);
+  const bool small = total <= kSmallExport;
+  int r = small ? s->ensure_partials((size_t)total) : s->ensure_exports(total);
   if (r) return r;
-  double* at = s->exports.p;
+  double* at = small ? s->partials : s->exports.p;
   for (int k = 0; k < count; ++k) {
     if (!wanted[k].host) continue;
     F.*wanted[k].slot = at;
@@ -1270,6 +1274,13 @@ static int export_fields(hlb_solver* s, const FieldRequest* wanted, int count) {
   if (hlb::launch_export_fields(s->dom, s->args_for_stream(), s->state[s->cur],
                                 s->post_stream ? 1 : 0, F, s->stream))
     return fail(HLB_E_DEVICE, "export kernel launch failed");
+  if (small) {
+    HIP_OR_FAIL(hipStreamSynchronize(s->stream));
+    for (int k = 0; k < count; ++k)
+      if (wanted[k].host)
+        std::memcpy(wanted[k].host, F.*wanted[k].slot, sizeof(double) * wanted[k].width * s->n);
+    return HLB_OK;
+  }
   std::vector<hlb::HostSegment> segments;
   for (int k = 0; k < count; ++k)
     if (wanted[k].host)

@@ -82,10 +82,12 @@ struct hlbn_net {
   Buf<float> gtmp;  // an output gradient of a layer that hlbn::dpre does not take
   Buf<uint16_t> dpre16;
   Buf<float> dpre32, part;
-  Buf<float> wc, loss_sums;
+  // pinned host memory: the loss per channel, written by the reduction itself
+  float* loss_sums = nullptr;
   int64_t head_chunk = 0;
 
   ~hlbn_net() {
+    if (loss_sums) (void)hipHostFree(loss_sums);
     for (auto& e : ev)
       if (e) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
@@ -336,7 +338,7 @@ int hlbn_create(int32_t side, int32_t batch, int32_t in_channels, int32_t out_ch
     HIPN(n->dpre32.alloc(unfused_pc));
     HIPN(n->gtmp.alloc(unfused_pc));
   }
-  HIPN(n->loss_sums.alloc(out_channels));
+  HIPN(hipHostMalloc((void**)&n->loss_sums, sizeof(float) * out_channels));
   const int64_t P0 = n->P[0];
   HIPN(n->xin.alloc(P0 * n->cinp));
   HIPN(n->in32.alloc(P0 * in_channels));
@@ -357,7 +359,6 @@ int hlbn_create(int32_t side, int32_t batch, int32_t in_channels, int32_t out_ch
   HIPN(n->lterm.alloc(P0 * out_channels));
   HIPN(n->tgt32.alloc(P0 * out_channels));
   HIPN(n->mask8.alloc(P0));
-  HIPN(n->wc.alloc(out_channels));
   if (refresh_weights(n.get())) return 1;
   HIPN(hipStreamSynchronize(n->stream));
   *out = n.release();
@@ -444,24 +445,20 @@ int hlbn_backward(hlbn_net* n, const float* target, const uint8_t* mask,
     t = n->tgt32.p;
     m = n->mask8.p;
   }
-  HIPN(hipMemcpyAsync(n->wc.p, channel_weights, sizeof(float) * n->cout, hipMemcpyHostToDevice,
-                      n->stream));
+  hlbn::ChannelWeights wc{};
+  std::copy(channel_weights, channel_weights + n->cout, wc.w);
   HIPN(hipEventRecord(n->ev[1], n->stream));
   const float inv = (float)(1.0 / (std::max(mask_count, 1.0) * n->cout));
-  KERN(hlbn::mse(P0, n->cout, n->out.p, t, m, n->wc.p, inv, n->dout.p, n->lterm.p, n->stream));
+  KERN(hlbn::mse(P0, n->cout, n->out.p, t, m, wc, inv, n->dout.p, n->lterm.p, n->stream));
   if (backward_impl(n)) return 1;
   HIPN(hipEventRecord(n->ev[2], n->stream));
   if (loss) {
     // loss terms summed per channel in a fixed order, then on the host
-    KERN(hlbn::channel_sum(n->lterm.p, P0, n->cout, n->part.p, n->head_chunk,
-                           n->loss_sums.p,
+    KERN(hlbn::channel_sum(n->lterm.p, P0, n->cout, n->part.p, n->head_chunk, n->loss_sums,
                            n->stream));
-    std::vector<float> h(n->cout);
-    HIPN(hipMemcpyAsync(h.data(), n->loss_sums.p, sizeof(float) * n->cout, hipMemcpyDeviceToHost,
-                        n->stream));
     HIPN(hipStreamSynchronize(n->stream));
     double l = 0;
-    for (float v : h) l += v;
+    for (int k = 0; k < n->cout; ++k) l += n->loss_sums[k];
     *loss = l;
   }
   HIPN(hipStreamSynchronize(n->stream));

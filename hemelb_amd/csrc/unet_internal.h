@@ -82,8 +82,12 @@ int head_bwd_data(int64_t P, int K, int O, const float* dout, const float* W, fl
                   void* stream);
 int head_wgrad(int64_t P, int K, int O, const float* dout, const uint16_t* h, float* part,
                int64_t chunk, float* dW, float* db, void* stream);
+// Loss weights of up to 16 output channels, passed with the launch.
+struct ChannelWeights {
+  float w[16];
+};
 int mse(int64_t P, int O, const float* out, const float* target, const uint8_t* mask,
-        const float* wc, float inv_count, float* dout, float* lterm, void* stream);
+        const ChannelWeights& wc, float inv_count, float* dout, float* lterm, void* stream);
 int adam(int64_t n, float* p, const float* g, float* m, float* v, float lr, float b1, float b2,
          float eps, float wd, float c1, float c2, void* stream);
 

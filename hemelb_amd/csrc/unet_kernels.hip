@@ -1102,15 +1102,15 @@ __global__ void k_head_wgrad_part(int64_t P, int K, int O, const float* __restri
 // dout = 2 w_c (out - t) m / (count * O).
 __global__ void k_mse(int64_t P, int O, const float* __restrict__ out,
                       const float* __restrict__ target, const uint8_t* __restrict__ mask,
-                      const float* __restrict__ wc, float inv_count,
+                      ChannelWeights wc, float inv_count,
                       float* __restrict__ dout, float* __restrict__ lterm) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= P * O) return;
   const int o = (int)(i % O);
   const float m = mask[i / O] ? 1.f : 0.f;
   const float d = (out[i] - target[i]) * m;
-  dout[i] = 2.f * wc[o] * d * inv_count;
-  lterm[i] = wc[o] * d * d * inv_count;
+  dout[i] = 2.f * wc.w[o] * d * inv_count;
+  lterm[i] = wc.w[o] * d * d * inv_count;
 }
 
 // Adam (decoupled weight decay) on binary32 master parameters.
@@ -1530,7 +1530,7 @@ int head_wgrad(int64_t P, int K, int O, const float* dout, const uint16_t* h, fl
 }
 
 int mse(int64_t P, int O, const float* out, const float* target, const uint8_t* mask,
-        const float* wc, float inv_count, float* dout, float* lterm, void* stream) {
+        const ChannelWeights& wc, float inv_count, float* dout, float* lterm, void* stream) {
   hipLaunchKernelGGL(k_mse, blocks_for(P * O), dim3(256), 0, (hipStream_t)stream, P, O, out,
                      target, mask, wc, inv_count, dout, lterm);
   return (int)hipGetLastError();

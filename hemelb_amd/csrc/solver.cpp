@@ -1068,14 +1068,37 @@ static int create_impl(const hlb_params* params, const hlb_domain* dm, const hlb
   A.rho0 = P.storage == HLB_STORE_FP64 ? 0.0 : P.rho0;
   // MRT relaxation rate of the viscous moments (DHumieres*MRTBasis.cc)
   A.mrt_s_tau = 1.0 / P.tau;
-  // Default launch shape: the workgroup size and workgroup-to-XCD order
-  // that measured fastest on the vessel tree for each storage (two sweeps
-  // of every shape): 128-thread workgroups in runs of 2 (one half block)
-  // per XCD for binary64 (0.7 % ahead of runs of 8) and in runs of 8 (two
-  // blocks) for binary32; 64-thread workgroups in runs of 16 (two blocks)
-  // for binary16 (1-2 % ahead of 128 threads in the hardware order).
-  A.threads = P.storage == HLB_STORE_FP16 ? 64u : 128u;
-  A.xcd_remap = P.storage == HLB_STORE_FP64 ? 2u : P.storage == HLB_STORE_FP32 ? 8u : 16u;
+  // Default launch shape: workgroup size and workgroup-to-XCD order, by how
+  // the domain fills the chip (us a step, each shape timed on vessel trees,
+  // cylinders and ensembles of 1280 to 7.9 M sites).
+  // * Up to one wave per SIMD the step is one wave's latency: one-wave
+  //   workgroups spread over all CUs, in runs of two blocks per XCD so that a
+  //   neighbour's line is in the same L2 (1280 sites D3Q15 binary64 6.0 ->
+  //   5.1, 43 k D3Q19 binary64 9.0 -> 8.1, binary32 7.7 -> 7.3).
+  // * While both state arrays stay in the 256 MB cache beyond the L2s, pulls
+  //   of another XCD's lines are cheap and what counts is that a CU takes a
+  //   new plane as soon as one ends: one-wave workgroups in the hardware
+  //   order (binary64: 221 k sites MRT 24.8 -> 22.7, 820 k 64.0 -> 60.5;
+  //   1.8 M no longer, 127.2 / 126.9).  Binary32 gains to 64 MB only (221 k
+  //   15.6 -> 15.0, 420 k 26.4 -> 26.0, but 848 k 32.9 / 34.2).
+  // * Beyond that HBM traffic counts: 128-thread workgroups in runs of 2 for
+  //   binary64 (7.9 M sites 508, hardware order 512, one-wave 533) and in
+  //   runs of 8 for binary32 (288; 302; 315).
+  // * Binary16: one-wave workgroups in runs of 16 from 420 k sites up (7.9 M
+  //   184, hardware order 203) and within 2 % of the best below.
+  constexpr uint32_t kSimds = 1024;
+  const uint64_t state_bytes = 2ull * storage_bytes(P.storage) * Q * (uint64_t)n;
+  const uint64_t cached = P.storage == HLB_STORE_FP64 ? 256ull << 20 : 64ull << 20;
+  if (P.storage == HLB_STORE_FP16 || s->dom.nwaves <= kSimds) {
+    A.threads = 64u;
+    A.xcd_remap = 16u;
+  } else if (state_bytes <= cached) {
+    A.threads = 64u;
+    A.xcd_remap = 0u;
+  } else {
+    A.threads = 128u;
+    A.xcd_remap = P.storage == HLB_STORE_FP64 ? 2u : 8u;
+  }
   s->initialised = false;
   *out = s.release();
   return HLB_OK;

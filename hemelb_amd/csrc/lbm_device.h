@@ -714,6 +714,21 @@ __device__ __forceinline__ bool lane_cross_z(uint32_t lane) {
   else return (lane & LaneBits<M>::Z) == (CZ > 0 ? 0u : LaneBits<M>::Z);
 }
 
+// The same as a mask: all ones where x - c leaves the block across its y (z)
+// face, else zero.  Bit 6 of (coordinate bits - 1), or of (coordinate bits +
+// 64 - all of them), is set exactly there.  (The empty statement keeps the
+// compiler from turning the mask back into a compare and selects.)
+template <int C, uint32_t BITS>
+__device__ __forceinline__ uint32_t lane_cross_mask(uint32_t lane) {
+  if constexpr (C == 0) return 0u;
+  else {
+    uint32_t m = (uint32_t)__builtin_amdgcn_sbfe(
+        (int)((lane & BITS) + (C > 0 ? 0xFFFFFFFFu : 64u - BITS)), 6u, 1u);
+    asm("" : "+v"(m));
+    return m;
+  }
+}
+
 // Block layout: every 8^3 block holding fluid owns 512 slots (x-plane major,
 // lanes in the storage's in-plane order above) and its Q directions are stored together, block after block
 // ([block][direction][512 slots]), so that one block's distributions are
@@ -899,37 +914,66 @@ struct BlockLayout32 : BlockLayout {
     using C = std::conditional_t<std::is_const<P>::value, const char, char>;
     return (P*)(((C*)base + uni) + r.lane * ES);
   }
-  template <int Q, int E, typename P>
-  static __device__ __forceinline__ P* src_ptr(const SiteRef& r, P* base) {
+  // Byte offset of the value at x - c_E, where `pick(t)` gives the block of
+  // neighbour-table entry t.  The lanes that leave the block across its y or
+  // z face add the difference of two blocks' offsets under a mask (modulo
+  // 2^32): one `and` with a scalar and a part of one three-way add.  A select
+  // between two scalar offsets needs both moved to vector registers first, as
+  // a vector instruction takes one scalar operand.  The D3Q19 LBGK pull's
+  // vector instructions a wave: 185 -> 138 (binary64, binary32), 113 -> 84
+  // (binary16).  It shows where a wave's latency counts (1280 sites BFL
+  // binary64 7.63 -> 7.45 us a step, 43 k sites 8.21 -> 7.97) and not where
+  // memory does (trees within 0.2 %; binary16, 7.9 M sites, 182.4 -> 181.7).
+  template <int Q, int E, typename P, class Pick>
+  static __device__ __forceinline__ uint32_t src_off(const SiteRef& r, Pick pick) {
     constexpr int CX = Lat<Q>::c[E][0], CY = Lat<Q>::c[E][1], CZ = Lat<Q>::c[E][2];
     constexpr uint32_t ES = sizeof(P), BS = (uint32_t)Q * 512u * ES;
     constexpr bool M = kMortonLanes<std::remove_const_t<P>>;
+    using B = LaneBits<M>;
     const int lx = (int)(r.w & 7u);
     const bool bx = CX != 0 && (CX > 0 ? lx == 0 : lx == 7);  // wave-uniform
-    const bool by = lane_cross_y<CY, M>(r.lane);
-    const bool bz = lane_cross_z<CZ, M>(r.lane);
     constexpr int i000 = 13, i100 = 13 - 9 * CX, i010 = 13 - 3 * CY, i001 = 13 - CZ;
     constexpr int i110 = 13 - 9 * CX - 3 * CY, i101 = 13 - 9 * CX - CZ;
     constexpr int i011 = 13 - 3 * CY - CZ, i111 = 13 - 9 * CX - 3 * CY - CZ;
     // wave-uniform: direction E's array in each candidate block, source plane
+    // (readfirstlane keeps the products scalar: without it the compiler moves
+    // the multiply into a vector multiply)
     const uint32_t uni = ((uint32_t)E * 512u + ((uint32_t)((lx - CX) & 7) << 6)) * ES;
-    // (readfirstlane keeps these products scalar: without it the compiler
-    // sinks the multiply below the per-lane select, into a vector multiply)
     const auto blk = [&](int32_t t) {
-      return __builtin_amdgcn_readfirstlane((uint32_t)t * BS + uni);
+      return __builtin_amdgcn_readfirstlane((uint32_t)pick(t) * BS);
     };
     const uint32_t n00 = blk(bx ? r.tb[i100] : r.tb[i000]);
-    const uint32_t n10 = blk(bx ? r.tb[i110] : r.tb[i010]);
-    const uint32_t n01 = blk(bx ? r.tb[i101] : r.tb[i001]);
-    const uint32_t n11 = blk(bx ? r.tb[i111] : r.tb[i011]);
-    const uint32_t nb = by ? (bz ? n11 : n10) : (bz ? n01 : n00);
-    const uint32_t yz = lane_shift<CY, CZ, M>(r.lane) * ES;
+    uint32_t off = lane_shift<CY, CZ, M>(r.lane) * ES;
+    const uint32_t my = lane_cross_mask<CY, B::Y>(r.lane), mz = lane_cross_mask<CZ, B::Z>(r.lane);
+    uint32_t n10 = 0, n01 = 0;
+    if constexpr (CY != 0) {
+      n10 = blk(bx ? r.tb[i110] : r.tb[i010]);
+      off += my & (n10 - n00);
+    }
+    if constexpr (CZ != 0) {
+      n01 = blk(bx ? r.tb[i101] : r.tb[i001]);
+      off += mz & (n01 - n00);
+    }
+    if constexpr (CY != 0 && CZ != 0) {
+      const uint32_t n11 = blk(bx ? r.tb[i111] : r.tb[i011]);
+      off += (my & mz) & (n11 - n10 - n01 + n00);
+    }
+    return off + __builtin_amdgcn_readfirstlane(n00 + uni);
+  }
+  template <int Q, int E, typename P>
+  static __device__ __forceinline__ P* src_ptr(const SiteRef& r, P* base) {
     constexpr int DP = inv_dir(E);
-    // a cut link reads the site's own slot of the inverse direction
-    // (both offsets are formed first so that the choice is a select, not a
+    // a cut link reads the site's own slot of the inverse direction (both
+    // offsets are formed first so that the choice is a bit select, not a
     // divergent branch)
-    const uint32_t own = own_off<Q, P>(r, DP), src = nb + yz;
-    const uint32_t off = ((r.cut >> (DP - 1)) & 1u) ? own : src;
+    const uint32_t own = own_off<Q, P>(r, DP);
+    const uint32_t src = src_off<Q, E, P>(r, [](int32_t t) { return t; });
+    uint32_t off = src;
+    if constexpr (DP > 0) {
+      uint32_t cut = (uint32_t)__builtin_amdgcn_sbfe((int)r.cut, DP - 1, 1u);
+      asm("" : "+v"(cut));
+      off = (cut & own) | (~cut & src);
+    }
     using C = std::conditional_t<std::is_const<P>::value, const char, char>;
     return (P*)((C*)base + off);
   }
@@ -938,28 +982,11 @@ struct BlockLayout32 : BlockLayout {
   // replaced by the own block, so that the address stays inside the state.
   template <int Q, int E, typename P>
   static __device__ __forceinline__ P* src_any_ptr(const SiteRef& r, P* base) {
-    constexpr int CX = Lat<Q>::c[E][0], CY = Lat<Q>::c[E][1], CZ = Lat<Q>::c[E][2];
-    constexpr uint32_t ES = sizeof(P), BS = (uint32_t)Q * 512u * ES;
-    constexpr bool M = kMortonLanes<std::remove_const_t<P>>;
-    const int lx = (int)(r.w & 7u);
-    const bool bx = CX != 0 && (CX > 0 ? lx == 0 : lx == 7);  // wave-uniform
-    const bool by = lane_cross_y<CY, M>(r.lane);
-    const bool bz = lane_cross_z<CZ, M>(r.lane);
-    constexpr int i000 = 13, i100 = 13 - 9 * CX, i010 = 13 - 3 * CY, i001 = 13 - CZ;
-    constexpr int i110 = 13 - 9 * CX - 3 * CY, i101 = 13 - 9 * CX - CZ;
-    constexpr int i011 = 13 - 3 * CY - CZ, i111 = 13 - 9 * CX - 3 * CY - CZ;
-    const uint32_t uni = ((uint32_t)E * 512u + ((uint32_t)((lx - CX) & 7) << 6)) * ES;
     const int32_t self = (int32_t)(r.w >> 3);
-    const auto blk = [&](int32_t t) {
-      return __builtin_amdgcn_readfirstlane((uint32_t)(t < 0 ? self : t) * BS + uni);
-    };
-    const uint32_t n00 = blk(bx ? r.tb[i100] : r.tb[i000]);
-    const uint32_t n10 = blk(bx ? r.tb[i110] : r.tb[i010]);
-    const uint32_t n01 = blk(bx ? r.tb[i101] : r.tb[i001]);
-    const uint32_t n11 = blk(bx ? r.tb[i111] : r.tb[i011]);
-    const uint32_t nb = by ? (bz ? n11 : n10) : (bz ? n01 : n00);
+    const uint32_t off =
+        src_off<Q, E, P>(r, [&](int32_t t) { return t < 0 ? self : t; });
     using C = std::conditional_t<std::is_const<P>::value, const char, char>;
-    return (P*)((C*)base + (nb + lane_shift<CY, CZ, M>(r.lane) * ES));
+    return (P*)((C*)base + off);
   }
   // Streamed store of slot d of the lane's site: a buffer store whose scalar
   // offset carries the wave-uniform part and whose vector offset is the
@@ -1195,7 +1222,7 @@ __device__ __forceinline__ void gather_early(const DevDomain& D, const StepArgs&
   using St = Store<S>;
   using Lay = BlockLayout32;
   const bool bnd = (D.wave_bnd[r.w] >> r.lane) & 1ull;
-  f[0] = St::ld(Lay::template own_ptr<Q>(r, fin, 0));
+  f[0] = St::ld(own_ptr<Q, Lay>(D, r, fin, 0));
   sfor<1, Q>([&](auto ei) {
     constexpr int e = decltype(ei)::value;
     f[e] = St::ld(Lay::template src_any_ptr<Q, e>(r, fin));
@@ -1205,7 +1232,7 @@ __device__ __forceinline__ void gather_early(const DevDomain& D, const StepArgs&
   if (bnd) {
     sfor<1, Q>([&](auto ei) {
       constexpr int e = decltype(ei)::value;
-      own[e] = St::ld(Lay::template own_ptr<Q>(r, fin, e));
+      own[e] = St::ld(own_ptr<Q, Lay>(D, r, fin, e));
     });
     if (A.wall == 1) {
       const uint4* q8 = reinterpret_cast<const uint4*>(D.b_q16 + (int64_t)r.rec * kQS16<Q>);

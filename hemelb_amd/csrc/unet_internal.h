@@ -45,8 +45,9 @@ struct WeightLayers {
     int co, ci;
     uint16_t *w16, *wt16;
   } layer[kCount];
+  uint32_t first_tile[kCount];   // of each layer's 16 x 16 tiles (set by refresh_weights)
 };
-int refresh_weights(const WeightLayers& layers, const float* params, void* stream);
+int refresh_weights(WeightLayers layers, const float* params, void* stream);
 // ReLU backward with the bias gradient: dpre16 = bf16 of dpost where post > 0,
 // db[c] = sum_p of its binary32 values (part: ceil(P / wgrad_chunk) * C), for
 // C dividing 256 (dpre_fused).  dpost by kind:

@@ -909,20 +909,31 @@ __global__ void k_channel_sum_part(const float* __restrict__ a, int64_t P, int C
 }
 
 // bf16 copies of the weights for the forward pass, w16[t][co][ci], and for
-// backward-data, wt16[26 - t][ci][co], of every layer (blockIdx.y): one launch
-// instead of one per layer, most of which lasted no longer than a launch.
-// (64-bit indices, as a layer may have more than 2^31 weights: the default
-// network takes 13.4 us, 14.0 with 32-bit ones.)
-__global__ __launch_bounds__(256) void k_refresh_weights(WeightLayers layers,
+// backward-data, wt16[26 - t][ci][co], of every layer in one launch instead of
+// one per layer, most of which lasted no longer than a launch.  A workgroup
+// takes one tap of a 16 x 16 tile through LDS, so that both copies are written
+// in whole 32-byte rows: bound by the bytes once a network is large.  (A weight
+// per thread with the transposed copy in strided 2-byte stores takes 13.4 us
+// on the default network, this 7.3; with Adam on the 75 M weights of channels
+// 128 to 1024 1000 us and 785.)  64-bit offsets, as a layer may have 2^31
+// weights.
+__global__ __launch_bounds__(256) void k_refresh_weights(WeightLayers layers, uint32_t first,
                                                          const float* __restrict__ params) {
-  const WeightLayers::Layer& l = layers.layer[blockIdx.y];
-  const int64_t n = (int64_t)l.co * l.ci, total = 27 * n, step = (int64_t)gridDim.x * 256;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += step) {
-    const int64_t t = i / n, r = i - t * n, o = r / l.ci, c = r - o * l.ci;
-    const uint16_t b = f2bf(params[l.woff + i]);
-    l.w16[i] = b;
-    l.wt16[((26 - t) * l.ci + c) * l.co + o] = b;
-  }
+  __shared__ uint16_t tile[16][17];
+  const uint32_t b = first + blockIdx.x;
+  int k = 0;
+  while (k + 1 < WeightLayers::kCount && b >= layers.first_tile[k + 1]) ++k;
+  const WeightLayers::Layer& l = layers.layer[k];
+  const uint32_t nc = l.ci / 16, per_tap = l.co / 16 * nc, in_layer = b - layers.first_tile[k];
+  const uint32_t t = in_layer / per_tap, at = in_layer - t * per_tap;
+  const uint32_t to = at / nc, tc = at - to * nc;
+  const int i = threadIdx.x / 16, j = threadIdx.x % 16;
+  const int64_t in = ((int64_t)t * l.co + to * 16 + i) * l.ci + tc * 16 + j;
+  const uint16_t v = f2bf(params[l.woff + in]);
+  l.w16[in] = v;
+  tile[i][j] = v;
+  __syncthreads();
+  l.wt16[((int64_t)(26 - t) * l.ci + tc * 16 + i) * l.co + to * 16 + j] = tile[j][i];
 }
 
 // dpre_bf16[i] = dpost[i] if post[i] > 0 else 0  (ReLU backward)
@@ -1414,9 +1425,17 @@ int channel_sum(const float* a, int64_t P, int C, float* part, int64_t chunk, fl
   return (int)hipGetLastError();
 }
 
-int refresh_weights(const WeightLayers& layers, const float* params, void* stream) {
-  hipLaunchKernelGGL(k_refresh_weights, dim3(128, WeightLayers::kCount), dim3(256), 0,
-                     (hipStream_t)stream, layers, params);
+int refresh_weights(WeightLayers layers, const float* params, void* stream) {
+  uint32_t tiles = 0;
+  for (int k = 0; k < WeightLayers::kCount; ++k) {
+    layers.first_tile[k] = tiles;
+    tiles += 27u * (layers.layer[k].co / 16) * (layers.layer[k].ci / 16);
+  }
+  // (a grid has fewer than 2^32 threads)
+  constexpr uint32_t kLaunch = 1u << 23;
+  for (uint32_t first = 0; first < tiles; first += kLaunch)
+    hipLaunchKernelGGL(k_refresh_weights, dim3(std::min(tiles - first, kLaunch)), dim3(256), 0,
+                       (hipStream_t)stream, layers, first, params);
   return (int)hipGetLastError();
 }
 

@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "unet_internal.h"
+#include "unet_plan.h"
 
 namespace hlbn {
 namespace {
@@ -1164,41 +1165,6 @@ void sum_chunks(const float* part, int64_t nchunks, int64_t n, float* out, hipSt
 }  // namespace
 
 namespace {
-// Launch plan of a forward convolution: NT output-channel tiles per wave
-// (an A fragment feeds NT MFMAs), MT position tiles (a B fragment feeds MT)
-// and the number of K slices.  Fine levels keep MT = 4 or 2; coarse levels,
-// with few positions, first take fewer position tiles per wave and then
-// split K so that the grid has about four waves per SIMD and each wave a
-// short chain of K steps.
-struct FwdPlan {
-  int mt, nt, nsplit, hpw;
-  int64_t waves;
-};
-FwdPlan fwd_plan(const ConvGeom& cg, int ci, int co) {
-  const int64_t P = (int64_t)cg.N * cg.D * cg.H * cg.W;
-  const int tiles = co / 16;
-  FwdPlan f;
-  f.nt = tiles >= 8 ? 8 : (tiles >= 3 ? 4 : tiles);
-  f.mt = f.nt >= 8 ? 2 : 4;
-  const int ngroups = (tiles + f.nt - 1) / f.nt;
-  constexpr int64_t kTarget = 4096;
-  while (f.mt > 1 && ((P + 16 * f.mt - 1) / (16 * f.mt)) * ngroups < kTarget) f.mt /= 2;
-  f.waves = ((P + 16 * f.mt - 1) / (16 * f.mt)) * ngroups;
-  const int nhalf = 27 * (ci / 16);
-  const int ksteps = (nhalf + 1) / 2;
-  int ns = (int)std::min<int64_t>(ksteps, (kTarget + f.waves - 1) / f.waves);
-  int kps = (ksteps + ns - 1) / ns;  // K steps per slice
-  f.hpw = 2 * kps;
-  f.nsplit = (nhalf + f.hpw - 1) / f.hpw;
-  if (f.nsplit <= 1) {
-    f.nsplit = 1;
-    f.hpw = nhalf + 1;
-  }
-  return f;
-}
-}  // namespace
-
-namespace {
 struct BoxCall {
   Grid3 g;
   ConvSrc src;
@@ -1225,80 +1191,26 @@ void box_launch(const BoxCall& c) {
     hipLaunchKernelGGL((k_conv_box<NG, NT, MT, WM, BD, BH, BW, false>), grid, block, 0, c.stream,
                        c.g, c.src, c.w, c.bias, c.co, c.y32, c.y16, c.yc, c.yoff, c.relu, 0);
 }
-// Whether k_conv_box has a form for ci input channels.
-bool box_channels(int ci) {
-  const int ng = ci / 16;
-  return (ng >= 1 && ng <= 4) || ng == 6 || ng == 8 || ng == 12;
-}
-// Boxes are 16 wide where that pads the width no more than 8, and hold as
-// many positions as still leave about two workgroups per CU: a large box
-// re-reads less halo, a small one fills the chip (32 -> 32 channels at
-// 2 x 32^3: 21 us in boxes of 64 positions and one output tile, 13 in boxes
-// of 128 and two).  Many input channels bound the box by LDS instead; there
-// half the box (12 groups) and twice (6) measured the same within 3 %.
-template <int BW>
-bool box_dispatch(const BoxCall& c, int ci) {
-  constexpr int H = BW == 16 ? 1 : 2;  // rows of w per 16 positions
-  const int64_t P = (int64_t)c.g.N * c.g.D * c.g.H * c.g.W;
-  const int T = c.co / 16;
-  const bool large = P >= 512 * 256, medium = P >= 256 * 128;
-  switch (ci / 16) {
-    case 1:
-      if (!medium) box_launch<1, 1, 1, 4, 1, 4 * H, BW>(c);
-      else if (!large && T % 2 == 0) box_launch<1, 2, 2, 4, 2, 4 * H, BW>(c);
-      else if (!large) box_launch<1, 1, 2, 4, 2, 4 * H, BW>(c);
-      else if (T % 3 == 0) box_launch<1, 3, 4, 4, 4, 4 * H, BW>(c);
-      else if (T % 2 == 0) box_launch<1, 2, 4, 4, 4, 4 * H, BW>(c);
-      else box_launch<1, 1, 8, 4, BW == 16 ? 4 : 8, 8, BW>(c);
-      return true;
-    case 2:
-      if (!medium) box_launch<2, 1, 1, 4, 1, 4 * H, BW>(c);
-      else if (!large && T % 2 == 0) box_launch<2, 2, 2, 4, 2, 4 * H, BW>(c);
-      else if (!large) box_launch<2, 1, 2, 4, 2, 4 * H, BW>(c);
-      else if (T % 3 == 0) box_launch<2, 3, 4, 4, 4, 4 * H, BW>(c);
-      else if (T % 2 == 0) box_launch<2, 2, 4, 4, 4, 4 * H, BW>(c);
-      else box_launch<2, 1, 4, 4, 4, 4 * H, BW>(c);
-      return true;
-    case 3:
-      if (!medium) box_launch<3, 1, 1, 4, 1, 4 * H, BW>(c);
-      else if (!large) box_launch<3, 1, 2, 4, 2, 4 * H, BW>(c);
-      else box_launch<3, 1, 4, 4, 4, 4 * H, BW>(c);
-      return true;
-    case 4:
-      if (T <= 2) box_launch<4, 1, 2, 2, 2, 2 * H, BW>(c);
-      else if (P >= 64 * 256) box_launch<4, 1, 4, 1, 2, 2 * H, BW>(c);
-      else box_launch<4, 1, 2, 1, 1, 2 * H, BW>(c);
-      return true;
-    case 6:
-      box_launch<6, 1, 2, 2, 2, 2 * H, BW>(c);
-      return true;
-    case 8:
-      if (P >= 64 * 256) box_launch<8, 1, 4, 1, 2, 2 * H, BW>(c);
-      else box_launch<8, 1, 1, 2, 1, 2 * H, BW>(c);
-      return true;
-    case 12:
-      box_launch<12, 1, 4, 1, 2, 2 * H, BW>(c);
-      return true;
+// False where no such form exists.
+bool box_launch_form(const BoxCall& c, const BoxForm& f) {
+#define HLBN_BOX(NG, NT, MT, WM, BD, BH, BW)       \
+  if (f == BoxForm{NG, NT, MT, WM, BD, BH, BW}) {  \
+    box_launch<NG, NT, MT, WM, BD, BH, BW>(c);     \
+    return true;                                   \
   }
+  HLBN_BOX_FORMS(HLBN_BOX)
+#undef HLBN_BOX
   return false;
 }
 }  // namespace
 
 int64_t conv_fwd_ws(const ConvGeom& cg, int ci, int co) {
-  if (box_channels(ci)) return 0;
+  if (box_form(cg, ci, co).ng) return 0;
   const FwdPlan f = fwd_plan(cg, ci, co);
   return f.nsplit > 1 ? (int64_t)f.nsplit * cg.N * cg.D * cg.H * cg.W * co : 0;
 }
 
 namespace {
-// Box width of the LDS-staged weight gradient for this level (0: the level
-// does not tile into 4 x BH x BW boxes and takes the direct kernel).
-int wgrad_box_width(const ConvGeom& cg) {
-  if (cg.D % 4) return 0;
-  if (cg.W % 16 == 0 && cg.H % 4 == 0) return 16;
-  if (cg.W % 8 == 0 && cg.H % 8 == 0) return 8;
-  return 0;
-}
 // Boxes per workgroup: at least about 1024 workgroups over the tile pairs.
 int64_t wgrad_boxes_per_group(const ConvGeom& cg, int ci, int co) {
   const int64_t nboxes = (int64_t)cg.N * cg.D * cg.H * cg.W / 256;
@@ -1308,7 +1220,7 @@ int64_t wgrad_boxes_per_group(const ConvGeom& cg, int ci, int co) {
 }  // namespace
 
 bool conv_takes_parts(const ConvGeom& cg, int ci) {
-  return box_channels(ci) && wgrad_box_width(cg) != 0;
+  return box_form(cg, ci, 16).ng != 0 && wgrad_box_width(cg) != 0;
 }
 
 int conv_fwd(const ConvGeom& cg, const uint16_t* x, const uint16_t* xu, int cu, int ci,
@@ -1318,12 +1230,11 @@ int conv_fwd(const ConvGeom& cg, const uint16_t* x, const uint16_t* xu, int cu, 
   const Grid3 g{cg.N, cg.D, cg.H, cg.W};
   const int64_t P = (int64_t)cg.N * cg.D * cg.H * cg.W;
   const FwdPlan f = fwd_plan(cg, ci, co);
-  if (box_channels(ci)) {
+  const BoxForm form = box_form(cg, ci, co);
+  if (form.ng) {
     const BoxCall c{g, ConvSrc{x, xu, xu ? cu : 0}, w, bias, co, y32, y16, yc, yoff, relu,
                     f.nsplit > 1 ? f.hpw / 2 : 0, (hipStream_t)stream};
-    const bool wide = (cg.W + 15) / 16 * 16 == (cg.W + 7) / 8 * 8;
-    if (!(wide ? box_dispatch<16>(c, ci) : box_dispatch<8>(c, ci)))
-      return (int)hipErrorInvalidValue;
+    if (!box_launch_form(c, form)) return (int)hipErrorInvalidValue;
     return (int)hipGetLastError();
   }
   if (xu) return (int)hipErrorInvalidValue;

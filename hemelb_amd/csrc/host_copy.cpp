@@ -108,10 +108,11 @@ struct Job {
 hipError_t copy_to_host(const std::vector<HostSegment>& segments, hipStream_t stream) {
   size_t total = 0;
   for (const HostSegment& g : segments) total += g.bytes;
+  if (total < kDirect) return copy_direct(segments, stream);
   Staging& st = staging();
   std::unique_lock<std::mutex> lock(st.mu, std::try_to_lock);
   // another thread's copy has the staging buffer: take the runtime's path
-  if (total < kDirect || !lock.owns_lock()) return copy_direct(segments, stream);
+  if (!lock.owns_lock()) return copy_direct(segments, stream);
   if (!st.pinned && hipHostMalloc((void**)&st.pinned, kSlots * kChunk) != hipSuccess) {
     st.pinned = nullptr;
     (void)hipGetLastError();

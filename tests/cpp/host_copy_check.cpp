@@ -1,0 +1,44 @@
+// Scenarios of hlb::copy_to_host on the fake HIP runtime, chosen by argv[1];
+// prints what happened and returns 0, or 1 after a wrong result.
+#include <chrono>
+#include <cstdio>
+#include <string>
+#include <vector>
+
+#include "fake_hip.h"
+#include "host_copy.h"
+
+namespace {
+
+constexpr size_t kLarge = (size_t(64) << 20) + 12345, kSmall = size_t(1) << 20;
+
+std::vector<char> pattern(size_t n, unsigned seed) {
+  std::vector<char> v(n);
+  for (size_t i = 0; i < n; ++i) v[i] = (char)((i * 2654435761u + seed) >> 11);
+  return v;
+}
+void nap(double s) { std::this_thread::sleep_for(std::chrono::duration<double>(s)); }
+
+// A small copy waits for its stream while another solver's large one starts.
+int small_beside_large() {
+  ihipStream_t a(0), b(0);
+  const auto small = pattern(kSmall, 1), large = pattern(kLarge, 2);
+  std::vector<char> small_out(kSmall), large_out(kLarge);
+  a.gate(false);
+  std::thread t([&] { (void)hlb::copy_to_host({{small_out.data(), small.data(), kSmall}}, &a); });
+  while (fake::direct == 0) nap(0.001);   // its copy is queued
+  const hipError_t e = hlb::copy_to_host({{large_out.data(), large.data(), kLarge}}, &b);
+  const int staged = fake::staged;
+  a.gate(true);
+  t.join();
+  std::printf("staged %d\n", staged);
+  return e == hipSuccess && small_out == small && large_out == large ? 0 : 1;
+}
+
+}  // namespace
+
+int main(int, char** argv) {
+  const std::string what = argv[1];
+  if (what == "small_beside_large") return small_beside_large();
+  return 2;
+}

@@ -11,9 +11,10 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace hlb {
@@ -47,23 +48,63 @@ hipError_t copy_direct(const std::vector<HostSegment>& segments, hipStream_t str
 
 // The chunks of one copy and the hand-over between the issuing thread and the
 // workers: chunk i travels through slot i % kSlots, which is issued again
-// only after done[i].
+// only after done[i].  The workers sleep until the stream has reached the copy
+// (the steps queued before it may take seconds); the copy itself is short, and
+// they poll for its chunks.
 struct Job {
   std::vector<HostSegment> chunks;
   std::vector<std::atomic<bool>> done;
   std::atomic<size_t> next{0}, issued{0};
   std::atomic<int> error{(int)hipSuccess};
-  hipEvent_t arrived[kSlots] = {};
-  char* pinned;
+  hipEvent_t arrived[kSlots] = {}, reached = nullptr;
+  char* pinned = nullptr;
   int device;
+  std::mutex mu;
+  std::condition_variable begun;
+  enum { kWaiting, kBegun, kDropped } state = kWaiting;
+  std::vector<std::thread> workers;
 
-  Job(std::vector<HostSegment> c, char* p, int dev)
-      : chunks(std::move(c)), done(chunks.size()), pinned(p), device(dev) {
+  Job(std::vector<HostSegment> c, int dev)
+      : chunks(std::move(c)), done(chunks.size()), device(dev) {
     for (auto& d : done) d.store(false, std::memory_order_relaxed);
   }
   ~Job() {
+    finish();
     for (auto& e : arrived)
       if (e) (void)hipEventDestroy(e);
+    if (reached) (void)hipEventDestroy(reached);
+  }
+  hipError_t create_events() {
+    hipError_t e = hipEventCreateWithFlags(&reached, hipEventDisableTiming | hipEventBlockingSync);
+    for (int k = 0; k < kSlots && e == hipSuccess; ++k)
+      e = hipEventCreateWithFlags(&arrived[k], hipEventDisableTiming);
+    return e;
+  }
+  // As many workers as the system gives, up to `wanted`.
+  bool start_workers(size_t wanted) {
+    try {
+      workers.reserve(wanted);
+      for (size_t k = 0; k < wanted; ++k) workers.emplace_back([this] { work(); });
+    } catch (const std::exception&) {
+    }
+    return !workers.empty();
+  }
+  void begin() {
+    {
+      std::lock_guard<std::mutex> lock(mu);
+      state = kBegun;
+    }
+    begun.notify_all();
+  }
+  // Waits for the workers; if the copy has not begun they have nothing to do.
+  void finish() {
+    {
+      std::lock_guard<std::mutex> lock(mu);
+      if (state == kWaiting) state = kDropped;
+    }
+    begun.notify_all();
+    for (auto& w : workers) w.join();
+    workers.clear();
   }
   void fail(hipError_t e) {
     int none = (int)hipSuccess;
@@ -73,6 +114,11 @@ struct Job {
 
   void work() {
     (void)hipSetDevice(device);
+    {
+      std::unique_lock<std::mutex> lock(mu);
+      begun.wait(lock, [this] { return state != kWaiting; });
+      if (state == kDropped) return;
+    }
     for (;;) {
       const size_t i = next.fetch_add(1);
       if (i >= chunks.size()) return;
@@ -99,6 +145,7 @@ struct Job {
       if (e == hipSuccess) e = hipEventRecord(arrived[slot], stream);
       if (e != hipSuccess) return fail(e);
       issued.store(i + 1, std::memory_order_release);
+      if (i == 0) begin();
     }
   }
 };
@@ -109,15 +156,6 @@ hipError_t copy_to_host(const std::vector<HostSegment>& segments, hipStream_t st
   size_t total = 0;
   for (const HostSegment& g : segments) total += g.bytes;
   if (total < kDirect) return copy_direct(segments, stream);
-  Staging& st = staging();
-  std::unique_lock<std::mutex> lock(st.mu, std::try_to_lock);
-  // another thread's copy has the staging buffer: take the runtime's path
-  if (!lock.owns_lock()) return copy_direct(segments, stream);
-  if (!st.pinned && hipHostMalloc((void**)&st.pinned, kSlots * kChunk) != hipSuccess) {
-    st.pinned = nullptr;
-    (void)hipGetLastError();
-    return copy_direct(segments, stream);
-  }
   std::vector<HostSegment> chunks;
   for (const HostSegment& g : segments)
     for (size_t a = 0; a < g.bytes; a += kChunk)
@@ -125,21 +163,27 @@ hipError_t copy_to_host(const std::vector<HostSegment>& segments, hipStream_t st
   int device = 0;
   hipError_t e = hipGetDevice(&device);
   if (e != hipSuccess) return e;
-  Job job(std::move(chunks), st.pinned, device);
-  for (auto& ev : job.arrived) {
-    e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-    if (e != hipSuccess) return e;
+  Job job(std::move(chunks), device);
+  e = job.create_events();
+  if (e == hipSuccess) e = hipEventRecord(job.reached, stream);
+  if (e != hipSuccess) return e;
+  const bool workers = job.start_workers(std::min<size_t>(kMaxWorkers, total / (2 * kChunk)));
+  // The staging memory is taken once there is something to copy, so that
+  // another thread's copy can have it meanwhile.
+  e = hipEventSynchronize(job.reached);
+  if (e != hipSuccess) return e;
+  Staging& st = staging();
+  std::unique_lock<std::mutex> lock(st.mu, std::try_to_lock);
+  // another thread's copy has the staging buffer: take the runtime's path
+  if (!workers || !lock.owns_lock()) return copy_direct(segments, stream);
+  if (!st.pinned && hipHostMalloc((void**)&st.pinned, kSlots * kChunk) != hipSuccess) {
+    st.pinned = nullptr;
+    (void)hipGetLastError();
+    return copy_direct(segments, stream);
   }
-  const size_t wanted = std::min<size_t>(kMaxWorkers, total / (2 * kChunk));
-  std::vector<std::thread> workers;
-  workers.reserve(wanted);
-  try {
-    for (size_t k = 0; k < wanted; ++k) workers.emplace_back([&job] { job.work(); });
-  } catch (const std::system_error&) {
-  }
-  if (workers.empty()) return copy_direct(segments, stream);
+  job.pinned = st.pinned;
   job.issue(stream);
-  for (auto& w : workers) w.join();
+  job.finish();
   // no copy may still write the staging buffer or read the source
   e = hipStreamSynchronize(stream);
   return job.failed() ? (hipError_t)job.error.load() : e;

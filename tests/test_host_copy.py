@@ -31,3 +31,12 @@ def check(tmp_path_factory):
 def test_a_small_copy_leaves_the_staging_memory_to_others(check):
     # 65 chunks of 1 MiB, all through the staging memory
     assert check("small_beside_large")["staged"] == 65
+
+
+def test_waiting_for_the_steps_before_it_costs_no_processor_time(check):
+    # 0.4 s of waiting, of which a tenth of one processor is allowed
+    assert check("waiting")["cpu"] < 0.04
+
+
+def test_a_copy_that_waits_for_its_steps_leaves_the_staging_memory_to_others(check):
+    assert check("large_beside_waiting")["staged"] == 65

@@ -150,6 +150,22 @@ struct Job {
   }
 };
 
+// Makes `device` the thread's current one for a scope.
+struct CurrentDevice {
+  int before = -1;
+  hipError_t set(int device) {
+    int now = 0;
+    hipError_t e = hipGetDevice(&now);
+    if (e != hipSuccess || now == device) return e;
+    e = hipSetDevice(device);
+    if (e == hipSuccess) before = now;
+    return e;
+  }
+  ~CurrentDevice() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+};
+
 }  // namespace
 
 hipError_t copy_to_host(const std::vector<HostSegment>& segments, hipStream_t stream) {
@@ -160,8 +176,12 @@ hipError_t copy_to_host(const std::vector<HostSegment>& segments, hipStream_t st
   for (const HostSegment& g : segments)
     for (size_t a = 0; a < g.bytes; a += kChunk)
       chunks.push_back({(char*)g.dst + a, (const char*)g.src + a, std::min(kChunk, g.bytes - a)});
+  // an event is recorded on streams of the device it was created on alone, and
+  // the caller's current device need not be the stream's
   int device = 0;
-  hipError_t e = hipGetDevice(&device);
+  hipError_t e = hipStreamGetDevice(stream, &device);
+  CurrentDevice current;
+  if (e == hipSuccess) e = current.set(device);
   if (e != hipSuccess) return e;
   Job job(std::move(chunks), device);
   e = job.create_events();
@@ -176,7 +196,9 @@ hipError_t copy_to_host(const std::vector<HostSegment>& segments, hipStream_t st
   std::unique_lock<std::mutex> lock(st.mu, std::try_to_lock);
   // another thread's copy has the staging buffer: take the runtime's path
   if (!workers || !lock.owns_lock()) return copy_direct(segments, stream);
-  if (!st.pinned && hipHostMalloc((void**)&st.pinned, kSlots * kChunk) != hipSuccess) {
+  // (portable: every device's copies go through it)
+  if (!st.pinned && hipHostMalloc((void**)&st.pinned, kSlots * kChunk, hipHostMallocPortable) !=
+                        hipSuccess) {
     st.pinned = nullptr;
     (void)hipGetLastError();
     return copy_direct(segments, stream);

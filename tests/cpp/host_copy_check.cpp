@@ -77,6 +77,16 @@ int large_beside_waiting() {
   return e1 == hipSuccess && e2 == hipSuccess && out1 == first && out2 == second ? 0 : 1;
 }
 
+// A solver on another device than the thread's current one.
+int other_device() {
+  ihipStream_t s(1);
+  const auto data = pattern(kLarge, 6);
+  std::vector<char> out(kLarge);
+  const hipError_t e = hlb::copy_to_host({{out.data(), data.data(), kLarge}}, &s);
+  std::printf("error %d current %d staged %d\n", (int)e, fake::device, (int)fake::staged);
+  return e != hipSuccess || out == data ? 0 : 1;
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -84,5 +94,6 @@ int main(int, char** argv) {
   if (what == "small_beside_large") return small_beside_large();
   if (what == "waiting") return waiting();
   if (what == "large_beside_waiting") return large_beside_waiting();
+  if (what == "other_device") return other_device();
   return 2;
 }

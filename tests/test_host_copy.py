@@ -40,3 +40,7 @@ def test_waiting_for_the_steps_before_it_costs_no_processor_time(check):
 
 def test_a_copy_that_waits_for_its_steps_leaves_the_staging_memory_to_others(check):
     assert check("large_beside_waiting")["staged"] == 65
+
+
+def test_the_solvers_device_need_not_be_the_current_one(check):
+    assert check("other_device") == {"error": 0, "current": 0, "staged": 65}

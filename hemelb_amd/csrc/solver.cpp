@@ -1484,15 +1484,17 @@ static int instance_chunks(hlb_solver* s) {
   const int64_t all = planes ? (int64_t)s->dom.nwaves : s->n;
   const int64_t size = (all / 2048 + unit) / unit * unit;
   std::vector<int64_t> range;
+  std::vector<int32_t> inst;
   for (const auto& r : s->runs) {
     const int64_t begin = planes ? r.wave0 : r.start, end = planes ? r.wave1 : r.end;
     for (int64_t a = begin; a < end; a += size) {
       range.push_back(a);
       range.push_back(std::min(end, a + size));
-      s->chunk_inst.push_back(r.inst);
+      inst.push_back(r.inst);
     }
   }
   HIP_OR_FAIL(s->d_chunks.upload(range));
+  s->chunk_inst = std::move(inst);  // the list is there once the device has it
   return HLB_OK;
 }
 

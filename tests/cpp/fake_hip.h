@@ -82,6 +82,7 @@ inline thread_local int device = 0;            // the thread's current device
 inline std::mutex mu;
 inline std::map<char*, size_t> pinned;         // hipHostMalloc
 inline std::atomic<int> staged{0}, direct{0};  // copies to pinned and to pageable memory
+inline std::function<void(hipEvent_t)> on_event = [](hipEvent_t) {};  // the stream reached it
 
 inline bool is_pinned(const void* p) {
   std::lock_guard<std::mutex> lock(mu);
@@ -148,6 +149,7 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   if (e->device != s->device) return hipErrorInvalidHandle;
   ++e->pending;
   s->push([e] {
+    fake::on_event(e);
     std::lock_guard<std::mutex> lock(e->mu);
     --e->pending;
     e->cv.notify_all();

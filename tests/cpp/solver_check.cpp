@@ -1,0 +1,140 @@
+// Scenarios of the solver's host code (csrc/solver.cpp) on the fake HIP
+// runtime, with the kernels replaced by stand-ins that note their arguments.
+// argv[1] chooses one; prints what happened.
+#include <cstdio>
+#include <string>
+#include <vector>
+
+#include "fake_hip_memory.h"
+#include "hemelb_amd.h"
+#include "lbm_internal.h"
+
+namespace {
+
+std::vector<int64_t> seen_range;      // of the last monitor launch
+bool monitor_had_range = false;
+
+}  // namespace
+
+namespace hlb {
+
+int monitor_groups(const DevDomain&) { return 1; }
+int launch_fill(const DevDomain&, const StepArgs&, const double*, void*, void*) { return 0; }
+int launch_step(const DevDomain&, const StepArgs&, const void*, void*, void*) { return 0; }
+int launch_collide_only(const DevDomain&, const StepArgs&, const void*, void*, void*) { return 0; }
+int launch_export_distributions(const DevDomain&, const StepArgs&, const void*, int,
+                                const int64_t*, double*, void*) {
+  return 0;
+}
+int launch_export_fields(const DevDomain&, const StepArgs&, const void*, int, const FieldPtrs&,
+                         void*) {
+  return 0;
+}
+int launch_import(const DevDomain&, const StepArgs&, const double*, const int64_t*, void*, void*) {
+  return 0;
+}
+int launch_import_equilibrium(const DevDomain&, const StepArgs&, const double*, const double*,
+                              const int64_t*, void*, void*) {
+  return 0;
+}
+int launch_copy_arrays(int, int64_t, int64_t, int64_t, int, const void*, void*, uint32_t, uint32_t,
+                       void*) {
+  return 0;
+}
+int launch_halo(int64_t, const int64_t*, int, const void*, void*, int, void*) { return 0; }
+int launch_monitor(const DevDomain&, const StepArgs&, const void*, int, const int64_t* range,
+                   int groups, double* partials, double*, void*) {
+  monitor_had_range = range != nullptr;
+  seen_range.clear();
+  if (range) seen_range.assign(range, range + 2 * groups);
+  std::fill(partials, partials + 5 * groups, 0.0);
+  return 0;
+}
+int launch_snapshot_velocity(const DevDomain&, const StepArgs&, const void*, int, double*, void*) {
+  return 0;
+}
+int launch_velocity_change(const DevDomain&, const StepArgs&, const void*, int, const int64_t*,
+                           int groups, const double*, const double*, double, double* partials,
+                           void*) {
+  std::fill(partials, partials + groups, 0.0);
+  return 0;
+}
+int scratch_address(int, double** out) {
+  static std::vector<double> scratch(kStaticScratchDoubles);
+  *out = scratch.data();
+  return 0;
+}
+int launch_scatter_pairs(int64_t, int64_t, int, int, const int64_t*, const double*, int, double,
+                         const double*, void*, void*) {
+  return 0;
+}
+int launch_gather_pairs(int64_t, int64_t, int, int, const int64_t*, const void*, int, double,
+                        const double*, double*, void*) {
+  return 0;
+}
+
+}  // namespace hlb
+
+namespace {
+
+// Isolated sites (every link a wall) in blocks of their own, one vessel each.
+struct Sites {
+  std::vector<int32_t> coords, ids, instance;
+  std::vector<uint32_t> type, wall, iolet;
+  std::vector<float> normals;
+  std::vector<double> tau;
+  hlb_solver* s = nullptr;
+
+  explicit Sites(int n) {
+    for (int i = 0; i < n; ++i) {
+      coords.insert(coords.end(), {32 * i, 0, 0});
+      normals.insert(normals.end(), {1.0f + i, 2.0f + i, 3.0f + i});
+      instance.push_back(i);
+    }
+    ids.assign(n, 0);
+    type.assign(n, HLB_SITE_FLUID);
+    wall.assign(n, (1u << 18) - 1);
+    iolet.assign(n, 0);
+    tau.assign(n, 0.8);
+    hlb_params p{};
+    p.lattice = 19;
+    p.tau = 0.8;
+    p.rho0 = 1.0;
+    hlb_domain d{n, coords.data(), type.data(), wall.data(), iolet.data(), ids.data(), nullptr,
+                 normals.data()};
+    const double rest[3] = {0.0, 0.0, 0.0};
+    if (hlb_create_ensemble(&p, &d, instance.data(), n, tau.data(), nullptr, 0, nullptr, 0, &s) ||
+        hlb_set_equilibrium(s, 1.0, rest)) {
+      std::printf("create: %s\n", hlb_last_error());
+      std::exit(1);
+    }
+  }
+  ~Sites() { hlb_destroy(s); }
+};
+
+// A failure while the per-vessel list of planes is sent to the device, then the
+// same call again.
+int instances_after(int& countdown) {
+  Sites v(3);
+  std::vector<hlb_instance_monitor> m(3);
+  countdown = 1;
+  const int first = hlb_reduce_instances(v.s, m.data());
+  countdown = 0;
+  const int second = hlb_reduce_instances(v.s, m.data());
+  std::printf("first %d second %d ranges %d", first, second, (int)seen_range.size() / 2);
+  bool ordered = monitor_had_range && seen_range.size() == 12;
+  for (size_t k = 0; k + 1 < seen_range.size(); ++k)
+    ordered = ordered && 0 <= seen_range[k] && seen_range[k] <= seen_range[k + 1] &&
+              seen_range[k + 1] <= 24;
+  std::printf(" ordered %d\n", (int)ordered);
+  return 0;
+}
+
+}  // namespace
+
+int main(int, char** argv) {
+  const std::string what = argv[1];
+  if (what == "instances_after_malloc") return instances_after(fake::fail_malloc);
+  if (what == "instances_after_memcpy") return instances_after(fake::fail_memcpy);
+  return 2;
+}

@@ -1,0 +1,37 @@
+"""The solver's host code after failed runtime calls (csrc/solver.cpp), on the
+CPU: linked with a fake HIP runtime that fails on demand and with stand-ins for
+the kernels (tests/cpp/solver_check.cpp)."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "hemelb_amd", "csrc")
+CPP = os.path.join(ROOT, "tests", "cpp")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+HLB_E_DEVICE = -2
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("solver") / "check")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Wno-missing-field-initializers",
+                    "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROCM, "include"),
+                    "-I", os.path.join(ROOT, "include"), "-I", CSRC, "-I", CPP,
+                    os.path.join(CSRC, "solver.cpp"), os.path.join(CSRC, "host_copy.cpp"),
+                    os.path.join(CPP, "solver_check.cpp"), "-pthread", "-o", exe], check=True)
+
+    def run(scenario):
+        r = subprocess.run([exe, scenario], capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+        words = r.stdout.split()
+        return dict(zip(words[::2], map(float, words[1::2])))
+    return run
+
+
+@pytest.mark.parametrize("failing", ["malloc", "memcpy"])
+def test_instance_ranges_are_sent_again_after_a_failure(check, failing):
+    # 3 vessels of 8 planes, 4 planes a workgroup
+    got = check("instances_after_" + failing)
+    assert got == {"first": HLB_E_DEVICE, "second": 0, "ranges": 6, "ordered": 1}

@@ -236,15 +236,22 @@ template <typename T>
 struct DevBuf {
   T* p = nullptr;
   size_t count = 0;
-  ~DevBuf() { if (p) (void)hipFree(p); }
+  ~DevBuf() { release(); }
   hipError_t alloc(size_t n) {
     count = n;
     return hipMalloc((void**)&p, sizeof(T) * (n ? n : 1));
   }
+  void release() {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+  }
+  // No buffer is left where this fails: p says that the values are there.
   hipError_t upload(const std::vector<T>& v) {
     hipError_t e = alloc(v.size());
-    if (e != hipSuccess || v.empty()) return e;
-    return hipMemcpy(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess && !v.empty())
+      e = hipMemcpy(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) release();
+    return e;
   }
   size_t bytes() const { return p ? sizeof(T) * (count ? count : 1) : 0; }
 };

@@ -1,6 +1,7 @@
 // Scenarios of the solver's host code (csrc/solver.cpp) on the fake HIP
 // runtime, with the kernels replaced by stand-ins that note their arguments.
 // argv[1] chooses one; prints what happened.
+#include <algorithm>
 #include <cstdio>
 #include <string>
 #include <vector>
@@ -13,6 +14,7 @@ namespace {
 
 std::vector<int64_t> seen_range;      // of the last monitor launch
 bool monitor_had_range = false;
+std::vector<float> seen_normals;      // of the last field export
 
 }  // namespace
 
@@ -26,8 +28,10 @@ int launch_export_distributions(const DevDomain&, const StepArgs&, const void*, 
                                 const int64_t*, double*, void*) {
   return 0;
 }
-int launch_export_fields(const DevDomain&, const StepArgs&, const void*, int, const FieldPtrs&,
-                         void*) {
+int launch_export_fields(const DevDomain& d, const StepArgs&, const void*, int,
+                         const FieldPtrs& f, void*) {
+  seen_normals.clear();
+  if (f.rec_normal) seen_normals.assign(f.rec_normal, f.rec_normal + 3 * d.nb);
   return 0;
 }
 int launch_import(const DevDomain&, const StepArgs&, const double*, const int64_t*, void*, void*) {
@@ -130,11 +134,27 @@ int instances_after(int& countdown) {
   return 0;
 }
 
+// The same for the wall normals of the stress outputs.
+int normals_after(int& countdown) {
+  Sites v(3);
+  std::vector<double> wss(3);
+  countdown = 1;
+  const int first = hlb_get_wall_shear_stress(v.s, wss.data());
+  countdown = 0;
+  const int second = hlb_get_wall_shear_stress(v.s, wss.data());
+  std::sort(seen_normals.begin(), seen_normals.end());
+  std::printf("first %d second %d normals %d\n", first, second,
+              (int)(seen_normals == std::vector<float>{1, 2, 2, 3, 3, 3, 4, 4, 5}));
+  return 0;
+}
+
 }  // namespace
 
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "instances_after_malloc") return instances_after(fake::fail_malloc);
   if (what == "instances_after_memcpy") return instances_after(fake::fail_memcpy);
+  if (what == "normals_after_malloc") return normals_after(fake::fail_malloc);
+  if (what == "normals_after_memcpy") return normals_after(fake::fail_memcpy);
   return 2;
 }

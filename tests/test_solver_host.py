@@ -35,3 +35,9 @@ def test_instance_ranges_are_sent_again_after_a_failure(check, failing):
     # 3 vessels of 8 planes, 4 planes a workgroup
     got = check("instances_after_" + failing)
     assert got == {"first": HLB_E_DEVICE, "second": 0, "ranges": 6, "ordered": 1}
+
+
+@pytest.mark.parametrize("failing", ["malloc", "memcpy"])
+def test_wall_normals_are_sent_again_after_a_failure(check, failing):
+    got = check("normals_after_" + failing)
+    assert got == {"first": HLB_E_DEVICE, "second": 0, "normals": 1}

@@ -1453,10 +1453,13 @@ int hlb_reduce_noalloc(hlb_solver* s, hlb_monitor* out) {
 int hlb_snapshot_velocity(hlb_solver* s) {
   if (!s) return fail(HLB_E_INVALID, "null solver");
   if (!s->initialised) return fail(HLB_E_STATE, "state not initialised");
-  if (!s->u_snap.p) HIP_OR_FAIL(s->u_snap.alloc(3 * s->npc));
+  const bool first = !s->u_snap.p;
+  if (first) HIP_OR_FAIL(s->u_snap.alloc(3 * s->npc));
   if (hlb::launch_snapshot_velocity(s->dom, s->args_for_stream(), s->state[s->cur],
-                                    s->post_stream ? 1 : 0, s->u_snap.p, s->stream))
+                                    s->post_stream ? 1 : 0, s->u_snap.p, s->stream)) {
+    if (first) s->u_snap.release();  // (an earlier snapshot stays)
     return fail(HLB_E_DEVICE, "velocity kernel launch failed");
+  }
   HIP_OR_FAIL(hipStreamSynchronize(s->stream));
   return HLB_OK;
 }

@@ -13,7 +13,7 @@
 namespace {
 
 std::vector<int64_t> seen_range;      // of the last monitor launch
-bool monitor_had_range = false;
+bool monitor_had_range = false, launch_fails = false;
 std::vector<float> seen_normals;      // of the last field export
 
 }  // namespace
@@ -55,7 +55,7 @@ int launch_monitor(const DevDomain&, const StepArgs&, const void*, int, const in
   return 0;
 }
 int launch_snapshot_velocity(const DevDomain&, const StepArgs&, const void*, int, double*, void*) {
-  return 0;
+  return launch_fails ? 1 : 0;
 }
 int launch_velocity_change(const DevDomain&, const StepArgs&, const void*, int, const int64_t*,
                            int groups, const double*, const double*, double, double* partials,
@@ -148,6 +148,18 @@ int normals_after(int& countdown) {
   return 0;
 }
 
+// A first snapshot that fails, the velocity change after it, and the two again.
+int snapshot_fails() {
+  Sites v(2);
+  double change = -1;
+  launch_fails = true;
+  const int failed = hlb_snapshot_velocity(v.s), without = hlb_velocity_change(v.s, 1.0, &change);
+  launch_fails = false;
+  const int taken = hlb_snapshot_velocity(v.s), with = hlb_velocity_change(v.s, 1.0, &change);
+  std::printf("failed %d without %d taken %d with %d\n", failed, without, taken, with);
+  return 0;
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -156,5 +168,6 @@ int main(int, char** argv) {
   if (what == "instances_after_memcpy") return instances_after(fake::fail_memcpy);
   if (what == "normals_after_malloc") return normals_after(fake::fail_malloc);
   if (what == "normals_after_memcpy") return normals_after(fake::fail_memcpy);
+  if (what == "snapshot_fails") return snapshot_fails();
   return 2;
 }

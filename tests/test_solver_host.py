@@ -10,7 +10,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "hemelb_amd", "csrc")
 CPP = os.path.join(ROOT, "tests", "cpp")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
-HLB_E_DEVICE = -2
+HLB_E_DEVICE, HLB_E_STATE = -2, -4
 
 
 @pytest.fixture(scope="module")
@@ -41,3 +41,8 @@ def test_instance_ranges_are_sent_again_after_a_failure(check, failing):
 def test_wall_normals_are_sent_again_after_a_failure(check, failing):
     got = check("normals_after_" + failing)
     assert got == {"first": HLB_E_DEVICE, "second": 0, "normals": 1}
+
+
+def test_a_snapshot_that_failed_is_no_snapshot(check):
+    assert check("snapshot_fails") == {"failed": HLB_E_DEVICE, "without": HLB_E_STATE,
+                                       "taken": 0, "with": 0}

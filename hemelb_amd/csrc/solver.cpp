@@ -1631,20 +1631,23 @@ int hlb_autotune(hlb_solver* s, int32_t steps, hlb_launch_shape* best, double* b
   const bool post_stream = s->post_stream;
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->p.device);
-  std::vector<hlb_launch_shape> cand;
+  // The shape held on entry first, so that no other replaces it without having
+  // been faster, then one-pass shapes (the defaults of every size among them)
+  // and strided ones.
+  hlb_launch_shape keep{};
+  hlb_get_launch_shape(s, &keep);
+  std::vector<hlb_launch_shape> cand{keep};
   for (int split : {1, 0}) {
     for (int th : {256, 128, 64})
       for (int xcd : {1, 0}) cand.push_back({th, 1, 0, xcd, split});
     for (int run : {2, 16, 64}) cand.push_back({256, 1, 0, run, split});
-    cand.push_back({128, 1, 0, 4, split});
-    cand.push_back({128, 1, 0, 8, split});
+    for (int run : {2, 4, 8}) cand.push_back({128, 1, 0, run, split});
+    cand.push_back({64, 1, 0, 16, split});
   }
   cand.push_back({256, 2, 0, 1, 0});
   cand.push_back({128, 2, 0, 1, 0});
   for (int th : {256, 128}) cand.push_back({th, 1, cus * 24 * 64 / th, 1, 0});
   cand.push_back({256, 2, cus * 24 * 64 / 256, 1, 0});
-  hlb_launch_shape keep{};
-  hlb_get_launch_shape(s, &keep);
   for (auto& c : cand) c.wide = keep.wide;  // the addressing stays the caller's
   double best_t = 1e300;
   hlb_launch_shape best_s = keep;
@@ -1652,7 +1655,7 @@ int hlb_autotune(hlb_solver* s, int32_t steps, hlb_launch_shape* best, double* b
   for (const auto& c : cand) {
     hlb_set_launch_shape(s, &c);
     double ms = 0;
-    rc = hlb_step(s, 2);  // warm
+    rc = hlb_step(s, best_t == 1e300 ? steps : 2);  // warm, the first trial above all
     if (!rc) rc = hlb_time_steps(s, steps, &ms);
     if (rc) break;
     if (ms < best_t) {

@@ -258,8 +258,9 @@ int hlb_velocity_change_instances(hlb_solver* s, const double* reference_speed,
  * round-robin order, 1 one contiguous range of the domain per XCD, K in
  * 2..4096 runs of K consecutive workgroups per XCD with the eight XCDs on
  * adjacent runs (the grid is padded to a multiple of 8K).
- * hlb_autotune times a set of shapes for `steps` steps each on the current
- * state, restores the state and time, and keeps the fastest. */
+ * hlb_autotune times a set of shapes, the one held on entry among them, for
+ * `steps` steps each on the current state, restores the state and time, and
+ * keeps the fastest. */
 typedef struct {
   int32_t threads;
   int32_t planes;

@@ -14,6 +14,7 @@ namespace {
 
 std::vector<int64_t> seen_range;      // of the last monitor launch
 bool monitor_had_range = false, launch_fails = false;
+struct { uint32_t threads, planes, xcd_remap; } fast_shape{0, 0, 0};  // 1 ms a step, others 2
 std::vector<float> seen_normals;      // of the last field export
 
 }  // namespace
@@ -22,7 +23,12 @@ namespace hlb {
 
 int monitor_groups(const DevDomain&) { return 1; }
 int launch_fill(const DevDomain&, const StepArgs&, const double*, void*, void*) { return 0; }
-int launch_step(const DevDomain&, const StepArgs&, const void*, void*, void*) { return 0; }
+int launch_step(const DevDomain&, const StepArgs& a, const void*, void*, void* stream) {
+  const bool fast = a.threads == fast_shape.threads && a.planes == fast_shape.planes &&
+                    a.xcd_remap == fast_shape.xcd_remap && a.split == 0 && a.groups == 0;
+  static_cast<hipStream_t>(stream)->push([fast] { fake::clock_ms += fast ? 1.0 : 2.0; });
+  return 0;
+}
 int launch_collide_only(const DevDomain&, const StepArgs&, const void*, void*, void*) { return 0; }
 int launch_export_distributions(const DevDomain&, const StepArgs&, const void*, int,
                                 const int64_t*, double*, void*) {
@@ -160,6 +166,27 @@ int snapshot_fails() {
   return 0;
 }
 
+// The tuner where one shape takes half the time of all others: the one held on
+// entry, or another (`held` null: the default shape).
+int tune(uint32_t threads, uint32_t planes, uint32_t remap, const hlb_launch_shape* held) {
+  Sites v(2);
+  fake::on_event = [](hipEvent_t e) {
+    std::lock_guard<std::mutex> lock(fake::mu);
+    fake::event_ms[e] = fake::clock_ms;
+  };
+  if (held && hlb_set_launch_shape(v.s, held)) return 1;
+  fast_shape = {threads, planes, remap};
+  hlb_launch_shape best{}, now{};
+  double ms = 0;
+  const int rc = hlb_autotune(v.s, 4, &best, &ms);
+  hlb_get_launch_shape(v.s, &now);
+  std::printf("error %d ms %g threads %d planes %d remap %d kept %d\n", rc, ms, best.threads,
+              best.planes, best.xcd_remap,
+              (int)(now.threads == best.threads && now.planes == best.planes &&
+                    now.xcd_remap == best.xcd_remap));
+  return 0;
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -169,5 +196,11 @@ int main(int, char** argv) {
   if (what == "normals_after_malloc") return normals_after(fake::fail_malloc);
   if (what == "normals_after_memcpy") return normals_after(fake::fail_memcpy);
   if (what == "snapshot_fails") return snapshot_fails();
+  if (what == "tune_default_fastest") return tune(64, 1, 16, nullptr);
+  if (what == "tune_held_fastest") {
+    const hlb_launch_shape held{256, 4, 0, 1, 0, 0};
+    return tune(256, 4, 1, &held);
+  }
+  if (what == "tune_other_default_fastest") return tune(128, 1, 2, nullptr);
   return 2;
 }

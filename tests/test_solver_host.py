@@ -1,6 +1,6 @@
-"""The solver's host code after failed runtime calls (csrc/solver.cpp), on the
-CPU: linked with a fake HIP runtime that fails on demand and with stand-ins for
-the kernels (tests/cpp/solver_check.cpp)."""
+"""The solver's host code (csrc/solver.cpp) after failed runtime calls, and its
+launch-shape tuner, on the CPU: linked with a fake HIP runtime that fails on
+demand and with stand-ins for the kernels (tests/cpp/solver_check.cpp)."""
 import os
 import subprocess
 
@@ -46,3 +46,14 @@ def test_wall_normals_are_sent_again_after_a_failure(check, failing):
 def test_a_snapshot_that_failed_is_no_snapshot(check):
     assert check("snapshot_fails") == {"failed": HLB_E_DEVICE, "without": HLB_E_STATE,
                                        "taken": 0, "with": 0}
+
+
+@pytest.mark.parametrize("scenario,shape", [
+    ("tune_default_fastest", (64, 1, 16)),         # the shape a small solver starts with
+    ("tune_held_fastest", (256, 4, 1)),            # one that the caller chose
+    ("tune_other_default_fastest", (128, 1, 2)),   # the one large binary64 domains start with
+])
+def test_the_tuner_knows_the_shape_held_and_the_defaults(check, scenario, shape):
+    got = check(scenario)
+    assert (got["error"], got["kept"], got["ms"]) == (0, 1, 1.0)
+    assert (got["threads"], got["planes"], got["remap"]) == shape

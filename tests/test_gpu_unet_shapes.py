@@ -1,8 +1,8 @@
 """The U-Net at sizes where its kernels' tiles, boxes and channel groups can go
 wrong: widths that are no multiple of the 16- or 8-wide boxes, levels smaller
-than a box, every form of the LDS convolution (groups of 16 channels, large
-and small boxes, K in one slice and in several) and the channel counts that
-have none.  The oracle and its tolerances are those of test_gpu_unet.py
+than a box, forms of the LDS convolution (groups of 16 channels, large and
+small boxes, K in one slice and in several; the others in
+test_gpu_unet_forms.py) and the channel counts that have none.  The oracle and its tolerances are those of test_gpu_unet.py
 (bfloat16 against binary64 with the same roundings)."""
 import numpy as np
 import pytest

@@ -8,6 +8,7 @@ import subprocess
 import pytest
 
 from hemelb_amd import warmstart as WS
+from tests import test_gpu_unet, test_gpu_unet_forms, test_gpu_unet_shapes
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -31,13 +32,13 @@ def plan(tmp_path_factory):
 LEVELS = [0, 0, 1, 1, 2, 2, 3, 3, 2, 2, 1, 1, 0, 0]
 
 
-def convolutions(side, batch, chans=WS.CHANNELS):
-    """(N, side, ci, co) of a training step's convolutions: forward, and the
+def convolutions(side, batch, chans=WS.CHANNELS, backward=True):
+    """(N, side, ci, co) of the forward convolutions, and with `backward` of the
     data gradients of all layers but the first."""
     calls = []
     for (name, ci, co), level in zip(WS.layer_shapes(chans), LEVELS):
         calls.append((batch, side >> level, ci, co))
-        if name != "e1a":
+        if backward and name != "e1a":
             calls.append((batch, side >> level, co, ci))
     return calls
 
@@ -63,3 +64,25 @@ def test_every_choice_is_compiled_and_concatenations_read_in_place_have_a_form(p
 ])
 def test_boxes_are_not_mostly_padding(plan, call, box):
     assert bool(plan([call])[0][0]) == box
+
+
+def convolutions_tested():
+    """Those of the GPU tests that compare with the oracle."""
+    trained = list(test_gpu_unet_forms.CASES)
+    for module in (test_gpu_unet, test_gpu_unet_shapes):
+        for mark in module.test_forward_and_gradients_match_oracle.pytestmark:
+            if mark.name == "parametrize":
+                trained += [getattr(c, "values", c) for c in mark.args[1]]
+    return [c for case in trained for c in convolutions(*case)] + [
+        c for case in test_gpu_unet_forms.OUTPUT_CASES for c in convolutions(*case, backward=False)]
+
+
+def test_gpu_tests_run_every_form(plan):
+    run = {(*form, sliced) for *form, sliced, _ in plan(convolutions_tested()) if form[0]}
+    assert {form[:7] for form in run} == set(plan())
+    # crops up to 128^3, half of what a 128^3 crop holds per batch, 6 at most
+    reached = {(*form, sliced): (side, batch) for side in range(8, 129, 8)
+               for batch in range(1, max(1, min(6, 128 ** 3 // (2 * side ** 3))) + 1)
+               for *form, sliced, _ in plan(convolutions(side, batch)) if form[0]}
+    missing = {k: v for k, v in reached.items() if k not in run}
+    assert not missing, missing

@@ -86,9 +86,10 @@ struct DevDomain {
 };
 
 // Outputs of launch_export_fields, in the caller's site order (null: not
-// wanted): density [n] and velocity [n][3], or any of the stress outputs
-// (wall shear stress, von Mises, shear rate [n], tensor [n][6], traction
-// and tangential traction [n][3]).
+// wanted): density [n] and velocity [n][3]; or any of the stress outputs (von
+// Mises, shear rate [n], tensor [n][6], traction and tangential traction
+// [n][3]); or the wall shear stress [nb] by boundary record, of those with a
+// wall.
 struct FieldPtrs {
   const int64_t* perm = nullptr;      // compact site -> caller's index
   double* density = nullptr;

@@ -8,6 +8,7 @@ import pytest
 
 from hemelb_amd import lb as L
 from hemelb_amd import workloads as WL
+from hemelb_amd.geometry import Domain
 from tests import cases as K
 
 pytestmark = pytest.mark.gpu
@@ -110,3 +111,29 @@ def test_large_exports_return_what_was_set(radius, length):
     one(0)
     with ThreadPoolExecutor(3) as pool:   # concurrent copies: one stages, the others do not
         list(pool.map(one, (1, 2, 3)))
+
+
+def test_wall_shear_stress_of_more_than_a_million_wall_sites():
+    # a sheet one site thick, every site at the wall: more boundary records
+    # than the export writes to pinned memory
+    side = 1025
+    x, y = np.divmod(np.arange(side * side), side)
+    coords = np.stack([x, y, np.zeros_like(x)], 1).astype(np.int32)
+    n = len(coords)
+    assert n > 1 << 20
+    inside = lambda p: ((p >= 0) & (p < [side, side, 1])).all(1)  # noqa: E731
+    mask = np.zeros(n, np.uint32)
+    for d in range(1, 19):
+        mask |= np.where(inside(coords + L.LATTICES[19].VECTORS[d]), 0, 1 << (d - 1)).astype(np.uint32)
+    rng = np.random.default_rng(7)
+    normal = rng.standard_normal((n, 3)).astype(np.float32)
+    normal /= np.linalg.norm(normal, axis=1, keepdims=True)
+    case = K.Case(Domain(19, coords, np.ones(n, np.uint32), mask, np.zeros(n, np.uint32),
+                         np.full(n, -1, np.int32), np.full((n, 18), 0.5, np.float32), normal,
+                         [], []))
+    print(f"[exports] {n} wall sites", flush=True)
+    f = rng.uniform(0.01, 0.1, (n, 19))
+    gpu, orc = case.product(), case.oracle()
+    gpu.set_distributions(f)
+    orc.set_f(f)
+    np.testing.assert_array_equal(gpu.wall_shear_stress(), orc.wall_shear_stress(normal))

@@ -329,8 +329,8 @@ __device__ __forceinline__ double second_moment(const double (&fneq)[Q]) {
 // Pi_ab = sum_l f_neq_l c_la c_lb in direction order (terms with
 // c_la c_lb = 0 add nothing):
 // * wall shear stress magnitude (Lattice.h:652-727): t_a = sum_b (Pi_ab n_b)
-//   temp, sqrt(|t|^2 - (t . n)^2), of the wall sites alone and by boundary
-//   record: the caller's array holds a constant elsewhere;
+//   temp, sqrt(|t|^2 - (t . n)^2) at wall sites, the largest double (the
+//   reference's NO_VALUE) elsewhere;
 // * stress tensor (CalculateStressTensor, 630-645): Pi * (1 - 1/(2 tau))
 //   plus (rho - 1) Cs2 on the diagonal, upper triangle xx xy xz yy yz zz;
 // * von Mises stress (508-552) and shear rate (728-753, 890-907);
@@ -343,13 +343,13 @@ __global__ __launch_bounds__(256) void k_export_fields(DevDomain D, StepArgs A,
   using L = Lat<Q>;
   SiteRef r;
   if (!Lay::locate(D, r)) return;
-  if (STRESS && F.wss && !r.wall) return;
+  if (STRESS && F.by_record && !r.wall) return;
   double f[Q];
   post_stream_site<Q, S, Lay>(D, A, fin, from_post_stream, r, f);
   double rho, mx, my, mz;
   moments<Q, double>(f, rho, mx, my, mz);
+  const int64_t c = STRESS && F.by_record ? (int64_t)r.rec : F.perm[Lay::compact(D, r)];
   if constexpr (!STRESS) {
-    const int64_t c = F.perm[Lay::compact(D, r)];
     if (F.density) F.density[c] = rho;
     if (F.velocity) {
       F.velocity[3 * c] = mx / rho;
@@ -375,21 +375,23 @@ __global__ __launch_bounds__(256) void k_export_fields(DevDomain D, StepArgs A,
   if (wall && F.rec_normal)
     for (int a = 0; a < 3; ++a) n[a] = (double)F.rec_normal[3 * (int64_t)r.rec + a];
   if (F.wss) {
-    // -sqrt(2) * the stress parameter of LbmParameters
-    // (LbmParameters.h:34-39), as Lattice.h:669 uses it
-    const double temp = (1.0 - 1.0 / (2.0 * ts)) / sqrt(2.0) * (-sqrt(2.0));
-    const double pi[3][3] = {{p00, p10, p20}, {p10, p11, p21}, {p20, p21, p22}};
-    double sq = 0.0, nn = 0.0;
-    for (int a = 0; a < 3; ++a) {
-      double t = 0.0;
-      for (int b = 0; b < 3; ++b) t += pi[a][b] * n[b] * temp;
-      sq += t * t;
-      nn += t * n[a];
+    double v = 1.7976931348623157e308;  // NO_VALUE, constants.h:47
+    if (wall) {
+      // -sqrt(2) * the stress parameter of LbmParameters
+      // (LbmParameters.h:34-39), as Lattice.h:669 uses it
+      const double temp = (1.0 - 1.0 / (2.0 * ts)) / sqrt(2.0) * (-sqrt(2.0));
+      const double pi[3][3] = {{p00, p10, p20}, {p10, p11, p21}, {p20, p21, p22}};
+      double sq = 0.0, nn = 0.0;
+      for (int a = 0; a < 3; ++a) {
+        double t = 0.0;
+        for (int b = 0; b < 3; ++b) t += pi[a][b] * n[b] * temp;
+        sq += t * t;
+        nn += t * n[a];
+      }
+      v = sqrt(sq - nn * nn);
     }
-    F.wss[r.rec] = sqrt(sq - nn * nn);
-    return;
+    F.wss[c] = v;
   }
-  const int64_t c = F.perm[Lay::compact(D, r)];
   const double fac = 1 - 1 / (2 * ts);
   const double pr = (rho - 1) * kCs2;
   const double s00 = p00 * fac + pr, s10 = p10 * fac, s20 = p20 * fac, s11 = p11 * fac + pr,
@@ -443,9 +445,11 @@ __global__ __launch_bounds__(256) void k_export_fields(DevDomain D, StepArgs A,
         for (int b = 0; b < 3; ++b) t[a] += sg[a][b] * n[b];
       for (int a = 0; a < 3; ++a) tn = tn + t[a] * n[a];
     }
+    // by record: consecutive lanes on consecutive words
+    const int64_t at = F.by_record ? c : 3 * c, next = F.by_record ? D.nb : 1;
     for (int a = 0; a < 3; ++a) {
-      if (F.traction) F.traction[3 * c + a] = t[a];
-      if (F.tangential) F.tangential[3 * c + a] = wall ? t[a] - n[a] * tn : 0.0;
+      if (F.traction) F.traction[at + a * next] = t[a];
+      if (F.tangential) F.tangential[at + a * next] = wall ? t[a] - n[a] * tn : 0.0;
     }
   }
 }

@@ -86,10 +86,11 @@ struct DevDomain {
 };
 
 // Outputs of launch_export_fields, in the caller's site order (null: not
-// wanted): density [n] and velocity [n][3]; or any of the stress outputs (von
-// Mises, shear rate [n], tensor [n][6], traction and tangential traction
-// [n][3]); or the wall shear stress [nb] by boundary record, of those with a
-// wall.
+// wanted): density [n] and velocity [n][3], or any of the stress outputs
+// (wall shear stress, von Mises, shear rate [n], tensor [n][6], traction
+// and tangential traction [n][3]).  by_record: the wall sites' outputs alone, by
+// boundary record: wall shear stress [nb], traction and tangential traction
+// [3][nb].
 struct FieldPtrs {
   const int64_t* perm = nullptr;      // compact site -> caller's index
   double* density = nullptr;
@@ -101,6 +102,7 @@ struct FieldPtrs {
   double* traction = nullptr;
   double* tangential = nullptr;
   const float* rec_normal = nullptr;  // [nb][3] wall normal of boundary record r
+  bool by_record = false;
   double tau = 0;                     // relaxation time (ensembles: blk_tau)
 };
 

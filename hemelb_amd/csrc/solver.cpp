@@ -1332,6 +1332,71 @@ int hlb_get_macroscopic(hlb_solver* s, double* density, double* velocity) {
   return export_fields(s, wanted, 2);
 }
 
+// The same for outputs of the wall sites alone, which hold `elsewhere` at every
+// other site.  Where the caller's arrays are up to kWallByRecord bytes each, the
+// wall sites' values come from the device by boundary record, and the constant
+// is written here meanwhile: wall shear stress of 494 k sites, 44 k of them at
+// a wall, 144 us (247 as a whole field), of 1.13 M with 19 k 280 (390);
+// traction of 819 k with 141 k 0.40 ms (0.81), both tractions of 1.13 M 0.75
+// (1.91).  Larger arrays are mostly mapped anew by malloc, and their page
+// faults decide, which the workers of a whole field's copy share: wall shear
+// stress of 7.6 M sites, 61 MB, 3.8 ms (2.4); traction of 3.4 M, 81 MB, 4.3
+// (2.9).  Up to 2^20 values the kernel writes pinned memory itself.
+constexpr int64_t kWallByRecord = int64_t(28) << 20;
+static int export_wall_fields(hlb_solver* s, const FieldRequest* wanted, int count,
+                              double elsewhere) {
+  const int64_t nb = s->dom.nb;
+  int64_t values = 0;
+  for (int k = 0; k < count; ++k) {
+    if (!wanted[k].host) continue;
+    values += wanted[k].width;
+    if ((int64_t)sizeof(double) * wanted[k].width * s->n > kWallByRecord)
+      return export_fields(s, wanted, count);
+  }
+  const int64_t total = values * nb;
+  const bool pinned = total <= 1 << 20;
+  int r = pinned ? s->ensure_partials((size_t)total) : s->ensure_exports(total);
+  if (r) return r;
+  hlb::FieldPtrs F;
+  F.rec_normal = s->d_rec_normals.p;
+  F.tau = s->p.tau;
+  F.by_record = true;
+  double* at = pinned ? s->partials : s->exports.p;
+  for (int k = 0; k < count; ++k) {
+    if (!wanted[k].host) continue;
+    F.*wanted[k].slot = at;
+    at += wanted[k].width * nb;
+  }
+  if (nb && hlb::launch_export_fields(s->dom, s->args_for_stream(), s->state[s->cur],
+                                      s->post_stream ? 1 : 0, F, s->stream))
+    return fail(HLB_E_DEVICE, "export kernel launch failed");
+  for (int k = 0; k < count; ++k) {
+    if (!wanted[k].host) continue;
+    if (elsewhere == 0.0)
+      std::memset(wanted[k].host, 0, sizeof(double) * wanted[k].width * s->n);
+    else
+      std::fill_n(wanted[k].host, wanted[k].width * s->n, elsewhere);
+  }
+  const double* from = s->partials;
+  std::vector<double> copied;
+  if (pinned) {
+    HIP_OR_FAIL(hipStreamSynchronize(s->stream));
+  } else {
+    copied.resize((size_t)total);
+    HIP_OR_FAIL(hlb::copy_to_host({{copied.data(), s->exports.p, sizeof(double) * total}},
+                                  s->stream));
+    from = copied.data();
+  }
+  for (int k = 0; k < count; ++k) {
+    if (!wanted[k].host) continue;
+    const int width = wanted[k].width;
+    for (const auto& w : s->wall_sites)
+      for (int a = 0; a < width; ++a) wanted[k].host[width * w.site + a] = from[a * nb + w.rec];
+    from += width * nb;
+  }
+  return HLB_OK;
+}
+
 int hlb_get_wall_shear_stress(hlb_solver* s, double* stress) {
   if (!s || !stress) return fail(HLB_E_INVALID, "null argument");
   if (!s->initialised) return fail(HLB_E_STATE, "state not initialised");
@@ -1339,34 +1404,8 @@ int hlb_get_wall_shear_stress(hlb_solver* s, double* stress) {
     return fail(HLB_E_STATE, "wall normals were not given to hlb_create");
   int r = s->ensure_normals();
   if (r) return r;
-  // The wall sites' values alone come from the device, the constant elsewhere is
-  // written here meanwhile: the whole field took 384 us on a disc of 1.13 M
-  // sites with 19 k at the wall, this 272; 317 and 234 on an 819 k-site tree
-  // with 141 k; the same 1.3 ms on a 4 M-site tree.  Up to 8 MB the kernel
-  // writes pinned memory itself.
-  const int64_t nb = s->dom.nb;
-  const bool pinned = nb <= 1 << 20;
-  r = pinned ? s->ensure_partials((size_t)nb) : s->ensure_exports(nb);
-  if (r) return r;
-  hlb::FieldPtrs F;
-  F.rec_normal = s->d_rec_normals.p;
-  F.tau = s->p.tau;
-  F.wss = pinned ? s->partials : s->exports.p;
-  if (nb && hlb::launch_export_fields(s->dom, s->args_for_stream(), s->state[s->cur],
-                                      s->post_stream ? 1 : 0, F, s->stream))
-    return fail(HLB_E_DEVICE, "export kernel launch failed");
-  std::fill(stress, stress + s->n, std::numeric_limits<double>::max());  // NO_VALUE, constants.h:47
-  const double* values = s->partials;
-  std::vector<double> copied;
-  if (pinned) {
-    HIP_OR_FAIL(hipStreamSynchronize(s->stream));
-  } else {
-    copied.resize((size_t)nb);
-    HIP_OR_FAIL(hlb::copy_to_host({{copied.data(), s->exports.p, sizeof(double) * nb}}, s->stream));
-    values = copied.data();
-  }
-  for (const auto& w : s->wall_sites) stress[w.site] = values[w.rec];
-  return HLB_OK;
+  const FieldRequest wanted[] = {{&hlb::FieldPtrs::wss, 1, stress}};
+  return export_wall_fields(s, wanted, 1, std::numeric_limits<double>::max());  // NO_VALUE, constants.h:47
 }
 
 int hlb_get_stress(hlb_solver* s, double* tensor, double* von_mises, double* shear_rate,
@@ -1384,6 +1423,9 @@ int hlb_get_stress(hlb_solver* s, double* tensor, double* von_mises, double* she
                                  {&hlb::FieldPtrs::shear_rate, 1, shear_rate},
                                  {&hlb::FieldPtrs::traction, 3, traction},
                                  {&hlb::FieldPtrs::tangential, 3, tangential}};
+  // traction is zero away from the walls (Common.h:107-121)
+  if ((traction || tangential) && !tensor && !von_mises && !shear_rate)
+    return export_wall_fields(s, wanted + 3, 2, 0.0);
   return export_fields(s, wanted, 5);
 }
 

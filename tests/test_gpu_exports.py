@@ -3,9 +3,12 @@ form and addressing: fields and stresses against the oracle's formulas on the
 exported distributions (bitwise, as the formulas are binary64 in one order),
 the exported distributions against the oracle's run, the reductions against
 numpy over the exported fields."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from hemelb_amd import _native as N
 from hemelb_amd import lb as L
 from hemelb_amd import workloads as WL
 from hemelb_amd.geometry import Domain
@@ -113,27 +116,50 @@ def test_large_exports_return_what_was_set(radius, length):
         list(pool.map(one, (1, 2, 3)))
 
 
-def test_wall_shear_stress_of_more_than_a_million_wall_sites():
-    # a sheet one site thick, every site at the wall: more boundary records
-    # than the export writes to pinned memory
-    side = 1025
+def sheet(side, rng):
+    """A sheet of side x side sites, one site thick: every site at a wall."""
     x, y = np.divmod(np.arange(side * side), side)
     coords = np.stack([x, y, np.zeros_like(x)], 1).astype(np.int32)
     n = len(coords)
-    assert n > 1 << 20
-    inside = lambda p: ((p >= 0) & (p < [side, side, 1])).all(1)  # noqa: E731
     mask = np.zeros(n, np.uint32)
     for d in range(1, 19):
-        mask |= np.where(inside(coords + L.LATTICES[19].VECTORS[d]), 0, 1 << (d - 1)).astype(np.uint32)
-    rng = np.random.default_rng(7)
+        to = coords + L.LATTICES[19].VECTORS[d]
+        inside = ((to >= 0) & (to < [side, side, 1])).all(1)
+        mask |= np.where(inside, 0, 1 << (d - 1)).astype(np.uint32)
     normal = rng.standard_normal((n, 3)).astype(np.float32)
     normal /= np.linalg.norm(normal, axis=1, keepdims=True)
-    case = K.Case(Domain(19, coords, np.ones(n, np.uint32), mask, np.zeros(n, np.uint32),
+    return K.Case(Domain(19, coords, np.ones(n, np.uint32), mask, np.zeros(n, np.uint32),
                          np.full(n, -1, np.int32), np.full((n, 18), 0.5, np.float32), normal,
                          [], []))
-    print(f"[exports] {n} wall sites", flush=True)
-    f = rng.uniform(0.01, 0.1, (n, 19))
-    gpu, orc = case.product(), case.oracle()
-    gpu.set_distributions(f)
-    orc.set_f(f)
-    np.testing.assert_array_equal(gpu.wall_shear_stress(), orc.wall_shear_stress(normal))
+
+
+# the outputs of the wall sites alone: more than 2^20 values, which do not go
+# through pinned memory, and arrays above 28 MiB, which come as whole fields (24
+# bytes a site, then 8 as well)
+@pytest.mark.parametrize("side,storage,layout", [
+    (40, "fp64", "blocks"), (1025, "fp64", "blocks"), (1025, "fp32", "compact_blocks"),
+    (1700, "fp64", "pull_table"), (2000, "fp16", "pull_table")])
+def test_wall_outputs_of_many_wall_sites(side, storage, layout):
+    rng = np.random.default_rng(side)
+    case = sheet(side, rng)
+    n, normal = case.domain.n, case.domain.normal
+    print(f"[exports] {n} wall sites {storage} {layout}", flush=True)
+    gpu = case.product(storage=storage, layout=layout)
+    gpu.set_distributions(rng.random((n, 19), np.float32).astype(np.float64) * 0.1 + 0.01)
+    f = gpu.get_distributions()
+    wss, stress = gpu.wall_shear_stress(), gpu.stress()
+    traction, tangential = np.full((n, 3), np.nan), np.full((n, 3), np.nan)
+    ptr = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
+    N.check(N.lib().hlb_get_stress(gpu._h, None, None, None, ptr(traction), ptr(tangential)))
+    np.testing.assert_array_equal(traction, stress["traction"])
+    np.testing.assert_array_equal(tangential, stress["tangential_traction"])
+    # both are of a site's own values: a smaller sheet with the same rows
+    rows = np.sort(rng.choice(n, 1600, replace=False))
+    small = sheet(40, rng)
+    small.domain.normal = np.ascontiguousarray(normal[rows])
+    orc = small.oracle()
+    orc.set_f(f[rows])
+    np.testing.assert_array_equal(wss[rows], orc.wall_shear_stress(small.domain.normal))
+    want = orc.stress(small.domain.normal)
+    for name in ("traction", "tangential_traction"):
+        np.testing.assert_array_equal(stress[name][rows], want[name])

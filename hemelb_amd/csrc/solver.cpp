@@ -1333,16 +1333,23 @@ int hlb_get_macroscopic(hlb_solver* s, double* density, double* velocity) {
 }
 
 // The same for outputs of the wall sites alone, which hold `elsewhere` at every
-// other site.  Where the caller's arrays are up to kWallByRecord bytes each, the
-// wall sites' values come from the device by boundary record, and the constant
-// is written here meanwhile: wall shear stress of 494 k sites, 44 k of them at
-// a wall, 144 us (247 as a whole field), of 1.13 M with 19 k 280 (390);
+// other site.  Where few sites are at a wall and the caller's arrays are small,
+// the wall sites' values come from the device by boundary record, and the
+// constant is written here meanwhile: wall shear stress of 494 k sites, 44 k of
+// them at a wall, 144 us (247 as a whole field), of 1.13 M with 19 k 280 (390);
 // traction of 819 k with 141 k 0.40 ms (0.81), both tractions of 1.13 M 0.75
-// (1.91).  Larger arrays are mostly mapped anew by malloc, and their page
-// faults decide, which the workers of a whole field's copy share: wall shear
-// stress of 7.6 M sites, 61 MB, 3.8 ms (2.4); traction of 3.4 M, 81 MB, 4.3
-// (2.9).  Up to 2^20 values the kernel writes pinned memory itself.
-constexpr int64_t kWallByRecord = int64_t(28) << 20;
+// (1.91).
+// * Each wall site is a scattered store of about 1 ns, a whole field costs 130 us
+//   and what it copies: 1.32 M sites with 420 k at a wall 640 us (500), 4 M with
+//   504 k 1.37 ms (1.34).
+// * Arrays from 32 MiB on are mapped anew by malloc, and their page faults
+//   decide, which the workers of a whole field's copy share: wall shear stress
+//   of 7.6 M sites, 61 MB, 3.8 ms (2.4); traction of 3.4 M, 81 MB, 4.3 (2.9).
+// Up to 2^20 values the kernel writes pinned memory itself.
+static bool wall_by_record(const hlb_solver* s, int width) {
+  return (int64_t)s->wall_sites.size() <= (int64_t(1) << 17) + s->n / 12 &&
+         (int64_t)sizeof(double) * width * s->n <= int64_t(28) << 20;
+}
 static int export_wall_fields(hlb_solver* s, const FieldRequest* wanted, int count,
                               double elsewhere) {
   const int64_t nb = s->dom.nb;
@@ -1350,8 +1357,7 @@ static int export_wall_fields(hlb_solver* s, const FieldRequest* wanted, int cou
   for (int k = 0; k < count; ++k) {
     if (!wanted[k].host) continue;
     values += wanted[k].width;
-    if ((int64_t)sizeof(double) * wanted[k].width * s->n > kWallByRecord)
-      return export_fields(s, wanted, count);
+    if (!wall_by_record(s, wanted[k].width)) return export_fields(s, wanted, count);
   }
   const int64_t total = values * nb;
   const bool pinned = total <= 1 << 20;

@@ -116,34 +116,35 @@ def test_large_exports_return_what_was_set(radius, length):
         list(pool.map(one, (1, 2, 3)))
 
 
-def sheet(side, rng):
-    """A sheet of side x side sites, one site thick: every site at a wall."""
-    x, y = np.divmod(np.arange(side * side), side)
-    coords = np.stack([x, y, np.zeros_like(x)], 1).astype(np.int32)
+def slab(side, depth, rng):
+    """side x side x depth sites between walls."""
+    shape = np.array([side, side, depth])
+    coords = np.indices(shape).reshape(3, -1).T.astype(np.int32)
     n = len(coords)
     mask = np.zeros(n, np.uint32)
     for d in range(1, 19):
         to = coords + L.LATTICES[19].VECTORS[d]
-        inside = ((to >= 0) & (to < [side, side, 1])).all(1)
+        inside = ((to >= 0) & (to < shape)).all(1)
         mask |= np.where(inside, 0, 1 << (d - 1)).astype(np.uint32)
     normal = rng.standard_normal((n, 3)).astype(np.float32)
     normal /= np.linalg.norm(normal, axis=1, keepdims=True)
-    return K.Case(Domain(19, coords, np.ones(n, np.uint32), mask, np.zeros(n, np.uint32),
-                         np.full(n, -1, np.int32), np.full((n, 18), 0.5, np.float32), normal,
-                         [], []))
+    return K.Case(Domain(19, np.ascontiguousarray(coords), np.ones(n, np.uint32), mask,
+                         np.zeros(n, np.uint32), np.full(n, -1, np.int32),
+                         np.full((n, 18), 0.5, np.float32), normal, [], []))
 
 
-# the outputs of the wall sites alone: more than 2^20 values, which do not go
-# through pinned memory, and arrays above 28 MiB, which come as whole fields (24
-# bytes a site, then 8 as well)
-@pytest.mark.parametrize("side,storage,layout", [
-    (40, "fp64", "blocks"), (1025, "fp64", "blocks"), (1025, "fp32", "compact_blocks"),
-    (1700, "fp64", "pull_table"), (2000, "fp16", "pull_table")])
-def test_wall_outputs_of_many_wall_sites(side, storage, layout):
-    rng = np.random.default_rng(side)
-    case = sheet(side, rng)
-    n, normal = case.domain.n, case.domain.normal
-    print(f"[exports] {n} wall sites {storage} {layout}", flush=True)
+# the outputs of the wall sites alone, which come by boundary record, also where
+# the two tractions are more than 2^20 values and do not go through pinned memory
+# (191 k of 990 k sites at a wall); or as whole fields, where most sites are at a
+# wall or the arrays are large (traction, then the wall shear stress as well)
+@pytest.mark.parametrize("side,depth,storage,layout", [
+    (40, 1, "fp64", "blocks"), (300, 11, "fp64", "blocks"), (300, 11, "fp32", "compact_blocks"),
+    (1025, 1, "fp64", "blocks"), (300, 14, "fp32", "blocks"), (300, 41, "fp16", "pull_table")])
+def test_wall_outputs(side, depth, storage, layout):
+    rng = np.random.default_rng(side + depth)
+    case = slab(side, depth, rng)
+    n, normal, wall = case.domain.n, case.domain.normal, case.domain.wall_mask != 0
+    print(f"[exports] {n} sites, {wall.sum()} at a wall, {storage} {layout}", flush=True)
     gpu = case.product(storage=storage, layout=layout)
     gpu.set_distributions(rng.random((n, 19), np.float32).astype(np.float64) * 0.1 + 0.01)
     f = gpu.get_distributions()
@@ -153,9 +154,11 @@ def test_wall_outputs_of_many_wall_sites(side, storage, layout):
     N.check(N.lib().hlb_get_stress(gpu._h, None, None, None, ptr(traction), ptr(tangential)))
     np.testing.assert_array_equal(traction, stress["traction"])
     np.testing.assert_array_equal(tangential, stress["tangential_traction"])
-    # both are of a site's own values: a smaller sheet with the same rows
-    rows = np.sort(rng.choice(n, 1600, replace=False))
-    small = sheet(40, rng)
+    assert (wss[~wall] == np.finfo(np.float64).max).all()
+    assert not traction[~wall].any() and not tangential[~wall].any()
+    # they are of a site's own values: a small sheet with the same rows
+    rows = np.sort(rng.choice(np.flatnonzero(wall), 1600, replace=False))
+    small = slab(40, 1, rng)
     small.domain.normal = np.ascontiguousarray(normal[rows])
     orc = small.oracle()
     orc.set_f(f[rows])

@@ -60,12 +60,14 @@ __global__ __launch_bounds__(256) void k_step(DevDomain D, StepArgs A,
                                               S* __restrict__ fout) {
   step_wave<Q, KERNEL, S, Lay>(D, A, fin, fout);
 }
-// The same step held to WAVES waves per SIMD, without spills: binary16 to 7
-// (at most 72 VGPRs; it is bound by the issue and latency of its vector
-// instructions rather than by bytes, and the seventh wave measured 3 % faster
-// on the vessel tree), binary32 to 6 (80 VGPRs; left to itself it takes 86, 5
-// waves, and the step of a 4 M-site tree 168.5 instead of 163.2 us).
-// Binary64 takes its natural 4: held to 5 it spills.
+// The same step held to kStepWaves waves per SIMD: binary16 to 7 (at most 72
+// VGPRs; it is bound by the issue and latency of its vector instructions rather
+// than by bytes, and the seventh wave measured 3 % faster on the vessel tree),
+// binary32 to 6 (80 VGPRs; left to itself it takes 86, 5 waves, and the step of
+// a 4 M-site tree 168.5 instead of 163.2 us).  Only the D3Q19 binary16 forms
+// with 64-bit addresses and of the compact layout spill for it, one register (8
+// bytes of scratch a lane; 109.4 and 167.9 us on that tree).  Binary64 takes
+// its natural 4: held to 5 it spills.
 template <typename S> constexpr int kStepWaves = sizeof(S) == 2 ? 7 : 6;
 template <int Q, int KERNEL, typename S, class Lay>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStepWaves<S>)))

@@ -204,10 +204,13 @@ __global__ __launch_bounds__(256) void k_conv_fwd(Grid3 g, const uint16_t* __res
 // same bits whichever kernel runs.
 //
 // Measured at 64^3 x 4 (k_conv_fwd before): 16 -> 16 channels 67 -> 25 us
-// (575 TF/s; its 67 MB take 13), 48 -> 16 147 -> 77, 16 -> 48 in binary32 144
-// -> 68 (its bytes take 45), 96 -> 32 at 32^3 106 -> 62; all convolutions and
-// data gradients of a training iteration 1.65 -> 0.55 ms.  Now bound by the
-// LDS reads of the position fragments (1 KB a product where NT is 1).
+// (575 TF/s; its 67 MB take 13), 48 -> 16 147 -> 75, 16 -> 48 in binary32 144
+// -> 66 (its bytes take 45), 96 -> 32 at 32^3 106 -> 59; all convolutions and
+// data gradients of a training iteration 1.65 -> 0.63 ms.  No unit is near its
+// limit now: by the counters the LDS is active for 9 to 26 % of the cycles and
+// the matrix cores for 5 to 32 %, and waves wait 36 to 61 % of their time, for
+// the box, staged before its products, and for the weights, with one or two
+// workgroups a CU to cover it.
 // --------------------------------------------------------------------------
 template <int I, int N, typename F>
 __device__ __forceinline__ void sfor(F&& f) {
@@ -636,8 +639,9 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(Grid3 g, const uint16_t* __r
 // Transposing on the way into LDS (dword loads, packing, three copies
 // shifted by dx) took most of the time before.  Measured at 64^3 x 4, a layer
 // of 16 -> 16 channels 75 -> 28 us (510 TF/s), all 14 layers of a training
-// iteration 0.62 -> 0.35 ms.  Bound by the LDS reads (1 KB a product with one
-// output tile) and the staging of 2.5 positions per position.
+// iteration 0.62 -> 0.30 ms.  By the counters, the LDS active 22 to 34 % of the
+// cycles, the matrix cores 23 to 34 %, waves waiting 30 to 48 % of their time at
+// the larger levels: the staging of 2.5 positions per position is not covered.
 // --------------------------------------------------------------------------
 template <int BW>
 struct WBox {

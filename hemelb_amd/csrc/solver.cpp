@@ -13,6 +13,7 @@
 #include <cstring>
 #include <limits>
 #include <memory>
+#include <new>
 #include <numeric>
 #include <string>
 #include <unordered_map>
@@ -1384,14 +1385,15 @@ static int export_wall_fields(hlb_solver* s, const FieldRequest* wanted, int cou
       std::fill_n(wanted[k].host, wanted[k].width * s->n, elsewhere);
   }
   const double* from = s->partials;
-  std::vector<double> copied;
+  std::unique_ptr<double[]> copied;
   if (pinned) {
     HIP_OR_FAIL(hipStreamSynchronize(s->stream));
   } else {
-    copied.resize((size_t)total);
-    HIP_OR_FAIL(hlb::copy_to_host({{copied.data(), s->exports.p, sizeof(double) * total}},
+    copied.reset(new (std::nothrow) double[(size_t)total]);
+    if (!copied) return fail(HLB_E_NOMEM, "no memory for the wall sites' values");
+    HIP_OR_FAIL(hlb::copy_to_host({{copied.get(), s->exports.p, sizeof(double) * total}},
                                   s->stream));
-    from = copied.data();
+    from = copied.get();
   }
   for (int k = 0; k < count; ++k) {
     if (!wanted[k].host) continue;

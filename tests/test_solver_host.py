@@ -10,7 +10,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "hemelb_amd", "csrc")
 CPP = os.path.join(ROOT, "tests", "cpp")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
-HLB_E_DEVICE, HLB_E_STATE = -2, -4
+HLB_E_DEVICE, HLB_E_NOMEM, HLB_E_STATE = -2, -3, -4
 
 
 @pytest.fixture(scope="module")
@@ -46,6 +46,10 @@ def test_wall_normals_are_sent_again_after_a_failure(check, failing):
 def test_a_snapshot_that_failed_is_no_snapshot(check):
     assert check("snapshot_fails") == {"failed": HLB_E_DEVICE, "without": HLB_E_STATE,
                                        "taken": 0, "with": 0}
+
+
+def test_wall_values_without_host_memory_are_an_error(check):
+    assert check("tractions_without_memory") == {"first": HLB_E_NOMEM, "second": 0, "by_record": 1}
 
 
 @pytest.mark.parametrize("scenario,shape", [
